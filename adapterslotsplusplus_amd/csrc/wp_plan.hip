@@ -9,18 +9,23 @@
 //      split into pieces of 32 tokens (the last one takes the remainder),
 //      slots assigned in token-start order by an exclusive scan;
 //   2. the grouping the apply kernels run on (no reference counterpart): the
-//      runs are sorted by adapter id (bitonic sort of 64-bit (id, run) keys, so
-//      token order is kept inside an adapter), concatenated into `perm`, and
-//      each adapter's tokens are cut into blocks of `bt` tokens.  Every touched
-//      adapter's weights are then streamed once per block instead of once per
-//      run (about 232 runs vs 49 adapters for 256 Zipf-routed decode tokens).
+//      tokens of ids >= 0 in a stable counting sort by adapter id (`perm`), each
+//      adapter's tokens cut into blocks of `bt` tokens.  Every touched adapter's
+//      weights are then streamed once per block instead of once per run (about
+//      232 runs vs 49 adapters for 256 Zipf-routed decode tokens).
 //
 // The reference uses one 256-thread block with a serial per-run scan and a
 // Hillis-Steele scan over shared memory, writing over PCIe into mapped host
-// memory.  Here: wave64 shuffle scans, LDS-resident arrays, HBM outputs written
-// by all threads in parallel (each output slot finds its run by binary search
-// over the scanned offsets), and capacities of 256 / 2048 / 8192 tokens.
+// memory.  Here the kernel is bound by latency alone (a few KB of traffic, one
+// workgroup), so it is built to pass few workgroup barriers: 64 consecutive
+// tokens are one wave's lanes, a run table is a 64-bit ballot per 64 tokens,
+// ranks among equal ids come from ballots and popcounts, and every wave scans
+// the per-wave counts by itself instead of waiting for another to do it.  A
+// step whose ids are below 256 takes two barriers in all; larger ids take the
+// same counting pass once per further 8 bits.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "wp_apply.h"
 #include "wp_sync.h"
@@ -29,59 +34,12 @@ namespace wp {
 namespace {
 
 
-// Exclusive scan of one int per thread across the workgroup.  `scratch` holds
-// NT/64 ints.  Returns the thread's exclusive prefix; *total gets the sum.
-// Begins and ends with a workgroup barrier.
-template <int NT>
-__device__ __forceinline__ int block_exclusive_scan(int v, int* scratch, int* total) {
-  constexpr int kWaves = NT / 64;
-  const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  int x = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int y = __shfl_up(x, off, 64);
-    if (lane >= off) x += y;
-  }
-  lds_barrier();
-  if (lane == 63) scratch[wid] = x;
-  lds_barrier();
-  if (wid == 0) {
-    int w = lane < kWaves ? scratch[lane] : 0;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int y = __shfl_up(w, off, 64);
-      if (lane >= off) w += y;
-    }
-    if (lane < kWaves) scratch[lane] = w;
-  }
-  lds_barrier();
-  const int base = wid > 0 ? scratch[wid - 1] : 0;
-  *total = scratch[kWaves - 1];
-  lds_barrier();
-  return base + x - v;
-}
-
-// Largest i in [0, n) with a[i] <= q, for non-decreasing a and a[0] <= q.
-__device__ __forceinline__ int upper_index(const int* a, int n, int q) {
-  int lo = 0;
-  int hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (a[mid] <= q) {
-      lo = mid;
-    } else {
-      hi = mid - 1;
-    }
-  }
-  return lo;
-}
-
 // Traced builds (-DWP_TRACE): thread 0 records the 100 MHz real-time counter
 // at the plan build's phase boundaries into m.trace[0..7], after waiting for
-// its memory operations: 0 entry, 1 ids in LDS (maintenance done), 2 run
-// starts, 3 segment table stored, 4 runs sorted, 5 perm stored, 6 block
-// table stored, 7 block token lists and header stored.
+// its memory operations: 0 entry, 1 ids loaded, 2 run masks exchanged (first
+// barrier, maintenance done), 3 segment pieces and digit counts exchanged
+// (second barrier), 4 segment table stored, 5 digit bases known, 6 perm and
+// block token lists stored, 7 block table and header stored.
 #ifdef WP_TRACE
 __device__ __forceinline__ void plan_stamp(const Maint& m, int i) {
   if (m.trace != nullptr && threadIdx.x == 0) {
@@ -222,15 +180,6 @@ __global__ __launch_bounds__(256) void stage_copy_kernel(StageJobs jobs) {
   }
 }
 
-// Runs sorted by counting (below) when there are at most kRankMax of them and
-// the waves' broadcast reads (keys x keys per thread x waves) stay within
-// kRankWork; past that, a bitonic sort.  Measured on MI355X: 256-token plans
-// 15.8 -> 12.7 us per build_seg_bounds; at 1024 threads the waves' reads
-// queue on the CU's LDS (2048 Zipf-routed tokens: 42 us bitonic, 96 us by
-// counting).
-constexpr int kRankMax = 1024;
-constexpr int kRankWork = 4096;
-
 // plan_kernel's explicit arguments, as laid out in its kernel-argument
 // segment: touch_kernel_args reads below this size only.
 struct PlanKernelArgs {
@@ -248,6 +197,186 @@ struct PlanKernelArgs {
 static_assert(offsetof(PlanKernelArgs, m) == 80 && sizeof(PlanKernelArgs) == 80 + sizeof(Maint),
               "plan_kernel's argument size as passed to touch_kernel_args");
 
+// ------------------------------------------------------------- plan build ----
+
+// Digits of one counting pass (8 bits).
+constexpr int kDigits = 256;
+
+__device__ __forceinline__ uint64_t lanes_below(int lane) { return (1ull << lane) - 1ull; }
+__device__ __forceinline__ int last_bit(uint64_t m) { return 63 - __builtin_clzll(m); }
+
+template <typename V, typename Op>
+__device__ __forceinline__ V wave_all_reduce(V v, Op op) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = op(v, __shfl_xor(v, off, 64));
+  return v;
+}
+
+// Position of the last start bit in the words before `first`, or -1.
+template <int NWORDS>
+__device__ __forceinline__ int last_start_before(const uint64_t* s_start, int first) {
+  if (first == 0) return -1;
+  const int lane = threadIdx.x & 63;
+  int v = -1;
+#pragma unroll
+  for (int k = 0; k < (NWORDS + 63) / 64; ++k) {
+    const int wi = lane + 64 * k;
+    if (wi < first) {
+      const uint64_t m = s_start[wi];
+      if (m != 0) v = wi * 64 + last_bit(m);
+    }
+  }
+  return wave_all_reduce(v, [](int a, int b) { return a > b ? a : b; });
+}
+
+// Set bits of the words before `first` (low half) and of all words (high half).
+template <int NWORDS>
+__device__ __forceinline__ uint32_t count_words(const uint64_t* s_words, int first) {
+  const int lane = threadIdx.x & 63;
+  uint32_t v = 0;
+#pragma unroll
+  for (int k = 0; k < (NWORDS + 63) / 64; ++k) {
+    const int wi = lane + 64 * k;
+    if (wi < NWORDS) {
+      const uint32_t c = static_cast<uint32_t>(__popcll(s_words[wi]));
+      v += (c << 16) + (wi < first ? c : 0u);
+    }
+  }
+  return wave_all_reduce(v, [](uint32_t a, uint32_t b) { return a + b; });
+}
+
+// Pieces of runs.  start[e] marks the first item of each run among the 64
+// items of this wave's word e (word index first + e, item i = 64 * word +
+// lane); `carry` is the last run start before the wave's words.  piece[e]
+// marks the items of `live` at a multiple of P from their run's start, and
+// rs[e] is the lane's run start.
+template <int E>
+__device__ __forceinline__ void mark_pieces(const uint64_t (&start)[E], const uint64_t (&live)[E], int first, int carry,
+                                            int P, uint64_t (&piece)[E], int (&rs)[E]) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t le = (lanes_below(lane) << 1) | 1ull;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int w0 = (first + e) * 64;
+    const uint64_t below = start[e] & le;
+    rs[e] = below != 0 ? w0 + last_bit(below) : carry;
+    const bool p = ((live[e] >> lane) & 1ull) != 0 && ((w0 + lane - rs[e]) & (P - 1)) == 0;
+    piece[e] = __ballot(p);
+    if (start[e] != 0) carry = w0 + last_bit(start[e]);
+  }
+}
+
+// Rank of each item among the wave's earlier items of the same digit (in item
+// order), and the wave's count per digit left in cnt[] (zeroed by the caller).
+// `bits`: digit bits that can be set.  The row is this wave's own and LDS
+// accesses of one wave complete in order; volatile keeps the compiler from
+// carrying a count across words.
+template <int E>
+__device__ __forceinline__ void rank_digits(const uint32_t (&dig)[E], const uint64_t (&live)[E], int bits,
+                                            volatile uint32_t* cnt, uint32_t (&rank)[E]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    rank[e] = 0;
+    if (live[e] == 0) continue;
+    uint64_t m = live[e];
+    for (int b = 0; b < bits; ++b) {
+      const bool one = ((dig[e] >> b) & 1u) != 0;
+      const uint64_t ones = __ballot(one);
+      m &= one ? ones : ~ones;
+    }
+    if ((live[e] >> lane) & 1ull) {
+      const uint32_t base = cnt[dig[e]];
+      rank[e] = base + static_cast<uint32_t>(__popcll(m & lanes_below(lane)));
+      if ((m & lanes_below(lane)) == 0) cnt[dig[e]] = base + static_cast<uint32_t>(__popcll(m));
+    }
+  }
+}
+
+// One wave's view of every wave's digit counts: digits 4 * lane .. + 3.
+struct Digits {
+  uint32_t tot[4];  // items of the digit
+  uint32_t pre[4];  // ... in the waves before this one
+  uint32_t off[4];  // items of all digits below
+  uint32_t blk[4];  // blocks of all digits below
+  uint32_t n_items, n_blocks, n_digits;
+};
+template <int NW>
+__device__ __forceinline__ Digits scan_digits(const uint32_t (*s_cnt)[kDigits], int wave, int max_digit, int bt_log2) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63;
+  Digits r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r.tot[j] = r.pre[j] = 0;
+  if (4 * lane <= max_digit) {
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const u32x4 c = *reinterpret_cast<const u32x4*>(&s_cnt[w][4 * lane]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        r.tot[j] += c[j];
+        r.pre[j] += w < wave ? c[j] : 0u;
+      }
+    }
+  }
+  // Items (at most 8192) and blocks (at most as many) in one scan.
+  const uint32_t round = (1u << bt_log2) - 1u;
+  uint32_t own[4], sum = 0;
+  r.n_digits = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    own[j] = r.tot[j] | (((r.tot[j] + round) >> bt_log2) << 16);
+    sum += own[j];
+    r.n_digits += static_cast<uint32_t>(__popcll(__ballot(r.tot[j] != 0)));
+  }
+  uint32_t inc = sum;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t y = __shfl_up(inc, off, 64);
+    if (lane >= off) inc += y;
+  }
+  const uint32_t all = __shfl(inc, 63, 64);
+  r.n_items = all & 0xffffu;
+  r.n_blocks = all >> 16;
+  uint32_t ex = inc - sum;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    r.off[j] = ex & 0xffffu;
+    r.blk[j] = ex >> 16;
+    ex += own[j];
+  }
+  return r;
+}
+
+// One block of the plan and (bentries != null) its adapter-table entry as of
+// this build (agent-scope loads: the maintenance may have installed it from
+// another wave), or an empty one.
+__device__ __forceinline__ void put_block(Block* blocks, Entry* bentries, const Maint& m, int q, int32_t id, int first,
+                                          int count) {
+  Block b;
+  b.adapter_id = id;
+  b.first = first;
+  b.count = count;
+  b.entry = id;
+  blocks[q] = b;
+  if (bentries != nullptr) {
+    uint64_t w[4] = {0, 0, 0, 0};
+    if (m.table != nullptr && id >= 0 && id < m.table_cap) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = agent_load64(reinterpret_cast<const uint64_t*>(m.table + id) + i);
+    }
+    uint64_t* dst = reinterpret_cast<uint64_t*>(bentries + q);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dst[i] = w[i];
+  }
+}
+
+// Measured on MI355X, build_seg_bounds per launch in a graph of 40 (launch
+// included), against a run table sorted by counting or by a bitonic sort
+// (Zipf(1.1) routing over 64 ids, before -> now, us): T=64 8.8 -> 3.9, 256
+// 12.6 -> 4.4, 512 20.1 -> 5.9, 1024 27.0 -> 6.5, 2048 41.7 -> 8.0, 4096
+// 80.5 -> 11.1, 8192 152.7 -> 18.9; 16 contiguous prompts, T=8192 24.2 ->
+// 16.1; ids up to 1e6, T=256 15.2 -> 7.3, T=8192 198.7 -> 41.2.
 template <int NT, int E>
 __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, int idx_is_int64, int T,
                                                   uint32_t* __restrict__ header, Segment* __restrict__ segments,
@@ -256,300 +385,279 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
                                                   int seg_cap, int block_cap, int bt, Maint m) {
   touch_kernel_args<static_cast<int>(sizeof(PlanKernelArgs))>();
   constexpr int CAP = NT * E;
-  // s_big: the ids (int64) first, then the sort keys, then per-run offsets.
-  __shared__ unsigned long long s_big[CAP];
-  __shared__ int s_a[CAP + 1];  // run starts, later group adapter ids
-  __shared__ int s_b[CAP + 1];  // per-run segment bases, later group offsets
-  __shared__ int s_scan[NT / 64];
-  __shared__ unsigned long long s_sorted[kRankMax];  // sorted keys (counting path)
-  long long* s_id = reinterpret_cast<long long*>(s_big);
+  constexpr int NW = NT / 64;
+  constexpr int NWORDS = NW * E;
+  static_assert(NW % 4 == 0 && CAP <= 65536 / 2, "digit columns per wave; 16-bit token positions");
+  __shared__ uint64_t s_start[NWORDS];  // run starts, one bit per item
+  __shared__ uint64_t s_piece[NWORDS];  // piece starts
+  __shared__ alignas(16) uint32_t s_cnt[NW][kDigits];
+  // Each wave's own digit bases: {items below | items of earlier waves << 16, blocks below}.
+  __shared__ uint2 s_base[NW][kDigits];
+  __shared__ uint32_t s_wmax[NW];
+  __shared__ uint32_t s_wflag[NW];
+  // Ids of 256 and more only: the keys by token, and the order of each pass.
+  __shared__ uint32_t s_key[CAP];
+  __shared__ uint16_t s_ord[2][CAP];
+  __shared__ int s_flag;
 
   const int tid = threadIdx.x;
-  const int e0 = tid * E;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int first = wave * E;  // this wave's first word
+  const int bt_log2 = 31 - __builtin_clz(static_cast<unsigned>(bt));
   plan_stamp(m, 0);
 
-  // 1. ids, loaded first so that their latency overlaps the maintenance's
-  //    (the routing does not depend on the adapter table).
+  // 1. ids: lane l of word w holds token 64 w + l.  The id before the wave's
+  //    first token, the publications' state, the poison word and the table
+  //    version load beside them (the routing does not depend on the table).
+  const auto load_id = [&](int i) {
+    return idx_is_int64 ? static_cast<const long long*>(idx)[i]
+                        : static_cast<long long>(static_cast<const int*>(idx)[i]);
+  };
   long long ids[E];
 #pragma unroll
-  for (int k = 0; k < E; ++k) {
-    const int i = tid + k * NT;
-    ids[k] = 0;
-    if (i < T)
-      ids[k] = idx_is_int64 ? static_cast<const long long*>(idx)[i]
-                            : static_cast<long long>(static_cast<const int*>(idx)[i]);
+  for (int e = 0; e < E; ++e) {
+    const int i = (first + e) * 64 + lane;
+    ids[e] = i < T ? load_id(i) : -1;
   }
-
-  // 0. Publications into the adapter table; the partial buffer's repair.
-  maintain(header, m, s_scan);
-  // The table version the block entry copies below are taken at (every
-  // install above has raised it before maintain's closing barrier).
-  // A build without copies records a version that no table write produces
-  // (the complement of the current one), so copies left by an earlier build
-  // can never pass for current ones.
-  const uint32_t table_ver =
-      tid == 0 ? __hip_atomic_load(&header[kHdrTableVer], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-
-  // ids -> LDS.
-#pragma unroll
-  for (int k = 0; k < E; ++k) s_id[tid + k * NT] = ids[k];
-  lds_barrier();
+  long long before = 0;
+  if (first > 0 && first * 64 - 1 < T) before = load_id(first * 64 - 1);
+  // A slot whose publication is absent or retired needs no maintenance.  The
+  // words are read unordered: a publication that was complete before this
+  // launch is seen whole, one still being written may wait for the next build
+  // (maintain() itself reads under the sequence lock).
+  uint32_t todo = 0;
+  if (m.table != nullptr && tid < m.n_pubs) {
+    const SlotPub* p = m.pubs + tid;
+    const int32_t id = __hip_atomic_load(&p->id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t gen = __hip_atomic_load(&p->gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t retired = __hip_atomic_load(m.retired + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    todo = id >= 0 && gen > retired ? 1u : 0u;
+  }
+  uint32_t table_ver = 0;
+  if (tid == 0) {
+    if (m.part != nullptr)
+      todo |= __hip_atomic_load(&header[kHdrPoison], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u ? 1u : 0u;
+    // The table version the block entry copies below are taken at.  A build
+    // without copies records a version that no table write produces (the
+    // complement of the current one), so copies left by an earlier build can
+    // never pass for current ones.
+    table_ver = __hip_atomic_load(&header[kHdrTableVer], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   plan_stamp(m, 1);
 
-  // 2. Run starts in token order (reference :484): s_a[r] = first token of run r.
-  bool is_start[E];
-  int nstart = 0;
+  // 2. Run starts in token order (reference :484) and the largest key.
+  uint64_t start[E], live[E];
+  uint32_t key[E];
+  uint32_t kmax = 0;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const int i = e0 + e;
-    is_start[e] = i < T && (i == 0 || s_id[i - 1] != s_id[i]);
-    nstart += is_start[e] ? 1 : 0;
+    const int i = (first + e) * 64 + lane;
+    long long prev = __shfl_up(ids[e], 1, 64);
+    if (lane == 0) prev = before;
+    start[e] = __ballot(i < T && (i == 0 || prev != ids[e]));
+    before = __shfl(ids[e], 63, 64);
+    const bool ok = i < T && ids[e] >= 0;
+    live[e] = __ballot(ok);
+    key[e] = static_cast<uint32_t>(static_cast<int>(ids[e]));
+    if (ok && key[e] > kmax) kmax = key[e];
+    if (lane == 0) s_start[first + e] = start[e];
   }
-  int n_runs = 0;
-  int rb = block_exclusive_scan<NT>(nstart, s_scan, &n_runs);
+  kmax = wave_all_reduce(kmax, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+  const uint64_t any_todo = __ballot(todo != 0);
+  if (lane == 0) {
+    s_wmax[wave] = kmax;
+    s_wflag[wave] = any_todo != 0 ? 1u : 0u;
+  }
+  // This wave's digit counts (a row only it writes and, until the second
+  // barrier, reads).
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    if (is_start[e]) s_a[rb++] = e0 + e;
-  }
-  if (tid == 0) s_a[n_runs] = T;
+  for (int j = 0; j < kDigits / 64; ++j) s_cnt[wave][lane + 64 * j] = 0u;
   lds_barrier();
+
+  uint32_t flag = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    kmax = s_wmax[w] > kmax ? s_wmax[w] : kmax;
+    flag |= s_wflag[w];
+  }
+  if (flag != 0) {
+    // Publications into the adapter table, the partial buffer's repair.
+    maintain(header, m, &s_flag);
+    __syncthreads();
+    if (tid == 0) table_ver = __hip_atomic_load(&header[kHdrTableVer], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   plan_stamp(m, 2);
 
-  // 3. Exported table.  Pieces per run: ceil(len/32) when id >= 0 (reference
-  //    :485-489); slot bases by exclusive scan in token-start order (:494-503).
-  int pieces[E];
-  int psum = 0;
+  // 3. The exported table's pieces: a run of id >= 0 starts one every 32
+  //    tokens (reference :485-489).  The first counting pass over the ids.
+  uint64_t piece[E];
+  int rs[E];
+  mark_pieces<E>(start, live, first, last_start_before<NWORDS>(s_start, first), kMaxSegmentTokens, piece, rs);
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (lane == 0) s_piece[first + e] = piece[e];
+  const bool small_ids = kmax < static_cast<uint32_t>(kDigits);
+  const int max_digit = small_ids ? static_cast<int>(kmax) : kDigits - 1;
+  uint32_t dig[E], rank[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const int r = e0 + e;
-    pieces[e] = 0;
-    if (r < n_runs) {
-      const int st = s_a[r];
-      if (s_id[st] >= 0) pieces[e] = (s_a[r + 1] - st + kMaxSegmentTokens - 1) / kMaxSegmentTokens;
-    }
-    psum += pieces[e];
+    dig[e] = key[e] & (kDigits - 1);
+    if (!small_ids) s_key[(first + e) * 64 + lane] = key[e];
   }
-  int n_segs = 0;
-  int sb = block_exclusive_scan<NT>(psum, s_scan, &n_segs);
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int r = e0 + e;
-    if (r < n_runs) s_b[r] = sb;
-    sb += pieces[e];
-  }
-  if (tid == 0) s_b[n_runs] = n_segs;
+  rank_digits<E>(dig, live, small_ids ? 32 - __builtin_clz(kmax | 1u) : 8, s_cnt[wave], rank);
   lds_barrier();
-  const int seg_out = n_segs < seg_cap ? n_segs : seg_cap;
-  for (int q = tid; q < seg_out; q += NT) {
-    const int r = upper_index(s_b, n_runs, q);
-    const int st = s_a[r];
-    const int len = s_a[r + 1] - st;
-    const int p = q - s_b[r];
-    const int rem = len - p * kMaxSegmentTokens;
-    Segment s;
-    s.adapter_id = static_cast<int>(s_id[st]);
-    s.token_start = st + p * kMaxSegmentTokens;
-    s.token_count = rem < kMaxSegmentTokens ? rem : kMaxSegmentTokens;
-    s.pad = 0;
-    segments[q] = s;
-  }
   plan_stamp(m, 3);
 
-  // 4. Sort the runs with id >= 0 by (adapter id, run index).
-  unsigned long long key[E];
-  int nvalid = 0;
+  // 4. Segment table: slots by token order (reference :494-503).
+  const uint32_t nseg = count_words<NWORDS>(s_piece, first);
+  const int n_segs = static_cast<int>(nseg >> 16);
+  int slot0 = static_cast<int>(nseg & 0xffffu);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const int r = e0 + e;
-    key[e] = ~0ull;
-    if (r < n_runs) {
-      const long long id = s_id[s_a[r]];
-      if (id >= 0) {
-        key[e] = (static_cast<unsigned long long>(static_cast<unsigned>(static_cast<int>(id))) << 32) |
-                 static_cast<unsigned>(r);
-        ++nvalid;
-      }
+    const int w = first + e;
+    const int i = w * 64 + lane;
+    const int slot = slot0 + __popcll(piece[e] & lanes_below(lane));
+    slot0 += __popcll(piece[e]);
+    if (!((piece[e] >> lane) & 1ull) || slot >= seg_cap) continue;
+    // The piece ends at the next run or piece start (at most 32 tokens on), or at T.
+    const uint64_t up = ((start[e] | piece[e]) >> lane) >> 1;
+    int end = T;
+    if (up != 0) {
+      end = i + 1 + __builtin_ctzll(up);
+    } else if (w + 1 < NWORDS) {
+      const uint64_t nx = s_start[w + 1] | s_piece[w + 1];
+      if (nx != 0) end = (w + 1) * 64 + __builtin_ctzll(nx);
     }
+    Segment s;
+    s.adapter_id = static_cast<int>(key[e]);
+    s.token_start = i;
+    s.token_count = end - i;
+    s.pad = 0;
+    segments[slot] = s;
   }
-  int n_vruns = 0;
-  int vb = block_exclusive_scan<NT>(nvalid, s_scan, &n_vruns);  // ends every read of s_id
+  plan_stamp(m, 4);
+
+  // 5. Tokens grouped by adapter, token order kept inside an adapter.
+  int n_tok, n_groups, n_blocks;
+  if (small_ids) {
+    const Digits g = scan_digits<NW>(s_cnt, wave, max_digit, bt_log2);
+    n_tok = static_cast<int>(g.n_items);
+    n_groups = static_cast<int>(g.n_digits);
+    n_blocks = static_cast<int>(g.n_blocks);
+    if (4 * lane <= max_digit) {
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    if (key[e] != ~0ull) s_big[vb++] = key[e];
-  }
-  const unsigned long long* skey = s_big;  // the sorted keys
-  if (n_vruns <= kRankMax && n_vruns * E * (NT / 64) <= kRankWork) {
-    // Keys are distinct (the run index is in them): a key's position is
-    // the number of keys below it.  Every lane reads the same key at once
-    // (an LDS broadcast), with no barrier per step, unlike a bitonic sort's
-    // log^2 rounds (7 of the 16 us of a 256-token plan).
-    lds_barrier();
+      for (int j = 0; j < 4; ++j) s_base[wave][4 * lane + j] = uint2{g.off[j] | (g.pre[j] << 16), g.blk[j]};
+    }
+    plan_stamp(m, 5);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      if (key[e] == ~0ull) continue;
-      int below = 0;
-#pragma unroll 8
-      for (int i = 0; i < n_vruns; ++i) below += s_big[i] < key[e] ? 1 : 0;
-      s_sorted[below] = key[e];
+      if (!((live[e] >> lane) & 1ull)) continue;
+      const int i = (first + e) * 64 + lane;
+      const uint2 bs = s_base[wave][dig[e]];
+      const int pos = static_cast<int>((bs.x >> 16) + rank[e]);  // inside the adapter's group
+      perm[static_cast<int>(bs.x & 0xffffu) + pos] = i;
+      const int q = static_cast<int>(bs.y) + (pos >> bt_log2);
+      if (q < block_cap) bperm[static_cast<int64_t>(q) * kBlockTokens + (pos & (bt - 1))] = i;
     }
-    lds_barrier();
-    skey = s_sorted;
+    plan_stamp(m, 6);
+    // Block table: wave w writes the blocks w / 4, w / 4 + NW / 4, ... of
+    // the digits 4 * lane + w % 4.
+    const int j = wave & 3;
+    const auto pick = [&](const uint32_t(&v)[4]) {
+      return static_cast<int>(j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3]);
+    };
+    const int tot = pick(g.tot), off = pick(g.off), blk0 = pick(g.blk);
+    const int nb = (tot + bt - 1) >> bt_log2;
+    for (int k = wave >> 2; k < nb; k += NW / 4)
+      if (blk0 + k < block_cap)
+        put_block(blocks, bentries, m, blk0 + k, 4 * lane + j, off + k * bt, min(bt, tot - k * bt));
   } else {
-    int P = 1;
-    while (P < n_vruns) P <<= 1;
-    for (int i = n_vruns + tid; i < P; i += NT) s_big[i] = ~0ull;
+    // Larger ids: the counting pass again over the next 8 bits of the order
+    // so far, then the groups' blocks from the sorted order the way the
+    // segments came from the token order.
+    n_tok = 0;
+    int cur = 0;
+    uint64_t lv[E];
+    uint32_t tok[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      lv[e] = live[e];
+      tok[e] = static_cast<uint32_t>((first + e) * 64 + lane);
+    }
+    for (int shift = 0;; shift += 8) {
+      const Digits g = scan_digits<NW>(s_cnt, wave, kDigits - 1, bt_log2);
+      n_tok = static_cast<int>(g.n_items);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s_base[wave][4 * lane + j].x = g.off[j] + g.pre[j];
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if ((lv[e] >> lane) & 1ull) s_ord[cur][s_base[wave][dig[e]].x + rank[e]] = static_cast<uint16_t>(tok[e]);
+      lds_barrier();
+      if (shift + 8 >= 32 || (kmax >> (shift + 8)) == 0) break;
+#pragma unroll
+      for (int j = 0; j < kDigits / 64; ++j) s_cnt[wave][lane + 64 * j] = 0u;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int q = (first + e) * 64 + lane;
+        lv[e] = __ballot(q < n_tok);
+        tok[e] = q < n_tok ? s_ord[cur][q] : 0u;
+        dig[e] = (s_key[tok[e]] >> (shift + 8)) & (kDigits - 1);
+      }
+      rank_digits<E>(dig, lv, 8, s_cnt[wave], rank);
+      cur ^= 1;
+      lds_barrier();
+    }
+    plan_stamp(m, 5);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int q = (first + e) * 64 + lane;
+      lv[e] = __ballot(q < n_tok);
+      tok[e] = q < n_tok ? s_ord[cur][q] : 0u;
+      dig[e] = s_key[tok[e]];
+      uint32_t prev = __shfl_up(dig[e], 1, 64);
+      if (lane == 0 && q > 0 && q < n_tok) prev = s_key[s_ord[cur][q - 1]];
+      start[e] = __ballot(q < n_tok && (q == 0 || prev != dig[e]));
+      if (lane == 0) s_start[first + e] = start[e];
+    }
     lds_barrier();
-    for (int k = 2; k <= P; k <<= 1) {
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        for (int i = tid; i < P; i += NT) {
-          const int ixj = i ^ j;
-          if (ixj > i) {
-            const unsigned long long a = s_big[i];
-            const unsigned long long b = s_big[ixj];
-            const bool ascending = (i & k) == 0;
-            if ((a > b) == ascending) {
-              s_big[i] = b;
-              s_big[ixj] = a;
-            }
-          }
-        }
-        lds_barrier();
+    n_groups = static_cast<int>(count_words<NWORDS>(s_start, first) >> 16);
+    mark_pieces<E>(start, lv, first, last_start_before<NWORDS>(s_start, first), bt, piece, rs);
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (lane == 0) s_piece[first + e] = piece[e];
+    lds_barrier();
+    const uint32_t nblk = count_words<NWORDS>(s_piece, first);
+    n_blocks = static_cast<int>(nblk >> 16);
+    int blk0 = static_cast<int>(nblk & 0xffffu);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int w = first + e;
+      const int q = w * 64 + lane;
+      const uint64_t le = (lanes_below(lane) << 1) | 1ull;
+      const int b = blk0 + __popcll(piece[e] & le) - 1;  // this position's block
+      blk0 += __popcll(piece[e]);
+      if (q >= n_tok) continue;
+      perm[q] = static_cast<int>(tok[e]);
+      if (b >= block_cap) continue;
+      bperm[static_cast<int64_t>(b) * kBlockTokens + ((q - rs[e]) & (bt - 1))] = static_cast<int>(tok[e]);
+      if (!((piece[e] >> lane) & 1ull)) continue;
+      const uint64_t up = ((start[e] | piece[e]) >> lane) >> 1;
+      int end = n_tok;
+      if (up != 0) {
+        end = q + 1 + __builtin_ctzll(up);
+      } else if (w + 1 < NWORDS) {
+        const uint64_t nx = s_start[w + 1] | s_piece[w + 1];
+        if (nx != 0) end = (w + 1) * 64 + __builtin_ctzll(nx);
       }
+      put_block(blocks, bentries, m, b, static_cast<int>(dig[e]), q, end - q);
     }
-  }
-
-  plan_stamp(m, 4);
-  // 5. perm: the tokens of the sorted runs, concatenated.
-  int len_e[E];
-  int start_e[E];
-  int gid_e[E];
-  bool gstart[E];
-  int lsum = 0;
-  int gcount = 0;
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int p = e0 + e;
-    len_e[e] = 0;
-    start_e[e] = 0;
-    gid_e[e] = 0;
-    gstart[e] = false;
-    if (p < n_vruns) {
-      const unsigned long long kk = skey[p];
-      const int r = static_cast<int>(kk & 0xffffffffull);
-      start_e[e] = s_a[r];
-      len_e[e] = s_a[r + 1] - s_a[r];
-      gid_e[e] = static_cast<int>(kk >> 32);
-      gstart[e] = p == 0 || (skey[p - 1] >> 32) != (kk >> 32);
-    }
-    lsum += len_e[e];
-    gcount += gstart[e] ? 1 : 0;
-  }
-  int n_tok = 0;
-  int ob = block_exclusive_scan<NT>(lsum, s_scan, &n_tok);  // ends every read of s_big keys and s_a
-  int off_e[E];
-  int* s_roff = reinterpret_cast<int*>(s_big);           // [CAP] run offsets into perm
-  int* s_rstart = reinterpret_cast<int*>(s_big) + CAP;   // [CAP] run first tokens
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int p = e0 + e;
-    off_e[e] = ob;
-    if (p < n_vruns) {
-      s_roff[p] = ob;
-      s_rstart[p] = start_e[e];
-    }
-    ob += len_e[e];
-  }
-  lds_barrier();
-  // perm[q] for q = tid + e*NT, kept in registers until the run tables are
-  // free, then in LDS for the block lists below.
-  int pv[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int q = tid + e * NT;
-    pv[e] = 0;
-    if (q < n_tok) {
-      const int p = upper_index(s_roff, n_vruns, q);
-      pv[e] = s_rstart[p] + (q - s_roff[p]);
-      perm[q] = pv[e];
-    }
-  }
-
-  plan_stamp(m, 5);
-  // 6. Groups (one per adapter) and their blocks of bt tokens.
-  int n_groups = 0;
-  int gb = block_exclusive_scan<NT>(gcount, s_scan, &n_groups);  // ends every read of s_roff / s_rstart
-  int* s_perm = reinterpret_cast<int*>(s_big) + CAP;             // [CAP] perm (over s_rstart)
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int q = tid + e * NT;
-    if (q < n_tok) s_perm[q] = pv[e];
-  }
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    if (gstart[e]) {
-      s_b[gb] = off_e[e];
-      s_a[gb] = gid_e[e];
-      ++gb;
-    }
-  }
-  if (tid == 0) s_b[n_groups] = n_tok;
-  lds_barrier();
-  int nb[E];
-  int bsum = 0;
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int g = e0 + e;
-    nb[e] = g < n_groups ? (s_b[g + 1] - s_b[g] + bt - 1) / bt : 0;
-    bsum += nb[e];
-  }
-  int n_blocks = 0;
-  int bb = block_exclusive_scan<NT>(bsum, s_scan, &n_blocks);
-  int* s_bbase = reinterpret_cast<int*>(s_big);  // [CAP] first block of each group
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int g = e0 + e;
-    if (g < n_groups) s_bbase[g] = bb;
-    bb += nb[e];
-  }
-  lds_barrier();
-  const int blk_out = n_blocks < block_cap ? n_blocks : block_cap;
-  for (int q = tid; q < blk_out; q += NT) {
-    const int g = upper_index(s_bbase, n_groups, q);
-    const int j = q - s_bbase[g];
-    const int n = s_b[g + 1] - s_b[g];
-    Block b;
-    b.adapter_id = s_a[g];
-    b.first = s_b[g] + j * bt;
-    b.count = n - j * bt < bt ? n - j * bt : bt;
-    b.entry = s_a[g];
-    blocks[q] = b;
-    if (bentries != nullptr) {
-      // The block's adapter-table entry (agent-scope loads: the maintenance
-      // above may have installed it from another wave), or an empty one.
-      uint64_t w[4] = {0, 0, 0, 0};
-      if (m.table != nullptr && b.entry >= 0 && b.entry < m.table_cap) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = agent_load64(reinterpret_cast<const uint64_t*>(m.table + b.entry) + i);
-      }
-      uint64_t* dst = reinterpret_cast<uint64_t*>(bentries + q);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dst[i] = w[i];
-    }
-  }
-  plan_stamp(m, 6);
-  // Block-padded token lists, from the LDS copy of perm.
-  for (int u = tid; u < blk_out * bt; u += NT) {
-    const int q = u / bt;
-    const int j = u - q * bt;
-    const int g = upper_index(s_bbase, n_groups, q);
-    const int n = s_b[g + 1] - s_b[g];
-    const int jj = (q - s_bbase[g]) * bt + j;  // position inside the group
-    if (jj < n) bperm[static_cast<int64_t>(q) * kBlockTokens + j] = s_perm[s_b[g] + jj];
+    plan_stamp(m, 6);
   }
 
   if (tid == 0) {
     header[kHdrNumSegments] = static_cast<uint32_t>(n_segs);
-    header[kHdrNumBlocks] = static_cast<uint32_t>(blk_out);
+    header[kHdrNumBlocks] = static_cast<uint32_t>(min(n_blocks, block_cap));
     header[kHdrNumGroups] = static_cast<uint32_t>(n_groups);
     header[kHdrNumValid] = static_cast<uint32_t>(n_tok);
     header[kHdrT] = static_cast<uint32_t>(T);
@@ -565,20 +673,27 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
 hipError_t launch_plan(const void* idx, int idx_is_int64, int T, uint32_t* header, Segment* segments, Block* blocks,
                        int32_t* perm, int32_t* bperm, Entry* bentries, int seg_cap, int block_cap, int bt,
                        const Maint* m, hipStream_t stream) {
-  if (T < 0 || bt < 1 || bt > kBlockTokens) return hipErrorInvalidValue;
+  if (T < 0 || bt < 1 || bt > kBlockTokens || (bt & (bt - 1)) != 0) return hipErrorInvalidValue;
   Maint mm{};
   if (m != nullptr) mm = *m;
   // Publications are applied by threads 0..n_pubs-1 of the smallest variant.
   if (mm.n_pubs < 0 || mm.n_pubs > 256) return hipErrorInvalidValue;
+  // The smallest capacity that holds T: a wave's words are consecutive, so a
+  // larger one would leave waves idle while others work their words in turn.
+  auto run = [&](auto nt, auto e) {
+    plan_kernel<decltype(nt)::value, decltype(e)::value><<<1, decltype(nt)::value, 0, stream>>>(
+        idx, idx_is_int64, T, header, segments, blocks, perm, bperm, bentries, seg_cap, block_cap, bt, mm);
+  };
   if (T <= 256) {
-    plan_kernel<256, 1><<<1, 256, 0, stream>>>(idx, idx_is_int64, T, header, segments, blocks, perm, bperm,
-                                               bentries, seg_cap, block_cap, bt, mm);
+    run(std::integral_constant<int, 256>{}, std::integral_constant<int, 1>{});
+  } else if (T <= 1024) {
+    run(std::integral_constant<int, 1024>{}, std::integral_constant<int, 1>{});
   } else if (T <= 2048) {
-    plan_kernel<1024, 2><<<1, 1024, 0, stream>>>(idx, idx_is_int64, T, header, segments, blocks, perm, bperm,
-                                                 bentries, seg_cap, block_cap, bt, mm);
+    run(std::integral_constant<int, 1024>{}, std::integral_constant<int, 2>{});
+  } else if (T <= 4096) {
+    run(std::integral_constant<int, 1024>{}, std::integral_constant<int, 4>{});
   } else if (T <= kPlanMaxTokens) {
-    plan_kernel<1024, 8><<<1, 1024, 0, stream>>>(idx, idx_is_int64, T, header, segments, blocks, perm, bperm,
-                                                 bentries, seg_cap, block_cap, bt, mm);
+    run(std::integral_constant<int, 1024>{}, std::integral_constant<int, 8>{});
   } else {
     return hipErrorInvalidValue;
   }

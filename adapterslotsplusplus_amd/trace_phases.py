@@ -282,8 +282,9 @@ def trace_plan(args):
     cases = [("cfg2 routing, T=256", wl.zipf_indices(256, 64, 1.1, 1)),
              ("cfg5 routing, T=128", torch.repeat_interleave(torch.arange(32), 4)),
              ("Zipf(1.1) over 64, T=2048", wl.zipf_indices(2048, 64, 1.1, 1))]
-    names = ["ids in LDS, maintenance done", "run starts", "segment table stored", "runs sorted",
-             "perm stored", "block table stored", "block token lists and header stored"]
+    names = ["ids loaded", "run masks exchanged, maintenance done", "pieces and digit counts exchanged",
+             "segment table stored", "digit bases known", "perm and block token lists stored",
+             "block table and header stored"]
     lines = ["### Phases of one `build_seg_bounds` plan build (traced build; median of 20 builds, us)", "",
              "| phase | " + " | ".join(c[0] for c in cases) + " |", "|---|" + "---|" * len(cases)]
     cols = []

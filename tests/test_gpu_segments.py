@@ -91,6 +91,26 @@ def test_random_routings_match_oracle(engine, T):
         assert blocks == oblocks
 
 
+@pytest.mark.parametrize("T", [63, 65, 256, 1024, 1025, 4096, 4097])
+@pytest.mark.parametrize("ids", ["edge", "one", "wide", "none"])
+def test_plan_counting_passes_match_oracle(engine, T, ids):
+    """The plan's counting passes at their edges: word and capacity edges in T,
+    ids on both sides of one 8-bit pass (255 / 256), of two, three and four
+    passes, one adapter for the whole step (a block table of one digit), and
+    no adapter at all."""
+    rng = np.random.default_rng(1000 + T)
+    choices = {"edge": [-1, 0, 1, 255], "one": [7], "none": [-1],
+               "wide": [0, 255, 256, 257, 65535, 65536, (1 << 24) + 3, (1 << 31) - 1]}[ids]
+    idx = np.repeat(rng.choice(choices, size=T), rng.choice([1, 1, 2, 33, 65], size=T))[:T]
+    announce(f"plan counting passes T={T} {ids}")
+    assert engine.build_seg_bounds(torch.from_numpy(idx.astype(np.int64)).cuda())
+    assert engine.read_segments() == [tuple(s) for s in so.seg_bounds(idx).tolist()]
+    perm, blocks = engine.read_plan()
+    operm, oblocks = oracle_blocks(idx)
+    assert perm == operm
+    assert blocks == oblocks
+
+
 def test_host_table_known_answers(engine, golden_dir):
     spec = kat(golden_dir, "segment_table_kat.json")
     A = torch.zeros(32, 64, dtype=torch.float16, device="cuda")
