@@ -165,6 +165,18 @@ hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t s
 // expand(): expand from a caller-provided token-indexed H.
 hipError_t launch_expand(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
 
+// vLLM V1's lora_expand: launch_expand on stacked weights where slice s reads
+// H at column s * a.hs1 of rows a.ldh apart (16-byte aligned, both multiples of
+// 16 bytes), in fp32 if h_f32; y + bias is rounded before the product, or
+// (zero_y) y is overwritten without being read.
+struct ExpandExt {
+  const void* bias[kMaxSlices];       // [num_ids, >= o_size] rows of the I/O type, or null
+  int64_t bias_stride[kMaxSlices];    // elements
+  int32_t zero_y;
+  int32_t h_f32;
+};
+hipError_t launch_expand_ext(int dtype_bf16, const ApplyArgs& a, const ExpandExt& x, hipStream_t stream);
+
 // Sets n 32-bit words at p to v (vector stores; a kernel, so that a caller
 // may capture it in a graph).
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t stream);
@@ -202,14 +214,14 @@ hipError_t launch_read_probe(const void* p, size_t bytes, void* sink, int workgr
 hipError_t launch_take_word(uint32_t* word, uint32_t* out, hipStream_t stream);
 
 // The per-token work of vLLM V1's LoRA op surface around the grouped kernels
-// (wp_aux.hip prep_kernel), one workgroup per block slot of the plan:
+// (wp_aux.hip prep_kernel), over the block slots of the plan:
 //   * h_src != null: the rank columns of slice s of token t's H,
 //     h_src[s * h_slice_stride + t * h_row_stride + k] (fp32 if h_f32, else
-//     the I/O type), rounded into h_dst[t * ldh_dst + s * rank + k];
-//   * zero_y: y[t, y_off[s] .. + o_size[s]) = 0 for every slice;
-//   * otherwise, for each slice with bias[s]: y = rn(y + bias[s][id]) over
-//     the window (bias rows bias_stride[s] elements apart; ids >= num_ids
-//     flagged kErrIdRange).
+//     the I/O type), rounded into h_dst[t * ldh_dst + s * rank + k] (an H whose
+//     rows launch_expand_ext cannot load as vectors);
+//   * for each slice with bias[s]: y = rn(y + bias[s][id]) over the window
+//     (bias rows bias_stride[s] elements apart; ids >= num_ids flagged
+//     kErrIdRange).
 struct PrepArgs {
   PlanView plan;
   int32_t n_slots;
@@ -224,8 +236,6 @@ struct PrepArgs {
   int32_t h_f32;
   void* y;
   int64_t ldy;
-  int32_t zero_y;
-  int32_t pad;
   int32_t o_size[kMaxSlices];
   int32_t y_off[kMaxSlices];
   const void* bias[kMaxSlices];

@@ -51,6 +51,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "wp_apply.h"
 #include "wp_device.h"
@@ -529,7 +530,8 @@ __device__ __forceinline__ OutChunk<T> out_chunk(const ApplyArgs& a, const Block
 // mixed ranks, expanded at RANK = 64); otherwise RANK.
 template <typename T, int RANK, bool DYN = false>
 __device__ __forceinline__ void load_chunk(const ApplyArgs& a, const OutChunk<T>& c, int32_t tok0,
-                                           typename VecOf<T>::v8 (&bf)[kOT][(RANK + 31) / 32], YRows& y0) {
+                                           typename VecOf<T>::v8 (&bf)[kOT][(RANK + 31) / 32], YRows& y0,
+                                           bool load_y = true) {
   constexpr int KS = (RANK + 31) / 32;
   const int rb = DYN ? c.res.rank : RANK;
   const int lane = threadIdx.x & 63;
@@ -549,9 +551,24 @@ __device__ __forceinline__ void load_chunk(const ApplyArgs& a, const OutChunk<T>
     }
   }
   int32_t tok[2];
-  yrows_tokens(ok ? tok0 : -1, tok);
+  yrows_tokens(ok && load_y ? tok0 : -1, tok);
   y0 = yrows_load<T>(a, c.y_off, ob, c.o_size, tok);
 }
+
+// Where an expand workgroup's H rows come from.
+enum HSource : int {
+  kHGlobal = 0,  // the caller's token-indexed H, I/O type
+  kHLds = 1,     // the block's rows in LDS (fused roles)
+  kHFloat = 2    // the caller's token-indexed H in fp32, rounded to the I/O type as it is loaded
+};
+
+// What the V1 expand adds to compute_chunk (kExt): y is not read (add_inputs
+// = False), or the chunk's bias row is added to it and rounded first.
+struct ChunkExt {
+  bool zero_y = false;
+  bool has_bias = false;
+  f32x4 bias[kOT];  // this lane's columns of the bias row
+};
 
 // Y[tokens, chunk columns] = rn(Y + H.B^T) for every token tile of the block;
 // H comes from LDS (fused; rows of hsl elements) or from the caller's
@@ -559,11 +576,12 @@ __device__ __forceinline__ void load_chunk(const ApplyArgs& a, const OutChunk<T>
 // in flight at once: their Y (and H) loads are issued together before the
 // MFMAs; y0 holds tile 0's Y, already loaded.  `stage` is this wave's
 // 16 x kStageStride LDS tile.
-template <typename T, int RANK, bool kHFromLds, int MAXT>
+template <typename T, int RANK, int HSRC, int MAXT, bool kExt = false>
 __device__ __forceinline__ void compute_chunk(const ApplyArgs& a, int b, const Block& blk, int32_t tok0,
                                               const OutChunk<T>& c,
                                               const typename VecOf<T>::v8 (&bf)[kOT][(RANK + 31) / 32],
-                                              const YRows& y0, const T* s_h, int hsl, T* stage) {
+                                              const YRows& y0, const T* s_h, int hsl, T* stage,
+                                              const ChunkExt& ext = ChunkExt{}) {
   using V8 = typename VecOf<T>::v8;
   constexpr int KS = (RANK + 31) / 32;
   const int lane = threadIdx.x & 63;
@@ -587,6 +605,8 @@ __device__ __forceinline__ void compute_chunk(const ApplyArgs& a, int b, const B
       yrows_tokens(tok_row[i], tok[i]);
       if (tt == 0)
         yt[i] = y0;
+      else if (kExt && ext.zero_y)
+        yt[i].v[0] = yt[i].v[1] = u32x4{0u, 0u, 0u, 0u};
       else
         yt[i] = yrows_load<T>(a, c.y_off, ob, c.o_size, tok[i]);
 #pragma unroll
@@ -594,8 +614,17 @@ __device__ __forceinline__ void compute_chunk(const ApplyArgs& a, int b, const B
         const int k = ks * 32 + kq;
         if (tok_row[i] < 0 || k >= RANK) {
           hf[i][ks] = zero8<T>();
-        } else if constexpr (kHFromLds) {
+        } else if constexpr (HSRC == kHLds) {
           hf[i][ks] = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(s_h + (tt * 16 + row) * hsl + c.h_col + k));
+        } else if constexpr (HSRC == kHFloat) {
+          const float* hp = static_cast<const float*>(a.h) + static_cast<int64_t>(tok_row[i]) * a.ldh + c.h_col + k;
+          const f32x4 lo = __builtin_bit_cast(f32x4, load16_global(hp));
+          const f32x4 hi = __builtin_bit_cast(f32x4, load16_global(hp + 4));
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            hf[i][ks][q] = static_cast<T>(lo[q]);
+            hf[i][ks][4 + q] = static_cast<T>(hi[q]);
+          }
         } else {
           hf[i][ks] = load8(static_cast<const T*>(a.h) + static_cast<int64_t>(tok_row[i]) * a.ldh + c.h_col + k);
         }
@@ -610,6 +639,13 @@ __device__ __forceinline__ void compute_chunk(const ApplyArgs& a, int b, const B
       f32x4 acc[kOT];
 #pragma unroll
       for (int ot = 0; ot < kOT; ++ot) acc[ot] = unpack4f<T>(*reinterpret_cast<const u32x2*>(st_row + ot * 16 + oq));
+      if constexpr (kExt) {
+        if (ext.has_bias) {
+#pragma unroll
+          for (int ot = 0; ot < kOT; ++ot)
+            acc[ot] = unpack4f<T>(__builtin_bit_cast(u32x2, round4<T>(acc[ot] + ext.bias[ot])));
+        }
+      }
 #pragma unroll
       for (int ot = 0; ot < kOT; ++ot)
 #pragma unroll
@@ -769,17 +805,17 @@ __device__ __forceinline__ void expand_body(const ApplyArgs& a, int b, int p, co
           if (cn[j].res.ptr != nullptr) load_chunk<T, RANK, kDyn>(a, cn[j], tok0, bfn[j], yqn[j]);
         }
       }
-      if (cur.res.ptr != nullptr) compute_chunk<T, RANK, true, 1>(a, b, blk, tok0, cur, bf, yq, s_h, hsl, stage);
+      if (cur.res.ptr != nullptr) compute_chunk<T, RANK, kHLds, 1>(a, b, blk, tok0, cur, bf, yq, s_h, hsl, stage);
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        if (cn[j].res.ptr != nullptr) compute_chunk<T, RANK, true, 1>(a, b, blk, tok0, cn[j], bfn[j], yqn[j], s_h, hsl, stage);
+        if (cn[j].res.ptr != nullptr) compute_chunk<T, RANK, kHLds, 1>(a, b, blk, tok0, cn[j], bfn[j], yqn[j], s_h, hsl, stage);
       for (int i = 3; i < a.n_sub; ++i) {
         const int oc = p + i * n_owg;
         if (oc >= a.n_ochunks) break;
         cur = out_chunk<T, kSliceH, PA>(a, blk, oc, pre);
         if (cur.res.err != 0 && cur.o_first == 0 && threadIdx.x == 0) flag_error(a.plan.header, cur.res.err);
         load_chunk<T, RANK, kDyn>(a, cur, tok0, bf, yq);
-        if (cur.res.ptr != nullptr) compute_chunk<T, RANK, true, 1>(a, b, blk, tok0, cur, bf, yq, s_h, hsl, stage);
+        if (cur.res.ptr != nullptr) compute_chunk<T, RANK, kHLds, 1>(a, b, blk, tok0, cur, bf, yq, s_h, hsl, stage);
       }
     } else if constexpr (ROLE == kFusedMulti) {
       // Rank 64: chunks after the first load when they are reached (its
@@ -792,10 +828,10 @@ __device__ __forceinline__ void expand_body(const ApplyArgs& a, int b, int p, co
           if (cur.res.err != 0 && cur.o_first == 0 && threadIdx.x == 0) flag_error(a.plan.header, cur.res.err);
           load_chunk<T, RANK, kDyn>(a, cur, tok0, bf, yq);
         }
-        if (cur.res.ptr != nullptr) compute_chunk<T, RANK, true, 1>(a, b, blk, tok0, cur, bf, yq, s_h, hsl, stage);
+        if (cur.res.ptr != nullptr) compute_chunk<T, RANK, kHLds, 1>(a, b, blk, tok0, cur, bf, yq, s_h, hsl, stage);
       }
     } else {
-      compute_chunk<T, RANK, kFusedRole, kFusedRole ? 1 : TILES>(a, b, blk, tok0, cur, bf, yq, s_h, hsl, stage);
+      compute_chunk<T, RANK, kFusedRole ? kHLds : kHGlobal, kFusedRole ? 1 : TILES>(a, b, blk, tok0, cur, bf, yq, s_h, hsl, stage);
     }
   }
 
@@ -1017,6 +1053,94 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
       default: expand_body<T, 8, ROLE, TILES, PA>(a, b, part, blk, t0, s_h, smem.stage(), &s_flag, pre); break;
     }
   }
+}
+
+// ---------------------------------------------------------- V1 expand ----
+//
+// vLLM V1's lora_expand in one launch: expand() on stacked weights, with H in
+// fp32 (rounded to the I/O type as it is loaded), the adapter's bias added to
+// y and rounded before the product, or y overwritten instead of read.  Each of
+// these was a pass of its own over H or y ahead of the expand (52 us at 48
+// tokens and 6144 columns).  Bound by HBM (y read and written); measured on
+// MI355X, a step of four layers' lora_shrink + lora_expand with biases at 48
+// tokens 374 -> 125 us, of two layers without biases at 1000 tokens 135 -> 104 us.
+template <typename T, int RANK, int TILES, int HSRC>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(TILES == 1 ? 5 : RANK == 64 ? 3 : 4)))
+void expand_ext_kernel(const uint32_t* header, const Block* __restrict__ blocks, const int32_t* __restrict__ bperm,
+                       int32_t per_block, ApplyArgs a, ExpandExt x) {
+  using V8 = typename VecOf<T>::v8;
+  constexpr int KS = (RANK + 31) / 32;
+  __shared__ alignas(16) T s_stage[kWaves * 16 * kStageStride];
+  const int b = static_cast<int>(blockIdx.x) / per_block;
+  const int part = static_cast<int>(blockIdx.x) - b * per_block;
+  const int n_blocks = static_cast<int>(header[kHdrNumBlocks]);
+  const Block blk = blocks[b];
+  const int lane = threadIdx.x & 63;
+  const int row = lane & 15;
+  const int32_t tok_in = bperm[static_cast<int64_t>(b) * kBlockTokens + row];
+  if (b == a.n_slots - 1 && part == 0 && threadIdx.x == 0 && n_blocks > a.n_slots)
+    flag_error(a.plan.header, kErrCapacity);
+  if ((b >= n_blocks) | (blk.count <= 0) | (tok_in < -1)) return;
+  const int32_t tok0 = row < blk.count ? tok_in : -1;
+  T* stage = s_stage + (threadIdx.x >> 6) * 16 * kStageStride;
+  const OutChunk<T> c = out_chunk<T, true>(a, blk, part);
+  if (c.res.err != 0 && c.o_first == 0 && threadIdx.x == 0) flag_error(a.plan.header, c.res.err);
+  const int wave = threadIdx.x >> 6;
+  const int ob = c.o_first + wave * (kOT * 16);
+  if (c.res.ptr == nullptr) {
+    // No weights: an expand that overwrites still clears the rows.
+    if (!x.zero_y) return;
+    const YRows z{{u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}}};
+    for (int tt = 0; tt * 16 < blk.count; ++tt) {
+      int32_t tok[2];
+      yrows_tokens(block_token(a, b, tt * 16 + row, blk.count), tok);
+      yrows_store<T>(a, c.y_off, ob, c.o_size, tok, z);
+    }
+    return;
+  }
+  ChunkExt ext;
+  ext.zero_y = x.zero_y != 0;
+  int s = 0;
+  while (s + 1 < a.w.n_slices && part >= a.w.oc_start[s + 1]) ++s;
+  ext.has_bias = x.bias[s] != nullptr;
+  V8 bf[kOT][KS];
+  YRows yq;
+  load_chunk<T, RANK>(a, c, tok0, bf, yq, !ext.zero_y);
+  const T* brow = static_cast<const T*>(x.bias[s]) + static_cast<int64_t>(blk.adapter_id) * x.bias_stride[s];
+#pragma unroll
+  for (int ot = 0; ot < kOT; ++ot) {
+    const int o = ob + ot * 16 + (lane >> 4) * 4;
+    ext.bias[ot] = ext.has_bias && o + 4 <= c.o_size ? unpack4f<T>(*reinterpret_cast<const u32x2*>(brow + o))
+                                                      : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  compute_chunk<T, RANK, HSRC, TILES, true>(a, b, blk, tok0, c, bf, yq, nullptr, 0, stage, ext);
+}
+
+template <typename T, int TILES, int HSRC>
+hipError_t launch_expand_ext_t(const ApplyArgs& a, const ExpandExt& x, hipStream_t stream) {
+  const int64_t n = static_cast<int64_t>(a.n_slots) * a.n_ochunks;
+  if (n <= 0) return hipSuccess;
+  const dim3 grid(static_cast<unsigned>(n));
+  const auto run = [&](auto rank) {
+    expand_ext_kernel<T, decltype(rank)::value, TILES, HSRC><<<grid, kThreads, 0, stream>>>(
+        a.plan.header, a.plan.blocks, a.plan.bperm, a.n_ochunks, a, x);
+  };
+  switch (a.rank) {
+    case 8: run(std::integral_constant<int, 8>{}); break;
+    case 16: run(std::integral_constant<int, 16>{}); break;
+    case 32: run(std::integral_constant<int, 32>{}); break;
+    case 64: run(std::integral_constant<int, 64>{}); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_expand_ext_d(const ApplyArgs& a, const ExpandExt& x, hipStream_t stream) {
+  if (a.tiles > 1)
+    return x.h_f32 ? launch_expand_ext_t<T, kTilesInFlight, kHFloat>(a, x, stream)
+                   : launch_expand_ext_t<T, kTilesInFlight, kHGlobal>(a, x, stream);
+  return x.h_f32 ? launch_expand_ext_t<T, 1, kHFloat>(a, x, stream) : launch_expand_ext_t<T, 1, kHGlobal>(a, x, stream);
 }
 
 // ------------------------------------------------------------- shrink() ----
@@ -1804,6 +1928,15 @@ hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t s
 hipError_t launch_expand(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
   if (a.w.n_a < 1 || a.w.n_a > kMaxSlices) return hipErrorInvalidValue;
   return launch_role<kExpandOnly>(dtype_bf16, a, stream);
+}
+
+hipError_t launch_expand_ext(int dtype_bf16, const ApplyArgs& a, const ExpandExt& x, hipStream_t stream) {
+  // H rows load as 16-byte vectors.
+  const int align = x.h_f32 ? 4 : 8;
+  if (a.w.mode != kStacked || a.w.n_a < 1 || a.w.n_a > kMaxSlices || (reinterpret_cast<uintptr_t>(a.h) % 16) != 0 ||
+      a.ldh % align != 0 || (a.w.n_a > 1 && a.hs1 % align != 0))
+    return hipErrorInvalidValue;
+  return dtype_bf16 ? launch_expand_ext_d<__bf16>(a, x, stream) : launch_expand_ext_d<_Float16>(a, x, stream);
 }
 
 }  // namespace wp

@@ -1815,17 +1815,13 @@ int wp_lora_expand(wp_engine* e, void* y, int64_t y_row_stride, const void* h, i
   if (num_loras <= 0) return fail(WP_ERR_INVALID, "%s: num_loras must be positive", who);
   if ((rc = check_plan_for(e, who, T)) != WP_OK) return rc;
   if (e->plan_T > e->tok_cap) return fail(WP_ERR_CAPACITY, "%s: the table reaches past the engine's H rows", who);
-  PrepArgs p{};
+  ExpandExt x{};
   ApplyArgs a{};
   {
     a = stacked_base(e, rank, num_loras, 1.0f);
-    a.h = e->hbuf;
-    a.ldh = static_cast<int64_t>(n_slices) * rank;
     a.y = y;
     a.ldy = y_row_stride;
-    a.hs1 = rank;
-    a.hs = n_slices * rank;
-    a.w.n_a = n_slices;  // slice s reads H columns [s * rank, (s + 1) * rank)
+    a.w.n_a = n_slices;  // slice s reads its own H
     a.w.n_slices = n_slices;
     const int cols = expand_cols_per_workgroup();
     int oc = 0;
@@ -1846,35 +1842,47 @@ int wp_lora_expand(wp_engine* e, void* y, int64_t y_row_stride, const void* h, i
       a.w.y_off[s] = y_col_offsets[s];
       a.w.oc_start[s] = oc;
       oc += static_cast<int>(ceil_div(out_features[s], cols));
-      p.o_size[s] = out_features[s];
-      p.y_off[s] = y_col_offsets[s];
-      p.bias[s] = add_inputs ? bs : nullptr;
-      p.bias_stride[s] = bs ? bias_stride0[s] : 0;
+      x.bias[s] = add_inputs ? bs : nullptr;
+      x.bias_stride[s] = bs ? bias_stride0[s] : 0;
     }
     a.w.oc_start[n_slices] = oc;
     a.n_ochunks = oc;
   }
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  // The input rounded into the engine's H rows (vLLM's lora_expand casts an
-  // fp32 input to the weights' type before the product), the windows zeroed
-  // when the expand overwrites, the biases added when it adds.
-  p.plan = plan_view(e);
-  p.n_slots = a.n_slots;
-  p.n_slices = n_slices;
-  p.num_ids = num_loras;
-  p.rank = rank;
-  p.h_src = h;
-  p.h_f32 = h_is_f32 ? 1 : 0;
-  p.h_slice_stride = h_slice_stride;
-  p.h_row_stride = h_row_stride;
-  p.h_dst = e->hbuf;
-  p.ldh_dst = n_slices * rank;
-  p.y = y;
-  p.ldy = y_row_stride;
-  p.zero_y = add_inputs ? 0 : 1;
-  WP_HIP(launch_prep(dtype == WP_DTYPE_BF16, p, stream));
-  WP_HIP(launch_expand(dtype == WP_DTYPE_BF16, a, stream));
+  x.zero_y = add_inputs ? 0 : 1;
+  // The expand reads the caller's H in place (fp32 rounded as it is loaded:
+  // vLLM's lora_expand casts an fp32 input to the weights' type before the
+  // product), if its rows load as 16-byte vectors and a slice's offset fits
+  // the kernel's 32-bit column; otherwise a pass of its own packs it into the
+  // engine's H rows first.
+  const int64_t vec = h_is_f32 ? 4 : 8;
+  const bool in_place = aligned(h, 16) && h_row_stride % vec == 0 &&
+                        (n_slices == 1 || (h_slice_stride % vec == 0 && h_slice_stride * (n_slices - 1) < (int64_t{1} << 31)));
+  if (in_place) {
+    a.h = const_cast<void*>(h);
+    a.ldh = h_row_stride;
+    a.hs1 = static_cast<int32_t>(n_slices == 1 ? 0 : h_slice_stride);
+    x.h_f32 = h_is_f32 ? 1 : 0;
+  } else {
+    PrepArgs p{};
+    p.plan = plan_view(e);
+    p.n_slots = a.n_slots;
+    p.n_slices = n_slices;
+    p.num_ids = num_loras;
+    p.rank = rank;
+    p.h_src = h;
+    p.h_f32 = h_is_f32 ? 1 : 0;
+    p.h_slice_stride = h_slice_stride;
+    p.h_row_stride = h_row_stride;
+    p.h_dst = e->hbuf;
+    p.ldh_dst = n_slices * rank;
+    WP_HIP(launch_prep(dtype == WP_DTYPE_BF16, p, stream));
+    a.h = e->hbuf;
+    a.ldh = static_cast<int64_t>(n_slices) * rank;
+    a.hs1 = rank;
+  }
+  WP_HIP(launch_expand_ext(dtype == WP_DTYPE_BF16, a, x, stream));
   return WP_OK;
 }
 

@@ -626,8 +626,9 @@ class WarpPipeEngine:
         y[t, off_s + o] = rn((add_inputs ? y'[t, off_s + o] : 0) + rn(h[s][t]) . B_s[id_t][o]^T)
         with slice windows consecutive from offset_start and y' = rn(y + bias)
         where lora_bias_stacked[s] is given (add_inputs only).  h: [n, T, r]
-        fp32 (rounded to y's dtype first, as V1 casts it) or y's dtype.  Two
-        launches; tokens without an adapter keep their rows."""
+        fp32 (rounded to y's dtype first, as V1 casts it) or y's dtype.  One
+        launch (two when h's rows are not whole 16-byte vectors); tokens without
+        an adapter keep their rows."""
         wbs = list(lora_b_stacked)
         n = len(wbs)
         rank = int(wbs[0].size(-1))

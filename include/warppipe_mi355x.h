@@ -315,8 +315,9 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
  * with y' = rn(y + bias[s][id_t]) where bias[s] is given (add_inputs only,
  * as V1 applies the bias before an expand that adds).  h is fp32 (h_is_f32;
  * rounded to the I/O type first, as V1's lora_expand casts it) or the I/O
- * type; slice s at h + s * h_slice_stride, rows h_row_stride apart.  Two
- * launches.  WP_NOT_HANDLED for a rank without kernels. */
+ * type; slice s at h + s * h_slice_stride, rows h_row_stride apart.  One
+ * launch, or two when h's rows are not whole 16-byte vectors (they are then
+ * packed first).  WP_NOT_HANDLED for a rank without kernels. */
 int wp_lora_expand(wp_engine* e, void* y, int64_t y_row_stride, const void* h, int32_t h_is_f32, int64_t h_slice_stride,
                    int64_t h_row_stride, int32_t n_slices, const void* const* wb, const int64_t* wb_stride0,
                    const int32_t* out_features, const int32_t* y_col_offsets, const void* const* bias,

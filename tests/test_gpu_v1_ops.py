@@ -349,3 +349,35 @@ def test_random_v1_calls(wrapper, seed):
     assert_close(z, zref, f"add_expand seed {seed}")
     assert wrapper.calls == ["update_metadata"], wrapper.calls
     assert pw._engine.device_errors() == 0
+
+
+@pytest.mark.parametrize("T", [17, 600])
+@pytest.mark.parametrize("rows", ["fp32", "fp32_odd", "io", "io_odd"])
+@pytest.mark.parametrize("rank,add_inputs", [(8, True), (32, False), (64, True)])
+def test_lora_expand_h_rows_and_modes(T, rows, rank, add_inputs):
+    """lora_expand over the H rows it loads in place (fp32 or the I/O type,
+    whole 16-byte vectors) and those it packs first (odd row strides), at 16-
+    and 64-token blocks, ragged chunk edges (260, 4 and 516 columns), with a
+    bias on one slice, and overwriting; a token whose id is past the weights
+    keeps its row, or is cleared by the overwriting form."""
+    dtype, L, outs = torch.bfloat16, 5, (260, 4, 516)
+    announce(f"lora_expand {rows} T={T} r={rank} add_inputs={add_inputs}")
+    eng = WarpPipeEngine(WarpPipeConfig(max_tokens=1024))
+    ids = torch.from_numpy(np.random.default_rng(T).integers(-1, L, size=T).astype(np.int64))
+    _, wbs, bias = weights(L, rank, 64, outs, dtype, 700, (1,))
+    pad = 1 if rows.endswith("odd") else 8
+    h = randn((3, T, rank + pad), 701, torch.float32 if rows.startswith("fp32") else dtype)
+    y0 = randn((T, sum(outs) + 4), 702, dtype)
+    dev_ids = ids.clone()
+    dev_ids[3] = L + 2
+    assert eng.build_seg_bounds(dev_ids.cuda())
+    y = y0.cuda()
+    assert eng.lora_expand(y, h.cuda(), wbs, outs, 4, add_inputs, bias if add_inputs else None)
+    torch.cuda.synchronize()
+    ids[3] = -1
+    ref = v1_ops.apply_bias(y0, cpu(bias) if add_inputs else None, outs, ids, 4)
+    ref = v1_ops.lora_expand(ref, h, cpu(wbs), outs, ids, 4, add_inputs)
+    if not add_inputs:
+        ref[3, 4:] = 0
+    assert_close(y, ref, f"lora_expand {rows}")
+    assert eng.device_errors() == 1
