@@ -155,8 +155,9 @@ constexpr int kShrinkSlices = 8;
 
 // One launch: shrink + expand of a whole add_lora call (partials, counters).
 hipError_t launch_fused(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
-// shrink(): one workgroup per (block, d-range) computes every rank row; the
-// block's last workgroup to finish sums the d-ranges into H[token].
+// shrink(): one workgroup per (block, group of A slices of at most 64 rows,
+// d-range); the block's last workgroup to finish sums the d-ranges into
+// H[token], slice s at element s * a.ldy of an H row.
 hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
 // shrink() of decode-sized plans: the fused kernel's shrink workgroups
 // (kShrinkRowsFused rows x d-range) and one reducer per block writing H;

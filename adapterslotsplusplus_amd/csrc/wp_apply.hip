@@ -1146,62 +1146,95 @@ hipError_t launch_expand_ext_d(const ApplyArgs& a, const ExpandExt& x, hipStream
 // ------------------------------------------------------------- shrink() ----
 //
 // shrink(), and the shrink half of large-plan add_lora calls: one workgroup
-// per (block, d-range) computes every rank row of the block, so each X
-// element is read once per call.  The d-range is streamed in K-slices of
-// kSliceK elements, software pipelined one slice ahead: the slice of A
-// (rank rows x kSliceK) is loaded once per workgroup and shared by the four
+// per (block, group of A slices, d-range) computes every rank row of the group
+// -- up to 64 rows, whole slices, so slices that share X read it once -- and
+// each X element is read once per group.  The d-range is streamed in K-slices
+// of kSliceK elements, software pipelined one slice ahead: the slice of A
+// (rows x kSliceK) is loaded once per workgroup and shared by the four
 // waves through LDS (double buffered), and each wave, which owns one
-// 16-token tile, loads its X fragments straight into registers.  The
-// block's d-ranges are summed by its last workgroup to finish (a per-block
-// counter), in d-range order, so the bits do not depend on timing; nothing
-// waits on another workgroup.
+// 16-token tile, loads its X through a tile of its own.  The
+// block's d-ranges are summed by its last workgroup to finish (a counter per
+// block and group), in d-range order, so the bits do not depend on timing;
+// nothing waits on another workgroup.
+//
+// A launch takes 10 us however small (a chain of loads, eight slices two at a
+// time, the last arriver's sum), and at 8192 tokens one compute unit's read
+// rate bounds it (X and A of three workgroups at about 40 GB/s).  So one launch
+// for every A slice, with X read once per 64 rows, replaced one launch each:
+// q/k/v with three A of rank 16, call total on MI355X 53.3 -> 34.3 us at 2048
+// tokens, 116 -> 84 at 8192 (rank 64: 79 -> 64, 157 -> 132).  512-column
+// d-ranges are slower from 2048 tokens up (8192, rank 64: 64.9 -> 73.5 us).
 constexpr int kSliceK = 128;
 constexpr int kSliceStride = kSliceK + 8;  // LDS row stride of an A slice: 16-byte skew per row
+// Words between the counters of a block's slice groups (64 bytes).
+constexpr int kGroupCounter = kCounterStride / kMaxSlices;
 
-template <typename T, int MAXR, bool kMixed>
+// MT: 16-row MFMA tiles of a group's rows (of the largest rank if kMixed).
+// The leading scalar arguments arrive in SGPRs at wave launch, as apply_kernel's do.
+template <typename T, int MT, bool kMixed>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kShrinkWavesPerSimd)))
-void shrink_kernel(ApplyArgs a) {
+void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, const int32_t* __restrict__ bperm,
+                   int32_t n_kc, int32_t per_block, int32_t per_group, ApplyArgs a) {
   using V8 = typename VecOf<T>::v8;
-  constexpr int MT = (MAXR + 15) / 16;          // 16-row MFMA tiles of the largest rank
   constexpr int KS = kSliceK / 32;              // K-steps per slice
   constexpr int XL = 16 * kSliceK / (64 * 8);   // a wave's whole-row X loads per slice (4)
+  const uint32_t ka_touch = touch_kernel_args_issue<static_cast<int>(sizeof(ApplyKernelArgs))>();
   __shared__ T s_a[2][MT * 16 * kSliceStride];
   // Each wave's X tile of the current slice: only that wave reads it, after
   // writing it, so one buffer suffices.
   __shared__ T s_x[kWaves][16 * kSliceStride];
   __shared__ int s_last;
   const int tid = static_cast<int>(threadIdx.x);
-  const int n_kc = a.n_chunks;
-  const int b = static_cast<int>(blockIdx.x) / n_kc;
-  const int c = static_cast<int>(blockIdx.x) - b * n_kc;
-  trace_stamp(a, 0);
-  trace_hw(a);
-  const int n_blocks = static_cast<int>(a.plan.header[kHdrNumBlocks]);
-  if (b == a.n_slots - 1 && c == 0 && tid == 0 && n_blocks > a.n_slots) flag_error(a.plan.header, kErrCapacity);
-  if (b >= n_blocks) return;
-  const Block blk = a.plan.blocks[b];
-  const Resolved<T> res = resolve_a<T>(a, blk);
-  if (res.ptr == nullptr) {
-    if (res.err != 0 && c == 0 && tid == 0) flag_error(a.plan.header, res.err);
-    return;
-  }
-  trace_tag(a, 3u | (static_cast<uint64_t>(b) << 8) | (static_cast<uint64_t>(c) << 32));
-  trace_stamp(a, 1);
-  const int rank = kMixed ? res.rank : MAXR;
-  const int n_mt = kMixed ? (rank + 15) >> 4 : MT;
-  const int d = a.d_model;
-  // The d-range [c * dc, ...) in groups of kShrinkSlices slices; k0/k1 are
-  // the current group's bounds.
-  const int kc_end = min((c + 1) * a.dc, d);
-  int k0 = c * a.dc;
-  int k1 = min(k0 + kShrinkSlices * kSliceK, kc_end);
+  const int b = static_cast<int>(blockIdx.x) / per_block;
+  const int part = static_cast<int>(blockIdx.x) - b * per_block;
+  const int grp = part / n_kc;
+  const int c = part - grp * n_kc;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int row = lane & 15;
   const int kq = (lane >> 4) * 8;
   const int tl = wave * 16 + row;  // this lane's token slot in the block (MFMA layout)
-  const int32_t* bp = a.plan.bperm + static_cast<int64_t>(b) * kBlockTokens;
-  const int32_t tok = tl < blk.count ? bp[tl] : -1;
+  const int xrow = lane >> 4;
+  const int xcol = (lane & 15) * 8;
+  trace_stamp(a, 0);
+  trace_hw(a);
+  // Independent loads, issued together: the exit test reads them all.
+  const int32_t* bp = bperm + static_cast<int64_t>(b) * kBlockTokens;
+  const int n_blocks = static_cast<int>(header[kHdrNumBlocks]);
+  const Block blk = blocks[b];
+  const int32_t tok_in = bp[tl];
+  int32_t xtok[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) xtok[i] = bp[wave * 16 + xrow + 4 * i];
+  PreEntry pre;
+  if (a.w.mode == kTable && a.w.a_base[0] != nullptr) {
+    pre.en = load_entry(static_cast<const Entry*>(a.w.a_base[0]) + b);
+    pre.ok = header[kHdrTableVer] == header[kHdrPlanVer];
+  }
+  if (b == a.n_slots - 1 && part == 0 && tid == 0 && n_blocks > a.n_slots) flag_error(a.plan.header, kErrCapacity);
+  touch_kernel_args_wait(ka_touch);
+  bool none = (b >= n_blocks) | (blk.count <= 0) | (tok_in < -1);
+#pragma unroll
+  for (int i = 0; i < XL; ++i) none |= xtok[i] < -1;
+  if (none) return;
+  const Resolved<T> res = resolve_a<T>(a, blk, 0, pre);
+  if (res.ptr == nullptr) {
+    if (res.err != 0 && part == 0 && tid == 0) flag_error(a.plan.header, res.err);
+    return;
+  }
+  trace_tag(a, 3u | (static_cast<uint64_t>(b) << 8) | (static_cast<uint64_t>(part) << 32));
+  trace_stamp(a, 1);
+  const int rank = kMixed ? res.rank : a.rank;
+  const int s0 = kMixed ? 0 : grp * per_group;  // the group's first A slice
+  const int n_rows = kMixed ? rank : min(per_group, a.w.n_a - s0) * rank;
+  const int n_mt = kMixed ? (rank + 15) >> 4 : MT;
+  const int d = a.d_model;
+  // The d-range [c * dc, ...) in passes of kShrinkSlices slices; k0/k1 are the current
+  // pass's bounds.
+  const int kc_end = min((c + 1) * a.dc, d);
+  int k0 = c * a.dc;
+  int k1 = min(k0 + kShrinkSlices * kSliceK, kc_end);
+  const int32_t tok = tl < blk.count ? tok_in : -1;
   const bool wave_live = wave * 16 < blk.count;
   // Every load below is unconditional, at an address clamped into the
   // operand (a missing token reads X row 0, a rank row past the adapter's
@@ -1214,31 +1247,37 @@ void shrink_kernel(ApplyArgs a) {
   // LDS tile and read back in the MFMA layout: X loaded straight in the MFMA
   // layout moves 64 bytes of 16 rows per instruction, 4.6 vs 6.2 TB/s for
   // the same bytes, measured on MI355X.
-  const int xrow = lane >> 4;
-  const int xcol = (lane & 15) * 8;
   const T* xr[XL];
 #pragma unroll
   for (int i = 0; i < XL; ++i) {
     const int t = wave * 16 + xrow + 4 * i;
-    const int32_t tk = t < blk.count ? bp[t] : -1;
-    xr[i] = static_cast<const T*>(a.x) + static_cast<int64_t>(tk >= 0 ? tk : 0) * a.ldx;
+    const int32_t tk = t < blk.count ? xtok[i] : 0;
+    xr[i] = static_cast<const T*>(a.x) + static_cast<int64_t>(tk) * a.ldx;
   }
   T* sx = s_x[wave];
-  // A slice loads: thread t moves 8 elements of rows t/16 + 16p.
+  // A slice loads: thread t moves 8 elements of rows t/16 + 16p (past the
+  // group's rows, of the last one again).
   const int arow = tid >> 4;
   const int acol = (tid & 15) * 8;
-  // Element offsets from the adapter's A (rank x d < 2^31 elements).
-  const int arow0 = min(arow, rank - 1) * d;
+  const T* ar[MT];
+#pragma unroll
+  for (int p = 0; p < MT; ++p) {
+    const int r = min(p * 16 + arow, n_rows - 1);
+    if (kMixed || a.w.n_a == 1) {
+      ar[p] = res.ptr + static_cast<int64_t>(r) * d;
+    } else {
+      const int s = r / rank;
+      ar[p] = static_cast<const T*>(a.w.a_base[s0 + s]) + static_cast<int64_t>(blk.adapter_id) * a.w.a_stride[s0 + s] +
+              static_cast<int64_t>(r - s * rank) * d;
+    }
+  }
   struct Slice {
     u32x4 a[MT];
     u32x4 x[XL];
   };
   auto load_slice = [&](Slice& sl, int ks0) {
 #pragma unroll
-    for (int p = 0; p < MT; ++p) {
-      const int off = (kMixed ? min(p * 16 + arow, rank - 1) * d : arow0 + p * 16 * d) + min(ks0 + acol, k1 - 8);
-      sl.a[p] = load16_global(res.ptr + off);
-    }
+    for (int p = 0; p < MT; ++p) sl.a[p] = load16_global(ar[p] + min(ks0 + acol, k1 - 8));
 #pragma unroll
     for (int i = 0; i < XL; ++i) sl.x[i] = load16_global(xr[i] + min(ks0 + xcol, k1 - 8));
   };
@@ -1282,63 +1321,64 @@ void shrink_kernel(ApplyArgs a) {
   // Blocks of one adapter read the same A slices; each block starts at a
   // different slice of its range (rotation by block index) so that they do
   // not all hit the same lines at once.
-  Slice s0, s1;
+  Slice q0, q1;
   for (; k0 < kc_end; k0 += kShrinkSlices * kSliceK, k1 = min(k0 + kShrinkSlices * kSliceK, kc_end)) {
     const int n_sl = (k1 - k0 + kSliceK - 1) / kSliceK;
     const int rot = b % n_sl;
     auto slice_k = [&](int i) { return k0 + (i + rot < n_sl ? i + rot : i + rot - n_sl) * kSliceK; };
-    load_slice(s0, slice_k(0));
-    load_slice(s1, slice_k(1 % n_sl));
+    load_slice(q0, slice_k(0));
+    load_slice(q1, slice_k(1 % n_sl));
 #pragma unroll
     for (int i = 0; i < kShrinkSlices; i += 2) {
-      run_slice(s0, 0, slice_k(i % n_sl), i < n_sl, i + 2 < kShrinkSlices, slice_k((i + 2) % n_sl));
-      run_slice(s1, 1, slice_k((i + 1) % n_sl), i + 1 < n_sl, i + 3 < kShrinkSlices, slice_k((i + 3) % n_sl));
+      run_slice(q0, 0, slice_k(i % n_sl), i < n_sl, i + 2 < kShrinkSlices, slice_k((i + 2) % n_sl));
+      run_slice(q1, 1, slice_k((i + 1) % n_sl), i + 1 < n_sl, i + 3 < kShrinkSlices, slice_k((i + 3) % n_sl));
     }
   }
   trace_stamp(a, 2);
-  // acc[m]: ranks m*16 + 4*(lane/16) + [0, 4) of token slot tl.
+  // acc[m]: rows m*16 + 4*(lane/16) + [0, 4) of token slot tl.
   const int rq = (lane >> 4) * 4;
-  T* H = static_cast<T*>(a.h);
   // fp32 H (vLLM's lora_shrink buffer): alpha * sum added to it, unrounded.
   const bool f32 = a.h_f32 != 0;
-  auto put_h = [&](int64_t at, f32x4 v) {
+  auto put_h = [&](int32_t token, int r, f32x4 v) {
+    const int s = kMixed || a.w.n_a == 1 ? 0 : r / rank;
+    const int64_t at = static_cast<int64_t>(token) * a.ldh + (s0 + s) * a.ldy + (r - s * rank);
     if (f32) {
       f32x4* hp = reinterpret_cast<f32x4*>(static_cast<float*>(a.h) + at);
       *hp = *hp + v;
     } else {
-      store4(H + at, v);
+      store4(static_cast<T*>(a.h) + at, v);
     }
   };
   if (n_kc == 1) {
     if (tok >= 0) {
 #pragma unroll
       for (int m = 0; m < MT; ++m)
-        if (m * 16 + rq < rank) put_h(static_cast<int64_t>(tok) * a.ldh + m * 16 + rq, acc[m] * res.alpha);
+        if (m * 16 + rq < n_rows) put_h(tok, m * 16 + rq, acc[m] * res.alpha);
     }
     return;
   }
   // Partial of this d-range, stored coherently; the stores have landed
   // before the count (s_waitcnt), so the last workgroup sees them all.
+  float* prow = a.part + static_cast<int64_t>(blk.first) * a.hs + s0 * rank;
+  const int64_t cs = static_cast<int64_t>(a.ptok) * a.hs;
   if (tok >= 0) {
-    float* prow = a.part + (static_cast<int64_t>(c) * a.ptok + blk.first + tl) * a.hs;
 #pragma unroll
     for (int m = 0; m < MT; ++m)
-      if (m * 16 + rq < rank) coherent_store_f4(prow + m * 16 + rq, acc[m]);
+      if (m * 16 + rq < n_rows) coherent_store_f4(prow + c * cs + static_cast<int64_t>(tl) * a.hs + m * 16 + rq, acc[m]);
   }
   wait_vm();
   __syncthreads();
-  uint32_t* counter = &a.consumed[static_cast<int64_t>(b) * kCounterStride];
+  uint32_t* counter = &a.consumed[static_cast<int64_t>(b) * kCounterStride + grp * kGroupCounter];
   if (tid == 0) s_last = atomic_add_u(counter, 1u) == static_cast<unsigned>(n_kc - 1) ? 1 : 0;
   __syncthreads();
   trace_stamp(a, 3);
   if (s_last == 0) return;
-  // Last workgroup of the block: H = rn(alpha * sum_c part[c]) in d-range
-  // order, then the counter is reset for the next call.  The partials are
-  // left as they are: every launch writes each word it later reads (the
+  // Last workgroup of the block and group: H = rn(alpha * sum_c part[c]) in
+  // d-range order, then the counter is reset for the next call.  The partials
+  // are left as they are: every launch writes each word it later reads (the
   // buffer is shrink()'s own, not the fused calls' with its empty pattern).
-  const int r4 = rank >> 2;
+  const int r4 = n_rows >> 2;
   const int units = blk.count * r4;
-  const int64_t cs = static_cast<int64_t>(a.ptok) * a.hs;
   // A thread's units are tid + 256 i (at most kBlockTokens * kMaxRank / 4 /
   // 256 = 4); their loads go out together, four d-ranges at a time.
   constexpr int kUnits = kBlockTokens * kMaxRank / 4 / kThreads;
@@ -1348,7 +1388,7 @@ void shrink_kernel(ApplyArgs a) {
   for (int i = 0; i < kUnits; ++i) {
     const int u = min(tid + i * kThreads, units - 1);
     const int j = u / r4;
-    p0[i] = a.part + (static_cast<int64_t>(blk.first) + j) * a.hs + (u - j * r4) * 4;
+    p0[i] = prow + static_cast<int64_t>(j) * a.hs + (u - j * r4) * 4;
     sum[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   for (int c0 = 0; c0 < n_kc; c0 += 4) {
@@ -1368,8 +1408,7 @@ void shrink_kernel(ApplyArgs a) {
     const int u = tid + i * kThreads;
     if (u < units) {
       const int j = u / r4;
-      const int32_t tj = a.plan.bperm[static_cast<int64_t>(b) * kBlockTokens + j];
-      put_h(static_cast<int64_t>(tj) * a.ldh + (u - j * r4) * 4, sum[i] * res.alpha);
+      put_h(bp[j], (u - j * r4) * 4, sum[i] * res.alpha);
     }
   }
   if (tid == 0) atomic_store_u(counter, 0u);
@@ -1378,19 +1417,26 @@ void shrink_kernel(ApplyArgs a) {
 
 template <typename T>
 hipError_t launch_shrink_t(const ApplyArgs& a0, hipStream_t stream) {
-  const int64_t n = static_cast<int64_t>(a0.n_slots) * a0.n_chunks;
+  const int per_group = a0.rank == 0 ? 1 : std::min(a0.w.n_a, kMaxRank / a0.rank);
+  const int per_block = a0.n_chunks * ((a0.w.n_a + per_group - 1) / per_group);
+  const int64_t n = static_cast<int64_t>(a0.n_slots) * per_block;
   if (n <= 0) return hipSuccess;
   const dim3 grid(static_cast<unsigned>(n));
   ApplyArgs a = a0;
   if (a.trace != nullptr && n * kTraceWords > a.trace_words) a.trace = nullptr;
-  switch (a.rank) {
-    case 8: shrink_kernel<T, 8, false><<<grid, kThreads, 0, stream>>>(a); break;
-    case 16: shrink_kernel<T, 16, false><<<grid, kThreads, 0, stream>>>(a); break;
-    case 32: shrink_kernel<T, 32, false><<<grid, kThreads, 0, stream>>>(a); break;
-    case 64: shrink_kernel<T, 64, false><<<grid, kThreads, 0, stream>>>(a); break;
-    case 0:  // mixed ranks: each block's adapter decides, up to kMaxRank
-      shrink_kernel<T, kMaxRank, true><<<grid, kThreads, 0, stream>>>(a);
-      break;
+  const auto run = [&](auto mt, auto mixed) {
+    shrink_kernel<T, decltype(mt)::value, decltype(mixed)::value><<<grid, kThreads, 0, stream>>>(
+        a.plan.header, a.plan.blocks, a.plan.bperm, a.n_chunks, per_block, per_group, a);
+  };
+  if (a.rank == 0) {  // mixed ranks: each block's adapter decides, up to kMaxRank
+    run(std::integral_constant<int, kMaxRank / 16>{}, std::true_type{});
+    return hipGetLastError();
+  }
+  switch ((per_group * a.rank + 15) / 16) {
+    case 1: run(std::integral_constant<int, 1>{}, std::false_type{}); break;
+    case 2: run(std::integral_constant<int, 2>{}, std::false_type{}); break;
+    case 3: run(std::integral_constant<int, 3>{}, std::false_type{}); break;
+    case 4: run(std::integral_constant<int, 4>{}, std::false_type{}); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -1916,7 +1962,9 @@ hipError_t launch_fused(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) 
   return a.n_sub > 1 ? launch_role<kFusedMulti>(dtype_bf16, a, stream) : launch_role<kFused>(dtype_bf16, a, stream);
 }
 hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
-  if (a.n_chunks < 1 || a.n_chunks > kMaxChunks || a.w.n_a != 1) return hipErrorInvalidValue;
+  if (a.n_chunks < 1 || a.w.n_a < 1 || a.w.n_a > kMaxSlices || a.n_chunks * a.hs > kMaxChunks * kMaxRank ||
+      (a.w.n_a > 1 && (a.w.mode != kStacked || a.rank == 0)))
+    return hipErrorInvalidValue;
   return dtype_bf16 ? launch_shrink_t<__bf16>(a, stream) : launch_shrink_t<_Float16>(a, stream);
 }
 hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {

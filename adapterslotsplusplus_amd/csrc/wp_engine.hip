@@ -160,12 +160,13 @@ inline void shrink_small_split(int d, int rank, ApplyArgs* a) {
   a->n_sub = 1;
 }
 
-// d-ranges of a shrink() launch: one workgroup per block and d-range, every
-// rank row; a d-range is kShrinkSlices x 128 columns (a multiple of that
-// past kMaxChunks ranges).
+// d-ranges of a shrink() launch: kShrinkSlices x 128 columns each (a multiple
+// of that where more ranges than kMaxChunks, or more partials than
+// kMaxChunks x kMaxRank per token, would be needed).
 inline void shrink_range_split(int d, ApplyArgs* a) {
   const int group = kShrinkSlices * 128;
-  const int64_t n = std::min<int64_t>(ceil_div(d, group), kMaxChunks);
+  const int64_t most = std::max(1, kMaxChunks * kMaxRank / std::max(a->hs, kMaxRank));
+  const int64_t n = std::min<int64_t>(ceil_div(d, group), most);
   a->dc = static_cast<int>(ceil_div(ceil_div(d, n), group) * group);
   a->n_chunks = static_cast<int>(ceil_div(d, a->dc));
   a->srows = 0;
@@ -1436,15 +1437,9 @@ int add_lora_impl(wp_engine* e, const char* who, void* y, const void* x, int32_t
     shrink_range_split(d_model, &a);
     a.part = e->spart;
     a.ptok = e->tok_cap;
-    for (int sa = 0; sa < n_a; ++sa) {
-      ApplyArgs as = a;
-      as.w.n_a = 1;
-      as.hs = as.hs1 = rank;  // the d-range partials' row (a single A slice)
-      as.w.a_base[0] = a.w.a_base[sa];
-      as.w.a_stride[0] = a.w.a_stride[sa];
-      as.h = static_cast<char*>(e->hbuf) + sizeof(uint16_t) * static_cast<size_t>(sa) * rank;
-      WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, as, stream));
-    }
+    ApplyArgs as = a;
+    as.ldy = rank;  // slice s at column s * rank of an H row
+    WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, as, stream));
     WP_HIP(launch_expand(dtype == WP_DTYPE_BF16, a, stream));
     return WP_OK;
   }
@@ -1732,26 +1727,38 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
   if ((rc = check_plan_for(e, who, T)) != WP_OK) return rc;
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
+  ApplyArgs a = stacked_base(e, rank, num_loras, scale);
+  a.x = x;
+  a.ldx = d_model;
+  a.d_model = d_model;
+  a.w.n_a = n_slices;
   for (int s = 0; s < n_slices; ++s) {
-    ApplyArgs a = stacked_base(e, rank, num_loras, scale);
-    a.x = x;
-    a.ldx = d_model;
-    a.d_model = d_model;
-    a.w.a_base[0] = wa[s];
-    a.w.a_stride[0] = wa_stride0[s];
-    a.h = out + s * out_slice_stride;
-    a.ldh = out_row_stride;
-    a.h_f32 = 1;
-    if (e->plan_bt <= 16) {
-      shrink_small_split(d_model, rank, &a);
-      a.red_first = 2 * static_cast<int64_t>(a.n_slots) <= static_cast<int64_t>(e->n_cu) * shrink_small_waves_per_simd() ? 1 : 0;
-      WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, a, stream));
-    } else {
-      shrink_range_split(d_model, &a);
-      a.part = e->spart;
-      a.ptok = e->tok_cap;
-      WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, a, stream));
+    a.w.a_base[s] = wa[s];
+    a.w.a_stride[s] = wa_stride0[s];
+  }
+  a.hs1 = rank;
+  a.hs = n_slices * rank;
+  a.h = out;
+  a.ldh = out_row_stride;
+  a.ldy = out_slice_stride;
+  a.h_f32 = 1;
+  if (e->plan_bt <= 16) {
+    for (int s = 0; s < n_slices; ++s) {
+      ApplyArgs as = a;
+      as.w.n_a = 1;
+      as.hs = rank;
+      as.w.a_base[0] = wa[s];
+      as.w.a_stride[0] = wa_stride0[s];
+      as.h = out + s * out_slice_stride;
+      shrink_small_split(d_model, rank, &as);
+      as.red_first = 2 * static_cast<int64_t>(as.n_slots) <= static_cast<int64_t>(e->n_cu) * shrink_small_waves_per_simd() ? 1 : 0;
+      WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, as, stream));
     }
+  } else {
+    shrink_range_split(d_model, &a);
+    a.part = e->spart;
+    a.ptok = e->tok_cap;
+    WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, a, stream));
   }
   return WP_OK;
 }

@@ -14,7 +14,7 @@ from adapterslotsplusplus_amd import punica_wrapper as pw
 from adapterslotsplusplus_amd.lora_linear import DraftLoRAContext, WarpPipeLoRAPackedLinear
 from oracle import bgmv
 from oracle import segments as so
-from tests.helpers import announce, assert_close, randn, seeds
+from tests.helpers import announce, assert_close, h_tie_flips, randn, seeds
 
 pytestmark = pytest.mark.gpu
 
@@ -301,4 +301,32 @@ def test_packed_linear_matches_separate_projections():
             delta = torch.bmm(h.float().unsqueeze(1), B.float()[ii].transpose(1, 2).contiguous())[:, 0]
             ref = torch.where(ok[:, None], (base.float() + delta).to(dt), base)
             assert_close(out["qkv"][i], ref, f"replay {rep} projection {i}")
+    assert engine.device_errors() == 0
+
+
+@pytest.mark.parametrize("rank,n", [(8, 2), (8, 3), (16, 3), (16, 4), (32, 3), (64, 2), (64, 4)])
+@pytest.mark.parametrize("d", [64, 1000, 2056])
+def test_large_plan_slice_groups(rank, n, d):
+    """Plans past the fused calls' size: a shrink workgroup computes every rank
+    row of as many A slices as make 64 rows, so groups of 16, 24, 48 and 64
+    rows, a last group of one slice, and d-ranges that end inside a slice.
+    Tolerance: the repository's, plus one H rounding step times |B| where an
+    exact H lies within fp32 summation error of a rounding midpoint."""
+    dtype = torch.bfloat16 if d == 1000 else torch.float16
+    announce(f"large-plan slice groups r={rank} n={n} d={d} {dtype}")
+    T, L = 4500, 7
+    idx = torch.sort(torch.from_numpy(np.random.default_rng(rank + n).integers(-1, L, size=T))).values
+    outs = [64, 20, 132, 36][:n]
+    idx, x, was, wbs, y0 = inputs(T, L, rank, d, outs, dtype, 800, idx)
+    offs = [sum(outs[:i]) for i in range(n)]
+    engine = WarpPipeEngine()
+    y = run(engine, idx, x, was, wbs, y0, 0.5, offs)
+    ref = bgmv.add_lora_nslice(y0, x, was, wbs, 0.5, so.seg_bounds(idx.numpy()).tolist(), offs)
+    slack = torch.zeros(y0.shape, dtype=torch.float32)
+    for a in range(L):
+        rows = torch.nonzero(idx == a).flatten()
+        for i, o in enumerate(outs):
+            flips = h_tie_flips(x[rows], was[i][a, 0], 0.5, dtype)
+            slack[rows, offs[i]:offs[i] + o] += (flips @ wbs[i][a, 0].double().abs().T).float()
+    assert_close(y, ref, f"slice groups r={rank} n={n} d={d}", slack=slack)
     assert engine.device_errors() == 0
