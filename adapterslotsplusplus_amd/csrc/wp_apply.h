@@ -91,9 +91,16 @@ constexpr uint32_t kDefaultSpinLimit = 1u << 17;
 // buffer's repair after a give-up); m may be null.
 // bentries (may be null): each block's adapter-table entry at the table
 // version left in header[kHdrPlanVer] (Weights::a_base in table mode).
+// fine (bt > kFineTokens only; may be null): the same tokens in a second table
+// of kFineTokens-token blocks, all of block_cap slots.
+struct FinePlan {
+  Block* blocks;
+  int32_t* bperm;
+  Entry* bentries;
+};
 hipError_t launch_plan(const void* idx, int idx_is_int64, int T, uint32_t* header, Segment* segments, Block* blocks,
-                       int32_t* perm, int32_t* bperm, Entry* bentries, int seg_cap, int block_cap, int bt,
-                       const Maint* m, hipStream_t stream);
+                       int32_t* perm, int32_t* bperm, Entry* bentries, const FinePlan* fine, int seg_cap, int block_cap,
+                       int bt, const Maint* m, hipStream_t stream);
 // The plan build's maintenance alone (one workgroup), for eager calls that
 // run between plan builds.
 hipError_t launch_maintain(uint32_t* header, const Maint& m, hipStream_t stream);

@@ -262,7 +262,7 @@ __device__ __forceinline__ bool wait_partials(const ApplyArgs& a, const Block& b
     const int n_rg = (rank + a.srows - 1) / a.srows;
     const int per_a = a.n_chunks * n_rg;
     const int n_probe = PA ? per_a * a.w.n_a : per_a;
-    // Word offsets into the partial buffer (at most 16 x 512 x 256 words).
+    // Word offsets into the partial buffer (at most 1024 x 8192 words).
     constexpr uint32_t kNone = 0xFFFFFFFFu;
     uint32_t probe[kProbes];
 #pragma unroll
@@ -983,7 +983,8 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   // three so that they are issued together, one memory latency in all:
   // tested on the count alone, the compiler would load the descriptor and the
   // token only after the count had arrived.
-  const int n_blocks = static_cast<int>(header[kHdrNumBlocks]);
+  // Only the four-tile expand runs on the plan's coarse table.
+  const int n_blocks = static_cast<int>(header[ROLE == kExpandOnly && TILES > 1 ? kHdrNumBlocks : kHdrNumFine]);
   // Roles that use the partial buffer do nothing while it is poisoned.
   const uint32_t poison = ROLE == kExpandOnly ? 0u : header[kHdrPoison];
   const Block blk = blocks[b];
@@ -1073,7 +1074,7 @@ void expand_ext_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   __shared__ alignas(16) T s_stage[kWaves * 16 * kStageStride];
   const int b = static_cast<int>(blockIdx.x) / per_block;
   const int part = static_cast<int>(blockIdx.x) - b * per_block;
-  const int n_blocks = static_cast<int>(header[kHdrNumBlocks]);
+  const int n_blocks = static_cast<int>(header[TILES > 1 ? kHdrNumBlocks : kHdrNumFine]);
   const Block blk = blocks[b];
   const int lane = threadIdx.x & 63;
   const int row = lane & 15;
@@ -1561,7 +1562,7 @@ void linear_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
   const int wg = static_cast<int>(blockIdx.x);
   // Blocks the grid has reducer slots for; a plan with more (only ids the
   // call cannot resolve make one) is reported, and the rest skipped.
-  const int n_plan = static_cast<int>(header[kHdrNumBlocks]);
+  const int n_plan = static_cast<int>(header[kHdrNumFine]);
   const int n_blocks = min(n_plan, a.n_slots);
   if (wg == 0 && tid == 0 && n_plan > a.n_slots) flag_error(a.plan.header, kErrCapacity);
   const uint32_t poison = header[kHdrPoison];

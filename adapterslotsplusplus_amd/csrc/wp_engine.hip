@@ -227,10 +227,15 @@ struct wp_engine {
   uint32_t* lin_flag = nullptr; // [2][block_cap] H flags and their reader counts (zero between calls)
   Entry* dtable = nullptr;      // [table_cap] id-indexed adapter table of build_seg_bounds plans
   Entry* bentries = nullptr;    // [block_cap] a build_seg_bounds plan's copy of each block's table entry
+  // The second table of build_seg_bounds plans over more than kSmallPlanTokens
+  // tokens: blocks of kFineTokens tokens (all [block_cap] slots).
+  Block* fblocks = nullptr;
+  int32_t* fbperm = nullptr;    // [block_cap][kBlockTokens]
+  Entry* fbentries = nullptr;
   bool plan_bentries = false;   // the last build_seg_bounds plan wrote bentries
   int table_cap = 0;
   int seg_cap = 0, block_cap = 0, tok_cap = 0, entry_cap = 0;
-  int ptok = 0;                 // plan positions of `part`: fused calls run on plans of <= kSmallPlanTokens
+  int ptok = 0;                 // plan positions `part` holds (fused_ptok: those a call spreads its d-ranges by)
   uint64_t part_words = 0, consumed_words = 0;
   int n_cu = 256;  // compute units of the device
   int32_t entry_offset = 0;  // table-mode calls on device-built plans read dtable + entry_offset
@@ -495,32 +500,95 @@ int evict_impl(wp_engine* e, int32_t id, hipStream_t stream) {
   return WP_OK;
 }
 
-PlanView plan_view(const wp_engine* e) {
+// fine: the 16-token table (the plan's own where its blocks are 16 tokens).
+PlanView plan_view(const wp_engine* e, bool fine = false) {
+  const bool second = fine && e->plan_bt > kFineTokens;
   PlanView v;
   v.header = e->header;
   v.segments = e->segs;
-  v.blocks = e->blocks;
+  v.blocks = second ? e->fblocks : e->blocks;
   v.perm = e->perm;
-  v.bperm = e->bperm;
+  v.bperm = second ? e->fbperm : e->bperm;
   return v;
 }
 
+// Whether the current plan has a table of 16-token blocks.
+bool has_fine(const wp_engine* e) { return e->plan_bt <= kFineTokens || e->plan_kind == 2; }
+
+// Plan positions per d-range of the partial buffer in this call: its chunks lie
+// as close as the plan allows (decode-sized plans keep theirs within 64 KB of
+// each other at rank 32).
+int fused_ptok(const wp_engine* e) {
+  return static_cast<int>(std::min<int64_t>(e->ptok, std::max<int64_t>(ceil_div(e->plan_T, kSmallPlanTokens), 1) * kSmallPlanTokens));
+}
+
+// Which of a plan's two tables a call runs on, past kSmallPlanTokens tokens
+// (below that there is only the 16-token one).  Short blocks spread a call
+// over more workgroups and hide its latency, long ones read an adapter's
+// weights once per 64 tokens: so the line lies at a number of tokens that falls
+// with the rank.  All figures MI355X, us per call, d = 4096 unless given, 16
+// contiguous prompts / Zipf(1.1) tokens over 64 adapters.
+
+// One fused launch on 16-token blocks, or shrink and expand launches.  Rank
+// times tokens up to 98304 (narrow outputs) or 61440 (over 32 output chunks,
+// where the expand's weights are the larger part):
+//   4096 columns, fused vs two launches: rank 8, 8192 tokens 42 / 47 vs 45 / 53;
+//   rank 16, 4096 26 / 29 vs 30 / 35; rank 32, 3072 27 / 31 vs 30 / 34, 4096
+//   33 / 39 vs 33 / 40; rank 64, 1536 25 / 30 vs 27 / 33, 2048 30 / 36 vs 30 / 34.
+//   3 x 4096 columns: rank 16, 2048 34 / 37 vs 38 / 44, 4096 57 / 63 vs 58 / 68;
+//   rank 64, 640 28 / 42 vs 32 / 48, 1024 37 / 50 vs 36 / 51.
+// With one A per slice the fused launch reads X per slice: ranks up to 32 and
+// 768 tokens (4096 + 2 x 1024 columns, rank 16, 640 tokens 18 / 22 vs 21 / 24,
+// 1024 22 / 29 vs 23 / 26; rank 32, 640 20 / 30 vs 24 / 35, 1024 30 / 37 vs 26 / 37;
+// rank 64, 640 33 / 47 vs 27 / 49).
+// Mixed ranks count as 48 or 60: 2048 tokens 29 / 31 vs 31 / 34 (3072 39 / 42 vs
+// 34 / 38), to 13824 columns 1024 33 / 42 vs 39 / 48 (1536 45 / 50 vs 43 / 53).
+bool fused_fits(const wp_engine* e, int rank, int n_a, int64_t n_ochunks) {
+  if (e->plan_bt <= kFineTokens) return true;
+  if (!has_fine(e)) return false;
+  if (n_a > 1) return rank != 0 && rank <= 32 && e->plan_T <= 768;
+  const bool wide = n_ochunks > 2 * kExpandWorkgroups;
+  const int64_t r = rank != 0 ? rank : wide ? 60 : 48;
+  return e->plan_T * r <= (wide ? 61440 : 98304);
+}
+
+// shrink() as many small workgroups and a reducer per 16-token block, or one
+// workgroup per 64-token block and d-range: up to 2048 tokens and rank times
+// tokens 65536 (mixed ranks as 32).  Small vs large, rank 16, 2048 tokens 11 /
+// 14 vs 13 / 15, 3072 14 / 16 vs 14 / 16; rank 64, 1024 14 / 18 vs 17 / 20, 2048
+// 19 / 22 vs 18 / 20; mixed, 2048 18 / 18 vs 19 / 20, 3072 21 / 23 vs 20 / 21.
+bool small_shrink_fits(const wp_engine* e, int rank) {
+  if (e->plan_bt <= kFineTokens) return true;
+  return has_fine(e) && e->plan_T <= 2048 && e->plan_T * (rank != 0 ? rank : 32) <= 65536;
+}
+
+// expand() over 16-token blocks, one tile in flight at eight waves per SIMD, or
+// 64-token blocks, four tiles at three to five.  Ranks up to 32 always: rank 16
+// 1024 tokens 9 / 9 vs 11 / 12, 8192 27 / 32 vs 38 / 38; rank 32, 8192 30 / 37
+// vs 39 / 40, to 13824 columns 95 / 116 vs 102 / 117.  Rank 64 reads twice the
+// weights per block: 640 tokens 9 / 13 vs 10 / 15, 1024 11 / 15 vs 11 / 16, 1536
+// 14 / 18 vs 12 / 17; mixed ranks 1024 10 / 12 vs 11 / 13, 2048 14 / 17 vs 13 / 16.
+bool fine_expand_fits(const wp_engine* e, int rank) {
+  if (e->plan_bt <= kFineTokens) return true;
+  return has_fine(e) && ((rank != 0 && rank <= 32) || e->plan_T <= (rank == 0 ? 1024 : 768));
+}
+
 // Fields every apply launch shares.
-ApplyArgs base_args(const wp_engine* e, int rank) {
+ApplyArgs base_args(const wp_engine* e, int rank, bool fine = false) {
   ApplyArgs a{};
   a.rank = rank;
   a.n_sub = 1;
-  a.tiles = (e->plan_bt + 15) / 16;
+  a.tiles = fine ? 1 : (e->plan_bt + 15) / 16;
   a.hs = rank == 0 ? kMaxRank : rank;
   a.hs1 = a.hs;
   a.w.n_a = 1;
-  a.ptok = e->ptok;
+  a.ptok = fused_ptok(e);
   a.part = e->part;
   a.consumed = e->consumed;
   a.spin_limit = e->spin_limit;
   a.trace = e->trace;
   a.trace_words = e->trace_words;
-  a.plan = plan_view(e);
+  a.plan = plan_view(e, fine);
   return a;
 }
 
@@ -533,11 +601,12 @@ ApplyArgs base_args(const wp_engine* e, int rank) {
 // Bounding by T alone would launch mostly empty workgroups on large plans
 // (8192 tokens: 8192 slots x 48 chunks for 144 real blocks, ~150 us of
 // dispatch), and a loop over items in the kernels costs their registers.
-int block_bound(const wp_engine* e, int64_t groups) {
+int block_bound(const wp_engine* e, int64_t groups, bool fine = false) {
   if (e->plan_kind == 1) return e->plan_blocks;
+  const int bt = fine ? kFineTokens : e->plan_bt;
   const int64_t T = e->plan_T;
   const int64_t g = std::min<int64_t>(T, std::max<int64_t>(groups, 1));
-  return static_cast<int>(std::min<int64_t>(T, T / e->plan_bt + g));
+  return static_cast<int>(std::min<int64_t>(T, T / bt + g));
 }
 
 // Distinct ids an adapter-store call on a device-built plan can resolve,
@@ -644,7 +713,7 @@ int wp_create(const wp_config* cfg_in, wp_engine** out) {
   e->block_cap = cfg.max_tokens + kRefMaxSegments;
   e->entry_cap = kRefMaxSegments;
   e->table_cap = cfg.max_adapter_ids;
-  e->ptok = std::min(cfg.max_tokens, kSmallPlanTokens);
+  e->ptok = cfg.max_tokens;
   e->part_words = static_cast<uint64_t>(kMaxChunks) * e->ptok * kMaxRank;
   e->consumed_words = static_cast<uint64_t>(e->block_cap) * kCounterStride;
   size_t off = 0;
@@ -665,6 +734,9 @@ int wp_create(const wp_config* cfg_in, wp_engine** out) {
   const size_t o_lin = carve(sizeof(uint32_t) * (kLinCounters + 2 * static_cast<size_t>(e->block_cap)));
   const size_t o_tab = carve(sizeof(Entry) * std::max(e->table_cap, 1));
   const size_t o_bent = carve(sizeof(Entry) * e->block_cap);
+  const size_t o_fblk = carve(sizeof(Block) * e->block_cap);
+  const size_t o_fbperm = carve(sizeof(int32_t) * static_cast<size_t>(e->block_cap) * kBlockTokens);
+  const size_t o_fbent = carve(sizeof(Entry) * e->block_cap);
   const size_t o_spart = carve(sizeof(float) * kMaxChunks * static_cast<size_t>(e->tok_cap) * kMaxRank);
   const size_t hbuf_bytes = sizeof(uint16_t) * static_cast<size_t>(e->tok_cap) * kMaxSlices * kMaxRank;
   const size_t o_hbuf = carve(hbuf_bytes);
@@ -684,6 +756,9 @@ int wp_create(const wp_config* cfg_in, wp_engine** out) {
   e->lin_flag = e->lin_cnt + kLinCounters;
   e->dtable = reinterpret_cast<Entry*>(e->ws + o_tab);
   e->bentries = reinterpret_cast<Entry*>(e->ws + o_bent);
+  e->fblocks = reinterpret_cast<Block*>(e->ws + o_fblk);
+  e->fbperm = reinterpret_cast<int32_t*>(e->ws + o_fbperm);
+  e->fbentries = reinterpret_cast<Entry*>(e->ws + o_fbent);
   e->spart = reinterpret_cast<float*>(e->ws + o_spart);
   e->hbuf = e->ws + o_hbuf;
   e->part = reinterpret_cast<float*>(e->ws + o_part);
@@ -1007,6 +1082,7 @@ int wp_build_segments(wp_engine* e, const int32_t* ids, int32_t K, const int32_t
   hdr[kHdrNumGroups] = static_cast<uint32_t>(entries.size());
   hdr[kHdrNumValid] = static_cast<uint32_t>(n_tok);
   hdr[kHdrT] = static_cast<uint32_t>(max_end);
+  hdr[kHdrNumFine] = hdr[kHdrNumBlocks];  // of use only where the blocks are kFineTokens tokens
 
   WP_HIP(hipMemcpyAsync(e->header, hdr, sizeof(uint32_t) * kHdrErrors, hipMemcpyHostToDevice, stream));
   if (K > 0) WP_HIP(hipMemcpyAsync(e->segs, hsegs, sizeof(Segment) * K, hipMemcpyHostToDevice, stream));
@@ -1049,8 +1125,9 @@ int wp_build_seg_bounds(wp_engine* e, const void* idx, int32_t idx_is_int64, int
   // Engines with registered adapters (table-mode calls) get each block's
   // table entry copied by the plan build; stacked-weight engines skip it.
   Entry* bent = e->adapters.empty() ? nullptr : e->bentries;
+  const FinePlan fine{e->fblocks, e->fbperm, bent ? e->fbentries : nullptr};
   WP_HIP(launch_plan(idx, idx_is_int64 ? 1 : 0, static_cast<int>(T), e->header, e->segs, e->blocks, e->perm,
-                     e->bperm, bent, e->seg_cap, e->block_cap, bt, &m, stream));
+                     e->bperm, bent, &fine, e->seg_cap, e->block_cap, bt, &m, stream));
   e->plan_bentries = bent != nullptr;
   // Slots whose copy had landed are in the table once this build has run
   // (event queries are not allowed while a graph is being captured).
@@ -1165,7 +1242,7 @@ int check_io(const char* who, int32_t dtype, const void* p16, const char* name) 
 }
 
 // Table-mode weights for the current plan.
-int table_weights(wp_engine* e, hipStream_t stream, Weights* w) {
+int table_weights(wp_engine* e, hipStream_t stream, Weights* w, bool fine = false) {
   w->mode = kTable;
   if (e->plan_kind == 1) {
     if (e->entry_offset != 0)
@@ -1185,7 +1262,8 @@ int table_weights(wp_engine* e, hipStream_t stream, Weights* w) {
   w->num_ids = std::max(0, e->table_cap - e->entry_offset);
   if (e->entry_count > 0) w->num_ids = std::min(w->num_ids, e->entry_count);
   // The plan's copies are of entries at offset 0 (a block's entry is its id).
-  w->a_base[0] = e->plan_bentries && e->entry_offset == 0 ? e->bentries : nullptr;
+  Entry* copies = fine && e->plan_bt > kFineTokens ? e->fbentries : e->bentries;
+  w->a_base[0] = e->plan_bentries && e->entry_offset == 0 ? copies : nullptr;
   return WP_OK;
 }
 
@@ -1318,16 +1396,17 @@ int wp_shrink(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t ran
   }
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  ApplyArgs a = base_args(e, rank);
+  const bool small = small_shrink_fits(e, rank);
+  ApplyArgs a = base_args(e, rank, small);
   a.x = X;
   a.ldx = d_model;
   a.h = H;
   a.ldh = h_row_stride;
   a.d_model = d_model;
-  if ((rc = table_weights(e, stream, &a.w)) != WP_OK) return rc;
+  if ((rc = table_weights(e, stream, &a.w, small)) != WP_OK) return rc;
   a.w.n_slices = 1;
-  a.n_slots = block_bound(e, resolvable_ids(e, stream));
-  if (e->plan_T <= kSmallPlanTokens) {
+  a.n_slots = block_bound(e, resolvable_ids(e, stream), small);
+  if (small) {
     // Decode-sized plans: many small shrink workgroups and a reducer per
     // block (the fused calls' shrink side), not one workgroup per block and
     // d-range streaming every rank row.
@@ -1376,12 +1455,13 @@ int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_
   }
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  ApplyArgs a = base_args(e, rank);
+  const bool small = fine_expand_fits(e, rank);
+  ApplyArgs a = base_args(e, rank, small);
   a.h = const_cast<void*>(H);
   a.ldh = h_row_stride;
   a.y = Y;
   a.ldy = y_row_stride;
-  if ((rc = table_weights(e, stream, &a.w)) != WP_OK) return rc;
+  if ((rc = table_weights(e, stream, &a.w, small)) != WP_OK) return rc;
   const int cols = expand_cols_per_workgroup();
   a.w.n_slices = 1;
   a.w.o_size[0] = out_features;
@@ -1389,7 +1469,7 @@ int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_
   a.w.oc_start[0] = 0;
   a.w.oc_start[1] = static_cast<int32_t>(ceil_div(out_features, cols));
   a.n_ochunks = a.w.oc_start[1];
-  a.n_slots = block_bound(e, resolvable_ids(e, stream));
+  a.n_slots = block_bound(e, resolvable_ids(e, stream), small);
   WP_HIP(launch_expand(dtype == WP_DTYPE_BF16, a, stream));
   return WP_OK;
 }
@@ -1415,17 +1495,17 @@ int add_lora_impl(wp_engine* e, const char* who, void* y, const void* x, int32_t
                 (long long)T);
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  a.tiles = (e->plan_bt + 15) / 16;
-  a.ptok = e->ptok;
+  const bool fused = fused_fits(e, rank, n_a, a.n_ochunks);
+  a.tiles = fused ? 1 : (e->plan_bt + 15) / 16;
+  a.ptok = fused_ptok(e);
   a.part = e->part;
   a.consumed = e->consumed;
   a.spin_limit = e->spin_limit;
   a.trace = e->trace;
   a.trace_words = e->trace_words;
-  a.plan = plan_view(e);
-  a.n_slots = block_bound(e, num_loras);
-  fused_split(&a, rank, d_model, e->n_cu);
-  if (e->plan_bt > 16) {
+  a.plan = plan_view(e, fused);
+  a.n_slots = block_bound(e, num_loras, fused);
+  if (!fused) {
     // Large plans (prefill-sized, 64-token blocks): shrink into the engine's
     // H (one launch per A slice, each into its columns of an H row), then
     // expand from it.  Each launch keeps several token tiles in flight per
@@ -1440,9 +1520,15 @@ int add_lora_impl(wp_engine* e, const char* who, void* y, const void* x, int32_t
     ApplyArgs as = a;
     as.ldy = rank;  // slice s at column s * rank of an H row
     WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, as, stream));
+    // H is by token, so the expand may run on the other table.
+    const bool fine = fine_expand_fits(e, rank);
+    a.tiles = fine ? 1 : a.tiles;
+    a.plan = plan_view(e, fine);
+    a.n_slots = block_bound(e, num_loras, fine);
     WP_HIP(launch_expand(dtype == WP_DTYPE_BF16, a, stream));
     return WP_OK;
   }
+  fused_split(&a, rank, d_model, e->n_cu);
   WP_HIP(launch_fused(dtype == WP_DTYPE_BF16, a, stream));
   return WP_OK;
 }
@@ -1488,7 +1574,7 @@ int wp_linear_lora(wp_engine* e, void* y, const void* x, const void* w, int64_t 
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   a.tiles = 1;
-  a.ptok = e->ptok;
+  a.ptok = fused_ptok(e);
   a.part = e->part;
   a.consumed = e->consumed;
   a.spin_limit = e->spin_limit;
@@ -1537,7 +1623,7 @@ int wp_add_lora_nslice(wp_engine* e, void* y, const void* x, int32_t n_slices, c
 int wp_shrink_expand(wp_engine* e, const void* X, void* Y, int32_t d_model, int32_t out_features, int32_t rank,
                      int64_t T, int64_t y_row_stride, int32_t y_col_offset, int32_t dtype, void* stream_) {
   if (!e) return fail(WP_ERR_INVALID, "shrink_expand: engine is NULL");
-  if (e->plan_kind == 0 || e->plan_T > kSmallPlanTokens) {
+  if (e->plan_kind == 0 || !fused_fits(e, rank, 1, ceil_div(out_features, expand_cols_per_workgroup()))) {
     // Large plans: shrink() into the engine's H, then expand() from it (the
     // same checks and errors as the two calls).
     const int64_t hs = rank == 0 ? kMaxRank : rank;
@@ -1568,13 +1654,13 @@ int wp_shrink_expand(wp_engine* e, const void* X, void* Y, int32_t d_model, int3
   }
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  ApplyArgs a = base_args(e, rank);
+  ApplyArgs a = base_args(e, rank, true);
   a.x = X;
   a.ldx = d_model;
   a.y = Y;
   a.ldy = y_row_stride;
   a.d_model = d_model;
-  if ((rc = table_weights(e, stream, &a.w)) != WP_OK) return rc;
+  if ((rc = table_weights(e, stream, &a.w, true)) != WP_OK) return rc;
   const int cols = expand_cols_per_workgroup();
   a.w.n_slices = 1;
   a.w.o_size[0] = out_features;
@@ -1582,7 +1668,7 @@ int wp_shrink_expand(wp_engine* e, const void* X, void* Y, int32_t d_model, int3
   a.w.oc_start[0] = 0;
   a.w.oc_start[1] = static_cast<int32_t>(ceil_div(out_features, cols));
   a.n_ochunks = a.w.oc_start[1];
-  a.n_slots = block_bound(e, resolvable_ids(e, stream));
+  a.n_slots = block_bound(e, resolvable_ids(e, stream), true);
   fused_split(&a, rank, d_model, e->n_cu);
   WP_HIP(launch_fused(dtype == WP_DTYPE_BF16, a, stream));
   return WP_OK;
@@ -1609,7 +1695,7 @@ int wp_shrink_expand_slices(wp_engine* e, const void* X, void* Y, int32_t d_mode
                                   "4-aligned)", s, y_col_offsets[s], y_col_offsets[s] + out_features[s],
                   (long long)y_row_stride);
   }
-  if (e->plan_T > kSmallPlanTokens || n_slices == 1) {
+  if (e->plan_bt > kFineTokens || n_slices == 1) {
     // Large plans (and a single slice): one shrink_expand per slice, each
     // on its layer's adapters.
     const int32_t off0 = e->entry_offset, cnt0 = e->entry_count;
@@ -1635,7 +1721,7 @@ int wp_shrink_expand_slices(wp_engine* e, const void* X, void* Y, int32_t d_mode
                 (long long)e->plan_T, (long long)T);
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  ApplyArgs a = base_args(e, rank);
+  ApplyArgs a = base_args(e, rank, true);
   a.x = X;
   a.ldx = d_model;
   a.y = Y;
@@ -1667,7 +1753,7 @@ int wp_shrink_expand_slices(wp_engine* e, const void* X, void* Y, int32_t d_mode
   // Blocks: bounded as for one layer's window (an id registered in any
   // slice's layer forms a block).
   const int64_t window = ids_per_layer > 0 ? ids_per_layer : static_cast<int64_t>(e->table_cap);
-  a.n_slots = block_bound(e, call_ids(e, stream, static_cast<int64_t>(e->adapters.size()), window));
+  a.n_slots = block_bound(e, call_ids(e, stream, static_cast<int64_t>(e->adapters.size()), window), true);
   fused_split(&a, rank, d_model, e->n_cu);
   WP_HIP(launch_fused(dtype == WP_DTYPE_BF16, a, stream));
   return WP_OK;
@@ -1683,13 +1769,13 @@ int wp_shrink_expand_slices(wp_engine* e, const void* X, void* Y, int32_t d_mode
 namespace {
 
 // Launch fields of a stacked-weight call that every V1 op shares.
-ApplyArgs stacked_base(const wp_engine* e, int32_t rank, int32_t num_loras, float scale) {
-  ApplyArgs a = base_args(e, rank);
+ApplyArgs stacked_base(const wp_engine* e, int32_t rank, int32_t num_loras, float scale, bool fine = false) {
+  ApplyArgs a = base_args(e, rank, fine);
   a.w.mode = kStacked;
   a.w.num_ids = num_loras;
   a.w.scale = scale;
   a.w.n_slices = 1;
-  a.n_slots = block_bound(e, num_loras);
+  a.n_slots = block_bound(e, num_loras, fine);
   return a;
 }
 
@@ -1727,7 +1813,8 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
   if ((rc = check_plan_for(e, who, T)) != WP_OK) return rc;
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  ApplyArgs a = stacked_base(e, rank, num_loras, scale);
+  const bool small = e->plan_bt <= kFineTokens;
+  ApplyArgs a = stacked_base(e, rank, num_loras, scale, small);
   a.x = x;
   a.ldx = d_model;
   a.d_model = d_model;
@@ -1742,7 +1829,7 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
   a.ldh = out_row_stride;
   a.ldy = out_slice_stride;
   a.h_f32 = 1;
-  if (e->plan_bt <= 16) {
+  if (small) {
     for (int s = 0; s < n_slices; ++s) {
       ApplyArgs as = a;
       as.w.n_a = 1;
@@ -1825,7 +1912,7 @@ int wp_lora_expand(wp_engine* e, void* y, int64_t y_row_stride, const void* h, i
   ExpandExt x{};
   ApplyArgs a{};
   {
-    a = stacked_base(e, rank, num_loras, 1.0f);
+    a = stacked_base(e, rank, num_loras, 1.0f, fine_expand_fits(e, rank));
     a.y = y;
     a.ldy = y_row_stride;
     a.w.n_a = n_slices;  // slice s reads its own H
@@ -1874,7 +1961,7 @@ int wp_lora_expand(wp_engine* e, void* y, int64_t y_row_stride, const void* h, i
   } else {
     PrepArgs p{};
     p.plan = plan_view(e);
-    p.n_slots = a.n_slots;
+    p.n_slots = block_bound(e, num_loras);
     p.n_slices = n_slices;
     p.num_ids = num_loras;
     p.rank = rank;
@@ -2035,7 +2122,7 @@ int wp_add_lora_static(void* y, const void* x, const void* idx, int32_t idx_is_i
   m.consumed_words = (kSOffPart - kSOffCons) / 4;
   WP_HIP(launch_plan(idx, idx_is_int64 ? 1 : 0, static_cast<int>(T), v.header, reinterpret_cast<Segment*>(base + kSOffSeg),
                      reinterpret_cast<Block*>(base + kSOffBlk), reinterpret_cast<int32_t*>(base + kSOffPerm),
-                     reinterpret_cast<int32_t*>(base + kSOffBperm), nullptr, kStaticSegCap, kStaticBlockCap, bt, &m,
+                     reinterpret_cast<int32_t*>(base + kSOffBperm), nullptr, nullptr, kStaticSegCap, kStaticBlockCap, bt, &m,
                      stream));
   a.tiles = 1;
   a.ptok = kStaticTokens;

@@ -191,10 +191,11 @@ struct PlanKernelArgs {
   int32_t* perm;
   int32_t* bperm;
   Entry* bentries;
+  FinePlan fine;
   int seg_cap, block_cap, bt;
   Maint m;
 };
-static_assert(offsetof(PlanKernelArgs, m) == 80 && sizeof(PlanKernelArgs) == 80 + sizeof(Maint),
+static_assert(offsetof(PlanKernelArgs, m) == 104 && sizeof(PlanKernelArgs) == 104 + sizeof(Maint),
               "plan_kernel's argument size as passed to touch_kernel_args");
 
 // ------------------------------------------------------------- plan build ----
@@ -299,10 +300,12 @@ struct Digits {
   uint32_t pre[4];  // ... in the waves before this one
   uint32_t off[4];  // items of all digits below
   uint32_t blk[4];  // blocks of all digits below
-  uint32_t n_items, n_blocks, n_digits;
+  uint32_t fblk[4]; // kFineTokens-token blocks of all digits below (fine only)
+  uint32_t n_items, n_blocks, n_fine, n_digits;
 };
 template <int NW>
-__device__ __forceinline__ Digits scan_digits(const uint32_t (*s_cnt)[kDigits], int wave, int max_digit, int bt_log2) {
+__device__ __forceinline__ Digits scan_digits(const uint32_t (*s_cnt)[kDigits], int wave, int max_digit, int bt_log2,
+                                              bool fine) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63;
   Digits r;
@@ -344,15 +347,48 @@ __device__ __forceinline__ Digits scan_digits(const uint32_t (*s_cnt)[kDigits], 
     r.off[j] = ex & 0xffffu;
     r.blk[j] = ex >> 16;
     ex += own[j];
+    r.fblk[j] = 0;
+  }
+  r.n_fine = r.n_blocks;
+  if (fine) {
+    sum = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      own[j] = (r.tot[j] + kFineTokens - 1) / kFineTokens;
+      sum += own[j];
+    }
+    inc = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = __shfl_up(inc, off, 64);
+      if (lane >= off) inc += y;
+    }
+    r.n_fine = __shfl(inc, 63, 64);
+    ex = inc - sum;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      r.fblk[j] = ex;
+      ex += own[j];
+    }
   }
   return r;
 }
 
-// One block of the plan and (bentries != null) its adapter-table entry as of
-// this build (agent-scope loads: the maintenance may have installed it from
-// another wave), or an empty one.
-__device__ __forceinline__ void put_block(Block* blocks, Entry* bentries, const Maint& m, int q, int32_t id, int first,
-                                          int count) {
+// An adapter's table entry as of this build (agent-scope loads: the maintenance
+// may have installed it from another wave), or an empty one.
+struct EntryWords {
+  uint64_t w[4];
+};
+__device__ __forceinline__ EntryWords read_entry(const Maint& m, int32_t id, bool wanted) {
+  EntryWords en{{0, 0, 0, 0}};
+  if (wanted && m.table != nullptr && id >= 0 && id < m.table_cap) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) en.w[i] = agent_load64(reinterpret_cast<const uint64_t*>(m.table + id) + i);
+  }
+  return en;
+}
+__device__ __forceinline__ void put_block(Block* blocks, Entry* bentries, int q, int32_t id, int first, int count,
+                                          const EntryWords& en) {
   Block b;
   b.adapter_id = id;
   b.first = first;
@@ -360,14 +396,9 @@ __device__ __forceinline__ void put_block(Block* blocks, Entry* bentries, const 
   b.entry = id;
   blocks[q] = b;
   if (bentries != nullptr) {
-    uint64_t w[4] = {0, 0, 0, 0};
-    if (m.table != nullptr && id >= 0 && id < m.table_cap) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = agent_load64(reinterpret_cast<const uint64_t*>(m.table + id) + i);
-    }
     uint64_t* dst = reinterpret_cast<uint64_t*>(bentries + q);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dst[i] = w[i];
+    for (int i = 0; i < 4; ++i) dst[i] = en.w[i];
   }
 }
 
@@ -382,7 +413,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
                                                   uint32_t* __restrict__ header, Segment* __restrict__ segments,
                                                   Block* __restrict__ blocks, int32_t* __restrict__ perm,
                                                   int32_t* __restrict__ bperm, Entry* __restrict__ bentries,
-                                                  int seg_cap, int block_cap, int bt, Maint m) {
+                                                  FinePlan fine, int seg_cap, int block_cap, int bt, Maint m) {
   touch_kernel_args<static_cast<int>(sizeof(PlanKernelArgs))>();
   constexpr int CAP = NT * E;
   constexpr int NW = NT / 64;
@@ -390,8 +421,10 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
   static_assert(NW % 4 == 0 && CAP <= 65536 / 2, "digit columns per wave; 16-bit token positions");
   __shared__ uint64_t s_start[NWORDS];  // run starts, one bit per item
   __shared__ uint64_t s_piece[NWORDS];  // piece starts
+  __shared__ uint64_t s_fpiece[NWORDS]; // ... of the fine table (ids of 256 and more)
   __shared__ alignas(16) uint32_t s_cnt[NW][kDigits];
-  // Each wave's own digit bases: {items below | items of earlier waves << 16, blocks below}.
+  // Each wave's own digit bases: {items below | items of earlier waves << 16,
+  // blocks below | fine blocks below << 16}.
   __shared__ uint2 s_base[NW][kDigits];
   __shared__ uint32_t s_wmax[NW];
   __shared__ uint32_t s_wflag[NW];
@@ -539,15 +572,18 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
   plan_stamp(m, 4);
 
   // 5. Tokens grouped by adapter, token order kept inside an adapter.
-  int n_tok, n_groups, n_blocks;
+  const bool has_fine = fine.blocks != nullptr;
+  const bool want_entry = bentries != nullptr;
+  int n_tok, n_groups, n_blocks, n_fine;
   if (small_ids) {
-    const Digits g = scan_digits<NW>(s_cnt, wave, max_digit, bt_log2);
+    const Digits g = scan_digits<NW>(s_cnt, wave, max_digit, bt_log2, has_fine);
     n_tok = static_cast<int>(g.n_items);
     n_groups = static_cast<int>(g.n_digits);
     n_blocks = static_cast<int>(g.n_blocks);
+    n_fine = static_cast<int>(g.n_fine);
     if (4 * lane <= max_digit) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s_base[wave][4 * lane + j] = uint2{g.off[j] | (g.pre[j] << 16), g.blk[j]};
+      for (int j = 0; j < 4; ++j) s_base[wave][4 * lane + j] = uint2{g.off[j] | (g.pre[j] << 16), g.blk[j] | (g.fblk[j] << 16)};
     }
     plan_stamp(m, 5);
 #pragma unroll
@@ -557,21 +593,56 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
       const uint2 bs = s_base[wave][dig[e]];
       const int pos = static_cast<int>((bs.x >> 16) + rank[e]);  // inside the adapter's group
       perm[static_cast<int>(bs.x & 0xffffu) + pos] = i;
-      const int q = static_cast<int>(bs.y) + (pos >> bt_log2);
+      const int q = static_cast<int>(bs.y & 0xffffu) + (pos >> bt_log2);
       if (q < block_cap) bperm[static_cast<int64_t>(q) * kBlockTokens + (pos & (bt - 1))] = i;
+      if (has_fine) {
+        const int f = static_cast<int>(bs.y >> 16) + pos / kFineTokens;
+        if (f < block_cap) fine.bperm[static_cast<int64_t>(f) * kBlockTokens + pos % kFineTokens] = i;
+      }
     }
     plan_stamp(m, 6);
-    // Block table: wave w writes the blocks w / 4, w / 4 + NW / 4, ... of
-    // the digits 4 * lane + w % 4.
-    const int j = wave & 3;
-    const auto pick = [&](const uint32_t(&v)[4]) {
-      return static_cast<int>(j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3]);
-    };
-    const int tot = pick(g.tot), off = pick(g.off), blk0 = pick(g.blk);
-    const int nb = (tot + bt - 1) >> bt_log2;
-    for (int k = wave >> 2; k < nb; k += NW / 4)
-      if (blk0 + k < block_cap)
-        put_block(blocks, bentries, m, blk0 + k, 4 * lane + j, off + k * bt, min(bt, tot - k * bt));
+    if constexpr (E == 1) {
+      // Block tables: wave w writes the blocks w / 4, w / 4 + NW / 4, ... of
+      // the digits 4 * lane + w % 4.
+      const int j = wave & 3;
+      const auto pick = [&](const uint32_t(&v)[4]) {
+        return static_cast<int>(j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3]);
+      };
+      const int id = 4 * lane + j;
+      const int tot = pick(g.tot), off = pick(g.off), blk0 = pick(g.blk), fblk0 = pick(g.fblk);
+      const EntryWords en = read_entry(m, id, want_entry && tot > 0);
+      for (int k = wave >> 2; k << bt_log2 < tot; k += NW / 4)
+        if (blk0 + k < block_cap) put_block(blocks, bentries, blk0 + k, id, off + k * bt, min(bt, tot - k * bt), en);
+      if (has_fine) {
+        for (int k = wave >> 2; k * kFineTokens < tot; k += NW / 4)
+          if (fblk0 + k < block_cap)
+            put_block(fine.blocks, fine.bentries, fblk0 + k, id, off + k * kFineTokens,
+                      min(kFineTokens, tot - k * kFineTokens), en);
+      }
+    } else {
+      // Larger plans: a thread per block finds its digit in the wave's bases
+      // (one adapter may own every block).
+      const auto table = [&](Block* out, Entry* oent, int n, int size_log2, int half) {
+        for (int q = tid; q < min(n, block_cap); q += NT) {
+          int lo = 0, hi = max_digit;
+          while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (static_cast<int>((s_base[wave][mid].y >> half) & 0xffffu) <= q) {
+              lo = mid;
+            } else {
+              hi = mid - 1;
+            }
+          }
+          const uint2 bs = s_base[wave][lo];
+          const int k = q - static_cast<int>((bs.y >> half) & 0xffffu);
+          const int at = static_cast<int>(bs.x & 0xffffu) + (k << size_log2);
+          const int end = lo < max_digit ? static_cast<int>(s_base[wave][lo + 1].x & 0xffffu) : n_tok;
+          put_block(out, oent, q, lo, at, min(1 << size_log2, end - at), read_entry(m, lo, want_entry));
+        }
+      };
+      table(blocks, bentries, n_blocks, bt_log2, 0);
+      if (has_fine) table(fine.blocks, fine.bentries, n_fine, 4, 16);
+    }
   } else {
     // Larger ids: the counting pass again over the next 8 bits of the order
     // so far, then the groups' blocks from the sorted order the way the
@@ -586,7 +657,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
       tok[e] = static_cast<uint32_t>((first + e) * 64 + lane);
     }
     for (int shift = 0;; shift += 8) {
-      const Digits g = scan_digits<NW>(s_cnt, wave, kDigits - 1, bt_log2);
+      const Digits g = scan_digits<NW>(s_cnt, wave, kDigits - 1, bt_log2, false);
       n_tok = static_cast<int>(g.n_items);
 #pragma unroll
       for (int j = 0; j < 4; ++j) s_base[wave][4 * lane + j].x = g.off[j] + g.pre[j];
@@ -623,34 +694,51 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
     lds_barrier();
     n_groups = static_cast<int>(count_words<NWORDS>(s_start, first) >> 16);
     mark_pieces<E>(start, lv, first, last_start_before<NWORDS>(s_start, first), bt, piece, rs);
-#pragma unroll
-    for (int e = 0; e < E; ++e)
-      if (lane == 0) s_piece[first + e] = piece[e];
-    lds_barrier();
-    const uint32_t nblk = count_words<NWORDS>(s_piece, first);
-    n_blocks = static_cast<int>(nblk >> 16);
-    int blk0 = static_cast<int>(nblk & 0xffffu);
+    uint64_t fpiece[E];
+    if (has_fine) {
+      int unused[E];
+      mark_pieces<E>(start, lv, first, last_start_before<NWORDS>(s_start, first), kFineTokens, fpiece, unused);
+    }
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const int w = first + e;
-      const int q = w * 64 + lane;
-      const uint64_t le = (lanes_below(lane) << 1) | 1ull;
-      const int b = blk0 + __popcll(piece[e] & le) - 1;  // this position's block
-      blk0 += __popcll(piece[e]);
-      if (q >= n_tok) continue;
-      perm[q] = static_cast<int>(tok[e]);
-      if (b >= block_cap) continue;
-      bperm[static_cast<int64_t>(b) * kBlockTokens + ((q - rs[e]) & (bt - 1))] = static_cast<int>(tok[e]);
-      if (!((piece[e] >> lane) & 1ull)) continue;
-      const uint64_t up = ((start[e] | piece[e]) >> lane) >> 1;
-      int end = n_tok;
-      if (up != 0) {
-        end = q + 1 + __builtin_ctzll(up);
-      } else if (w + 1 < NWORDS) {
-        const uint64_t nx = s_start[w + 1] | s_piece[w + 1];
-        if (nx != 0) end = (w + 1) * 64 + __builtin_ctzll(nx);
+      if (lane != 0) continue;
+      s_piece[first + e] = piece[e];
+      if (has_fine) s_fpiece[first + e] = fpiece[e];
+    }
+    lds_barrier();
+    const auto table = [&](const uint64_t(&pc)[E], const uint64_t* s_pc, int size, Block* out, int32_t* operm,
+                           Entry* oent) {
+      const uint32_t nblk = count_words<NWORDS>(s_pc, first);
+      int blk0 = static_cast<int>(nblk & 0xffffu);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int w = first + e;
+        const int q = w * 64 + lane;
+        const uint64_t le = (lanes_below(lane) << 1) | 1ull;
+        const int b = blk0 + __popcll(pc[e] & le) - 1;  // this position's block
+        blk0 += __popcll(pc[e]);
+        if (q >= n_tok || b >= block_cap) continue;
+        operm[static_cast<int64_t>(b) * kBlockTokens + ((q - rs[e]) & (size - 1))] = static_cast<int>(tok[e]);
+        if (!((pc[e] >> lane) & 1ull)) continue;
+        const uint64_t up = ((start[e] | pc[e]) >> lane) >> 1;
+        int end = n_tok;
+        if (up != 0) {
+          end = q + 1 + __builtin_ctzll(up);
+        } else if (w + 1 < NWORDS) {
+          const uint64_t nx = s_start[w + 1] | s_pc[w + 1];
+          if (nx != 0) end = (w + 1) * 64 + __builtin_ctzll(nx);
+        }
+        const int id = static_cast<int>(dig[e]);
+        put_block(out, oent, b, id, q, end - q, read_entry(m, id, want_entry));
       }
-      put_block(blocks, bentries, m, b, static_cast<int>(dig[e]), q, end - q);
+      return static_cast<int>(nblk >> 16);
+    };
+    n_blocks = table(piece, s_piece, bt, blocks, bperm, bentries);
+    n_fine = has_fine ? table(fpiece, s_fpiece, kFineTokens, fine.blocks, fine.bperm, fine.bentries) : n_blocks;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int q = (first + e) * 64 + lane;
+      if (q < n_tok) perm[q] = static_cast<int>(tok[e]);
     }
     plan_stamp(m, 6);
   }
@@ -658,6 +746,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
   if (tid == 0) {
     header[kHdrNumSegments] = static_cast<uint32_t>(n_segs);
     header[kHdrNumBlocks] = static_cast<uint32_t>(min(n_blocks, block_cap));
+    header[kHdrNumFine] = static_cast<uint32_t>(min(n_fine, block_cap));
     header[kHdrNumGroups] = static_cast<uint32_t>(n_groups);
     header[kHdrNumValid] = static_cast<uint32_t>(n_tok);
     header[kHdrT] = static_cast<uint32_t>(T);
@@ -671,18 +760,23 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
 
 // Host launcher: the smallest capacity variant that holds T.
 hipError_t launch_plan(const void* idx, int idx_is_int64, int T, uint32_t* header, Segment* segments, Block* blocks,
-                       int32_t* perm, int32_t* bperm, Entry* bentries, int seg_cap, int block_cap, int bt,
-                       const Maint* m, hipStream_t stream) {
+                       int32_t* perm, int32_t* bperm, Entry* bentries, const FinePlan* fine, int seg_cap, int block_cap,
+                       int bt, const Maint* m, hipStream_t stream) {
   if (T < 0 || bt < 1 || bt > kBlockTokens || (bt & (bt - 1)) != 0) return hipErrorInvalidValue;
   Maint mm{};
   if (m != nullptr) mm = *m;
+  FinePlan ff{};
+  if (fine != nullptr && bt > kFineTokens) ff = *fine;
+  // Both tables carry entries, or neither.
+  if (ff.blocks != nullptr && (ff.bperm == nullptr || (ff.bentries == nullptr) != (bentries == nullptr)))
+    return hipErrorInvalidValue;
   // Publications are applied by threads 0..n_pubs-1 of the smallest variant.
   if (mm.n_pubs < 0 || mm.n_pubs > 256) return hipErrorInvalidValue;
   // The smallest capacity that holds T: a wave's words are consecutive, so a
   // larger one would leave waves idle while others work their words in turn.
   auto run = [&](auto nt, auto e) {
     plan_kernel<decltype(nt)::value, decltype(e)::value><<<1, decltype(nt)::value, 0, stream>>>(
-        idx, idx_is_int64, T, header, segments, blocks, perm, bperm, bentries, seg_cap, block_cap, bt, mm);
+        idx, idx_is_int64, T, header, segments, blocks, perm, bperm, bentries, ff, seg_cap, block_cap, bt, mm);
   };
   if (T <= 256) {
     run(std::integral_constant<int, 256>{}, std::integral_constant<int, 1>{});

@@ -30,12 +30,15 @@ constexpr int kRefMaxSegments = 256;
 // Most tokens per work block, and the slot stride of bperm: one adapter's
 // weights are streamed once per block.
 constexpr int kBlockTokens = 64;
-// Plans over at most this many tokens (decode-sized steps) cut blocks at 16
-// tokens instead, one MFMA token tile: more, shorter blocks spread a hot
+// Blocks of 16 tokens, one MFMA token tile: more, shorter blocks spread a hot
 // adapter over more workgroups, and its repeated weight reads are served by
-// the caches while the blocks run side by side.
+// the caches while the blocks run side by side.  Plans over at most
+// kSmallPlanTokens tokens (decode-sized steps) have only these; larger
+// device-built plans have both, and each call takes the table that suits its
+// ranks and sizes (wp_engine.hip fused_pays).
+constexpr int kFineTokens = 16;
 constexpr int kSmallPlanTokens = 512;
-inline constexpr int plan_block_tokens(int64_t T) { return T <= kSmallPlanTokens ? 16 : kBlockTokens; }
+inline constexpr int plan_block_tokens(int64_t T) { return T <= kSmallPlanTokens ? kFineTokens : kBlockTokens; }
 // Word pattern of an empty fp32 partial: a quiet NaN whose payload has bits
 // set below bit 13.  Partials are fp32 sums of products of bf16/fp16 values;
 // a NaN among them is the canonical quiet NaN or carries a payload widened
@@ -74,22 +77,25 @@ enum HeaderWord : int {
   kHdrNumGroups = 2,
   kHdrNumValid = 3,
   kHdrT = 4,
-  kHdrErrors = 5,
-  kHdrBlockTokens = 6,
+  // Blocks of the fine (16-token) table: the plan's own blocks where they are
+  // 16 tokens, else the second table of a device-built plan.
+  kHdrNumFine = 5,
+  kHdrErrors = 6,
+  kHdrBlockTokens = 7,
   // Non-zero once a wait on partials gave up (kErrSpin): the partial buffer may
   // hold words a late shrink workgroup wrote after its block's readers
   // emptied it.  Kernels that use the buffer skip their work while it is set;
   // the next plan build (or wp_read_device_errors) refills the buffer with
   // kPartialEmpty, clears the counters and resets the word.
-  kHdrPoison = 7,
+  kHdrPoison = 8,
   // Raised by every write into the id-indexed adapter table (the entry-write
   // kernel, a plan build's installed publications).
-  kHdrTableVer = 8,
+  kHdrTableVer = 9,
   // The table version a plan build copied its blocks' entries at (see
   // Weights::a_base); the copies hold while the two words are equal.  A
   // build without copies stores the complement of the current version, so
   // copies an earlier build left behind never count as current.
-  kHdrPlanVer = 9,
+  kHdrPlanVer = 10,
   kHdrWords = 16
 };
 

@@ -330,9 +330,9 @@ class WarpPipeEngine:
     def shrink_expand(self, X, Y, out_features, rank, y_offset: int = 0, layer=None):
         """shrink() then expand() as one call (not in the reference):
         Y[:, y_offset:y_offset+o] += rn(alpha * X . A^T) . B^T per segment, in
-        place.  Decode-sized plans run in one launch with no H round trip
-        (rank=0: mixed ranks); larger plans run the two halves through the
-        engine's own H."""
+        place.  Plans of up to about 98304 / rank tokens run in one launch with
+        no H round trip (rank=0: mixed ranks); larger ones run the two halves
+        through the engine's own H."""
         rank = int(rank or 0)
         self._on_device(X, "X")
         self._on_device(Y, "Y")

@@ -71,7 +71,8 @@ int wp_abi_version(void);
 int wp_rank_supported(int32_t rank);
 
 /* Most tokens per work block in a plan over T tokens (16 for T <= 512, else
- * 64), as wp_read_plan reports the blocks.  No reference counterpart: the
+ * 64), as wp_read_plan reports the blocks (larger build_seg_bounds plans hold a
+ * second table of 16-token blocks for the calls that run better on it).  No reference counterpart: the
  * by-adapter blocking is this library's own. */
 int wp_block_tokens(int64_t T);
 
@@ -197,9 +198,10 @@ int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_
 
 /* shrink() followed by expand() over the adapter store, as one call: no
  * counterpart in the reference (its callers run the two after each other,
- * bindings:132-148).  Decode-sized plans (at most 512 tokens) run both halves
+ * bindings:132-148).  Plans of up to 512 tokens, and larger build_seg_bounds
+ * plans as far as the rank allows (about 98304 / rank tokens), run both halves
  * in one launch with no H round trip (rank = 0: mixed ranks, each adapter's
- * own); larger plans run shrink then expand through the engine's own H.  Results
+ * own); others run shrink then expand through the engine's own H.  Results
  * match the two calls within the fp tolerance (the d-range split, and so the
  * fp32 summation order of H, can differ). */
 int wp_shrink_expand(wp_engine* e, const void* X, void* Y, int32_t d_model, int32_t out_features, int32_t rank,

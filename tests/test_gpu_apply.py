@@ -769,3 +769,101 @@ def test_shrink_expand_shape_errors():
     assert engine.device_errors() & 4
     with pytest.raises(RuntimeError, match="2-D"):
         engine.shrink_expand(X.view(2, 16, 256), Y, 256, 16)
+
+
+# Both sides of each line between a plan's two block tables past 512 tokens:
+# (rank, T, output widths, one A per slice, adapter ids).
+TABLE_LINES = [
+    (64, 1536, [260], False, "low"), (64, 1537, [260], False, "low"),     # fused / two launches, narrow
+    (16, 6144, [132], False, "high"), (16, 6145, [132], False, "high"),
+    (8, 8192, [516], False, "one"),
+    (64, 960, [8452], False, "low"), (64, 961, [8452], False, "one"),     # ... over 32 output chunks
+    (32, 768, [260, 64], True, "low"), (32, 769, [260, 64], True, "high"),  # one A per slice
+    (64, 513, [260, 64], True, "one"),
+]
+
+
+@pytest.mark.parametrize("case", TABLE_LINES, ids=lambda c: f"r{c[0]}-T{c[1]}-{len(c[2])}x{c[2][0]}-{c[4]}")
+def test_add_lora_on_both_tables(case):
+    """Calls on plans of more than 512 tokens, next to the lines where they move
+    between the 16-token and the 64-token block table: a hot adapter beside
+    single tokens ("low" ids), ids of two counting passes ("high"), one
+    adapter for every token, and tokens without one.  Tolerance: the
+    repository's, plus one H rounding step times |B| at exact ties."""
+    rank, T, outs, per_slice, kind = case
+    dtype = DTYPES[T % 2]
+    d, L = 264, 300 if kind == "high" else 12
+    announce(f"both tables r={rank} T={T} outs={outs} per_slice={per_slice} ids={kind} {dtype}")
+    rng = np.random.default_rng(T + rank)
+    if kind == "one":
+        idx = np.full(T, 5)
+    else:
+        idx = np.where(rng.random(T) < 0.4, L - 2, rng.integers(-1, L, size=T))
+    x, y0 = randn((T, d), 900, dtype), randn((T, sum(outs)), 901, dtype)
+    n_a = len(outs) if per_slice else 1
+    was = [randn((L, 1, rank, d), 902 + i, dtype, 0.05) for i in range(n_a)]
+    wbs = [randn((L, 1, o, rank), 906 + i, dtype, 0.02) for i, o in enumerate(outs)]
+    offs = [sum(outs[:i]) for i in range(len(outs))]
+    engine = WarpPipeEngine()
+    assert engine.build_seg_bounds(torch.from_numpy(idx.astype(np.int64)).cuda())
+    y = y0.cuda()
+    dwa = [w.cuda() for w in was]
+    assert engine.add_lora_slices(y, x.cuda(), dwa if per_slice else dwa[0], [w.cuda() for w in wbs], 0.5, offs)
+    torch.cuda.synchronize()
+    segs = so.seg_bounds(idx).tolist()
+    ref = y0
+    slack = torch.zeros(y0.shape, dtype=torch.float32)
+    for i, (wb, off) in enumerate(zip(wbs, offs)):
+        wa = was[i if per_slice else 0]
+        ref = bgmv.add_lora(ref, x, wa, [wb], 0.5, segs, [off])
+        for a in np.unique(idx[idx >= 0]):
+            rows = torch.from_numpy(np.nonzero(idx == a)[0])
+            flips = h_tie_flips(x[rows], wa[a, 0], 0.5, dtype)
+            slack[rows, off:off + outs[i]] += (flips @ wb[a, 0].double().abs().T).float()
+    assert_close(y, ref, "both tables", slack=slack)
+    assert engine.device_errors() == 0
+
+
+@pytest.mark.parametrize("T", [768, 769, 1024, 1025, 2048, 2049])
+@pytest.mark.parametrize("rank", [0, 64])
+def test_store_on_both_tables(T, rank):
+    """shrink(), expand() and shrink_expand() next to the lines between the two
+    block tables, at mixed ranks and rank 64: both tables' copies of the adapter
+    entries, before and after an adapter is replaced without a new plan."""
+    dtype, d, o, K = DTYPES[T % 2], 264, 132, 9
+    announce(f"store on both tables T={T} rank={rank} {dtype}")
+    engine = WarpPipeEngine()
+    ranks = [rank or (8, 16, 32, 64)[i % 4] for i in range(K)]
+    adapters = {}
+
+    def put(i, seed):
+        A, B = randn((ranks[i], d), seed, dtype, 0.05), randn((o, ranks[i]), seed + 1, dtype, 0.02)
+        engine.register_adapter(i, A.cuda(), B.cuda(), 0.5, rank=ranks[i])
+        adapters[i] = (A, B, 0.5)
+
+    for i in range(K):
+        put(i, 1000 + 2 * i)
+    rng = np.random.default_rng(T)
+    idx = np.where(rng.random(T) < 0.4, 3, rng.integers(-1, K, size=T))
+    assert engine.build_seg_bounds(torch.from_numpy(idx.astype(np.int64)).cuda())
+    segs = so.seg_bounds(idx).tolist()
+    X, Y0 = randn((T, d), 1100, dtype), randn((T, o), 1101, dtype)
+    for step in range(2):
+        if step == 1:
+            engine.evict_adapter(3)
+            put(3, 1200)
+        H = engine.shrink(X.cuda(), d, rank, T)
+        Y, Y1 = Y0.cuda(), Y0.cuda()
+        engine.expand(H, Y, o, rank)
+        engine.shrink_expand(X.cuda(), Y1, o, rank)
+        torch.cuda.synchronize()
+        H_ref = bgmv.shrink(X, segs, adapters, rank if rank else 64, T)
+        Y_ref = bgmv.expand(H_ref, Y0, segs, adapters)
+        slack = torch.zeros(Y0.shape, dtype=torch.float32)
+        for aid, (A, B, alpha) in adapters.items():
+            rows = torch.from_numpy(np.nonzero(idx == aid)[0])
+            slack[rows] += (h_tie_flips(X[rows], A, alpha, dtype) @ B.double().abs().T).float()
+        assert_close(H, H_ref, f"H step {step}")
+        assert_close(Y, Y_ref, f"Y step {step}", slack=slack)
+        assert_close(Y1, Y_ref, f"shrink_expand step {step}", slack=slack)
+        assert engine.device_errors() == 0
