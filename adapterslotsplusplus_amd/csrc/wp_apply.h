@@ -167,7 +167,8 @@ hipError_t launch_fused(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
 // H[token], slice s at element s * a.ldy of an H row.
 hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
 // shrink() of decode-sized plans: the fused kernel's shrink workgroups
-// (kShrinkRowsFused rows x d-range) and one reducer per block writing H;
+// (kShrinkRowsFused rows x d-range) of every A slice and one reducer per block
+// and slice writing its H at element s * a.ldy of a row;
 // a.part is the fused calls' partial buffer (kPartialEmpty between calls).
 hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
 // expand(): expand from a caller-provided token-indexed H.

@@ -255,7 +255,7 @@ __device__ __forceinline__ void shrink_body(const ApplyArgs& a, int b, int c, in
 constexpr int kProbesPerLane = 4;
 template <bool PA>
 __device__ __forceinline__ bool wait_partials(const ApplyArgs& a, const Block& blk, int rank, int* s_flag,
-                                              uint32_t wmask = 1u) {
+                                              uint32_t wmask = 1u, int col = 0) {
   constexpr int kProbes = PA ? kProbesPerLane : 1;
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
@@ -276,7 +276,7 @@ __device__ __forceinline__ bool wait_partials(const ApplyArgs& a, const Block& b
         const int kc = k - rg * a.n_chunks;
         // Only slices whose shrink side writes (one A per slice, table mode).
         if (!PA || ((wmask >> sa) & 1u))
-          probe[q] = static_cast<uint32_t>((kc * a.ptok + blk.first) * a.hs + sa * a.hs1 + rg * a.srows);
+          probe[q] = static_cast<uint32_t>((kc * a.ptok + blk.first) * a.hs + sa * a.hs1 + rg * a.srows + col);
       }
     }
     int ok = 1;
@@ -312,13 +312,15 @@ __device__ __forceinline__ bool wait_partials(const ApplyArgs& a, const Block& b
 // (Sharing a unit between lanes and combining with shuffles cost the
 // single-slice kernel spills and measured slower.)  emit(j, r0, v2)
 // receives each unit.
+// col: the first column collected in a partial row (the same in
+// wait_partials and clear_partials).
 template <int CB, typename Emit>
 __device__ __forceinline__ void collect_partials(const ApplyArgs& a, const Block& blk, const int R2, float alpha,
-                                                  Emit emit) {
+                                                  Emit emit, int col = 0) {
   const int n_units = blk.count * R2;
   const int nch = a.n_chunks;
   const uint32_t cstride = static_cast<uint32_t>(a.ptok) * static_cast<uint32_t>(a.hs) * 4u;
-  const char* pbase = reinterpret_cast<const char*>(a.part + static_cast<int64_t>(blk.first) * a.hs);
+  const char* pbase = reinterpret_cast<const char*>(a.part + static_cast<int64_t>(blk.first) * a.hs + col);
   for (int u = threadIdx.x; u < n_units; u += kThreads) {
     const int j = u / R2;
     const int r0 = (u - j * R2) * 2;
@@ -379,7 +381,8 @@ __device__ __forceinline__ void await_partials(const ApplyArgs& a, const Block& 
 // (count x rank values of every d-range) once its last reader is done, so the
 // next call finds the buffer empty.  `nthreads` threads take part.  Like every
 // access to the partial buffer, the stores are device-coherent.
-__device__ __forceinline__ void clear_partials(const ApplyArgs& a, const Block& blk, int rank, int tid, int nthreads) {
+__device__ __forceinline__ void clear_partials(const ApplyArgs& a, const Block& blk, int rank, int tid, int nthreads,
+                                               int col = 0) {
   const int r4 = rank / 4;
   const int per_chunk = blk.count * r4;
   const int total = per_chunk * a.n_chunks;
@@ -389,7 +392,7 @@ __device__ __forceinline__ void clear_partials(const ApplyArgs& a, const Block& 
     const int q = u - c * per_chunk;
     const int j = q / r4;
     const int r0 = (q - j * r4) * 4;
-    coherent_store_f4(a.part + (static_cast<int64_t>(c) * a.ptok + blk.first + j) * a.hs + r0, e);
+    coherent_store_f4(a.part + (static_cast<int64_t>(c) * a.ptok + blk.first + j) * a.hs + r0 + col, e);
   }
 }
 
@@ -852,22 +855,24 @@ __device__ __forceinline__ void expand_body(const ApplyArgs& a, int b, int p, co
   }
 }
 
-// shrink() of decode-sized plans (role kShrinkOnly): block b's one reader
-// sums its partials into H[token] = rn(alpha * sum_c part[c]) and, once
-// every thread has read its words, restores kPartialEmpty over them.
+// shrink() of decode-sized plans (role kShrinkOnly): block b's one reader of
+// A slice sa sums its partials into H[token] = rn(alpha * sum_c part[c]) and,
+// once every thread has read its words, restores kPartialEmpty over them.
 template <typename T>
-__device__ __forceinline__ void reduce_to_h(const ApplyArgs& a, int b, const Block& blk, int* s_flag,
+__device__ __forceinline__ void reduce_to_h(const ApplyArgs& a, int b, int sa, const Block& blk, int* s_flag,
                                             PreEntry pre = PreEntry{}) {
-  const Resolved<T> res = resolve_a<T>(a, blk, 0, pre);
+  const Resolved<T> res = resolve_a<T>(a, blk, sa, pre);
   // Rank rows the shrink side wrote (none if it could not resolve the adapter).
   const int wrote = res.ptr != nullptr ? res.rank : 0;
   if (wrote <= 0) return;
-  if (blk.count * wrote * a.n_chunks > 2048) wait_partials<false>(a, blk, wrote, s_flag);
+  const int col = sa * a.hs1;
+  if (blk.count * wrote * a.n_chunks > 2048) wait_partials<false>(a, blk, wrote, s_flag, 1u, col);
   T* H = static_cast<T*>(a.h);
   const int32_t* toks = a.plan.bperm + static_cast<int64_t>(b) * kBlockTokens;
   const bool f32 = a.h_f32 != 0;
+  const int64_t h0 = sa * a.ldy;
   collect_partials<8>(a, blk, wrote / 2, res.alpha, [&](int j, int r0, f32x2 v) {
-    const int64_t at = static_cast<int64_t>(toks[j]) * a.ldh + r0;
+    const int64_t at = h0 + static_cast<int64_t>(toks[j]) * a.ldh + r0;
     if (f32) {
       // fp32 H (vLLM's lora_shrink buffer): added to, not rounded.
       f32x2* hp = reinterpret_cast<f32x2*>(static_cast<float*>(a.h) + at);
@@ -878,10 +883,10 @@ __device__ __forceinline__ void reduce_to_h(const ApplyArgs& a, int b, const Blo
     o[0] = static_cast<T>(v[0]);
     o[1] = static_cast<T>(v[1]);
     *reinterpret_cast<typename VecOf<T>::v2*>(H + at) = o;
-  });
+  }, col);
   trace_stamp(a, 4);
   __syncthreads();
-  clear_partials(a, blk, wrote, threadIdx.x, kThreads);
+  clear_partials(a, blk, wrote, threadIdx.x, kThreads, col);
 }
 
 // ---------------------------------------------------------------- kernels ----
@@ -964,13 +969,15 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   T* s_h = reinterpret_cast<T*>(smem.buf());
   const int S = ROLE == kExpandOnly ? 0 : n_shrink;
   const int wg = static_cast<int>(blockIdx.x);
-  // shrink() with a.red_first: the block reducers are workgroups
-  // 0..n_slots-1, resident from the start, and the shrink workgroups follow.
+  // shrink() with a.red_first: the block reducers (one per A slice) are
+  // workgroups 0..n_red-1, resident from the start, and the shrink workgroups
+  // follow.
   const bool red_first = ROLE == kShrinkOnly && a.red_first != 0;
-  const bool shrink_role = ROLE != kExpandOnly && (red_first ? wg >= a.n_slots : wg < S);
+  const int n_red = PA ? a.n_slots * per_block : a.n_slots;
+  const bool shrink_role = ROLE != kExpandOnly && (red_first ? wg >= n_red : wg < S);
   int b, part;
   if (shrink_role) {
-    const int sw = red_first ? wg - a.n_slots : wg;
+    const int sw = red_first ? wg - n_red : wg;
     b = sw / per_shrink;
     part = sw - b * per_shrink;
   } else {
@@ -1033,7 +1040,7 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
     return;
   }
   if constexpr (ROLE == kShrinkOnly) {
-    reduce_to_h<T>(a, b, blk, &s_flag, pre);
+    reduce_to_h<T>(a, b, PA ? part : 0, blk, &s_flag, pre);
   } else if constexpr (RANK != 0) {
     expand_body<T, RANK, ROLE, TILES, PA>(a, b, part, blk, t0, s_h, smem.stage(), &s_flag, pre);
   } else if constexpr (PA) {
@@ -1446,9 +1453,10 @@ hipError_t launch_shrink_t(const ApplyArgs& a0, hipStream_t stream) {
 template <typename T, int RANK, int ROLE, int TILES>
 void launch_kernel(const ApplyArgs& a, dim3 grid, int32_t per_shrink, int32_t n_shrink, int32_t per_block,
                    hipStream_t stream) {
-  // One A per slice only in the fused roles; a separate instantiation, so the
-  // shared-A kernels keep their constant indexing and single-probe gate.
-  if constexpr (ROLE == kFused || ROLE == kFusedMulti) {
+  // One A per slice not in expand() (its H is the caller's); a separate
+  // instantiation, so the shared-A kernels keep their constant indexing and
+  // single-probe gate.
+  if constexpr (ROLE != kExpandOnly) {
     if (a.w.n_a > 1) {
       apply_kernel<T, RANK, ROLE, TILES, true><<<grid, kThreads, 0, stream>>>(
           a.plan.header, a.plan.blocks, a.plan.bperm, per_shrink, n_shrink, per_block, a);
@@ -1969,8 +1977,9 @@ hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, hipStream_t stream)
   return dtype_bf16 ? launch_shrink_t<__bf16>(a, stream) : launch_shrink_t<_Float16>(a, stream);
 }
 hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
-  if (a.srows != kShrinkRowsFused || a.n_ochunks != 1 || a.n_sub != 1 || a.n_chunks < 1 || a.n_chunks > kMaxChunks ||
-      a.w.n_a != 1)
+  if (a.srows != kShrinkRowsFused || a.n_ochunks != a.w.n_a || a.n_sub != 1 || a.n_chunks < 1 ||
+      a.n_chunks > kMaxChunks || a.w.n_a < 1 || a.w.n_a > kMaxSlices || a.hs != a.w.n_a * a.hs1 ||
+      a.n_chunks * a.hs > kMaxChunks * kMaxRank || (a.w.n_a > 1 && (a.w.mode != kStacked || a.rank == 0)))
     return hipErrorInvalidValue;
   return launch_role<kShrinkOnly>(dtype_bf16, a, stream);
 }

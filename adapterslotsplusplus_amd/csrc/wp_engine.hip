@@ -148,15 +148,17 @@ inline void shrink_split(int d, int rank, int rows, int n_a, int hs, int64_t slo
 // about 512 columns (each wave's share one batch of loads), or 1024 columns
 // past eight ranges (fewer workgroups than residency rounds; measured on
 // MI355X at d = 13824, and at d = 5120: cfg3 gate/up 42.8 -> 42.2 us per
-// call), at most kMaxChunks; one reducer workgroup per block.
+// call), at most kMaxChunks; one reducer workgroup per block and A slice.
 inline void shrink_small_split(int d, int rank, ApplyArgs* a) {
   int64_t n = std::max<int64_t>(ceil_div(d, 512), 1);
   if (n > 8) n = std::min<int64_t>(ceil_div(d, 1024), kMaxChunks);
+  // The A slices' partials side by side, within the partial buffer.
+  n = std::min<int64_t>(n, kMaxChunks * kMaxRank / a->hs);
   a->dc = static_cast<int>(ceil_div(ceil_div(d, n), 128) * 128);
   a->n_chunks = static_cast<int>(ceil_div(d, a->dc));
   a->srows = kShrinkRowsFused;
   a->n_rgroups = shrink_rank_groups(rank, kShrinkRowsFused);
-  a->n_ochunks = 1;
+  a->n_ochunks = a->w.n_a;
   a->n_sub = 1;
 }
 
@@ -560,6 +562,13 @@ bool fused_fits(const wp_engine* e, int rank, int n_a, int64_t n_ochunks) {
 bool small_shrink_fits(const wp_engine* e, int rank) {
   if (e->plan_bt <= kFineTokens) return true;
   return has_fine(e) && e->plan_T <= 2048 && e->plan_T * (rank != 0 ? rank : 32) <= 65536;
+}
+
+// A small shrink's reducers go first when they take at most half of the
+// resident workgroups: they then poll while the shrink workgroups stream
+// instead of being dispatched after them.
+int reducers_first(const wp_engine* e, const ApplyArgs& a) {
+  return 2 * static_cast<int64_t>(a.n_slots) * a.w.n_a <= static_cast<int64_t>(e->n_cu) * shrink_small_waves_per_simd() ? 1 : 0;
 }
 
 // expand() over 16-token blocks, one tile in flight at eight waves per SIMD, or
@@ -1411,10 +1420,7 @@ int wp_shrink(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t ran
     // block (the fused calls' shrink side), not one workgroup per block and
     // d-range streaming every rank row.
     shrink_small_split(d_model, rank, &a);
-    // The reducers first when they take at most half of the resident
-    // workgroups: they then poll while the shrink workgroups stream instead
-    // of being dispatched after them.
-    a.red_first = 2 * static_cast<int64_t>(a.n_slots) <= static_cast<int64_t>(e->n_cu) * shrink_small_waves_per_simd() ? 1 : 0;
+    a.red_first = reducers_first(e, a);
     WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, a, stream));
   } else {
     shrink_range_split(d_model, &a);
@@ -1830,17 +1836,11 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
   a.ldy = out_slice_stride;
   a.h_f32 = 1;
   if (small) {
-    for (int s = 0; s < n_slices; ++s) {
-      ApplyArgs as = a;
-      as.w.n_a = 1;
-      as.hs = rank;
-      as.w.a_base[0] = wa[s];
-      as.w.a_stride[0] = wa_stride0[s];
-      as.h = out + s * out_slice_stride;
-      shrink_small_split(d_model, rank, &as);
-      as.red_first = 2 * static_cast<int64_t>(as.n_slots) <= static_cast<int64_t>(e->n_cu) * shrink_small_waves_per_simd() ? 1 : 0;
-      WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, as, stream));
-    }
+    // Every slice in one launch: a launch takes 7 us at 48 tokens, its bytes
+    // under 1 (a step of four layers, three slices each 125 -> 68 us, MI355X).
+    shrink_small_split(d_model, rank, &a);
+    a.red_first = reducers_first(e, a);
+    WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, a, stream));
   } else {
     shrink_range_split(d_model, &a);
     a.part = e->spart;

@@ -381,3 +381,30 @@ def test_lora_expand_h_rows_and_modes(T, rows, rank, add_inputs):
         ref[3, 4:] = 0
     assert_close(y, ref, f"lora_expand {rows}")
     assert eng.device_errors() == 1
+
+
+@pytest.mark.parametrize("T", [5, 130, 512])
+@pytest.mark.parametrize("rank,n,d", [(8, 2, 136), (32, 3, 4096), (64, 2, 10240), (64, 4, 6152)])
+def test_lora_shrink_slices_one_launch(T, rank, n, d):
+    """lora_shrink of several A slices on a decode-sized table: the slices'
+    partials side by side in the partial buffer (four of rank 64 fill it with
+    four d-ranges), one reducer per block and slice, added to a buffer that
+    already holds values and has wider rows than the rank; run twice, so that
+    the first call has to leave the partial buffer empty."""
+    dtype, L = torch.float16, 6
+    announce(f"lora_shrink slices T={T} r={rank} n={n} d={d}")
+    ids = torch.from_numpy(np.random.default_rng(T + n).integers(-1, L, size=T).astype(np.int64))
+    was, _, _ = weights(L, rank, d, (16,) * n, dtype, 900)
+    x = randn((T, d), 910, dtype)
+    h0 = randn((n, T, rank + 4), 911, torch.float32)
+    eng = WarpPipeEngine(WarpPipeConfig(max_tokens=512))
+    assert eng.build_seg_bounds(ids.cuda())
+    h = h0.cuda()
+    for _ in range(2):
+        assert eng.lora_shrink(h, x.cuda(), was, 0.5)
+    torch.cuda.synchronize()
+    ref = h0
+    for _ in range(2):
+        ref = v1_ops.lora_shrink(ref, x, cpu(was), 0.5, ids)
+    assert_close(h, ref, "lora_shrink slices", rtol=1e-4, atol=1e-4)
+    assert eng.device_errors() == 0
