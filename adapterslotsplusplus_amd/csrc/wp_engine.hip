@@ -186,6 +186,9 @@ constexpr int32_t kMaxTableIds = 1 << 22;
 // Column-tile counters of linear_lora: (token groups x output columns / 16)
 // of one call at most.
 constexpr int kLinCounters = 1 << 16;
+// Tokens whose partials (kMaxChunks d-ranges of kMaxRank columns) the fused
+// calls' buffer holds.
+constexpr int kPartTokens = 2048;
 // Staging slots an engine may have (publications are applied by one thread each).
 constexpr int kMaxStagingSlots = 256;
 
@@ -220,7 +223,7 @@ struct wp_engine {
   int32_t* bperm = nullptr;     // [block_cap][kBlockTokens]
   uint32_t* consumed = nullptr; // [block_cap][kCounterStride]
   Entry* plan_entries = nullptr;
-  float* part = nullptr;        // [kMaxChunks][ptok][kMaxRank] fp32 partial H of fused calls (kPartialEmpty between calls)
+  float* part = nullptr;        // fp32 partial H of fused calls: [d-ranges][fused_ptok][hs] (kPartialEmpty between calls)
   float* spart = nullptr;       // [kMaxChunks][tok_cap][kMaxRank] d-range partials of shrink() launches (no invariant)
   void* hbuf = nullptr;         // [tok_cap][kMaxSlices x kMaxRank] 2-byte H of large-plan add_lora calls
   SlotPub* pubs = nullptr;      // [num_staging_slots] staging publications
@@ -237,7 +240,6 @@ struct wp_engine {
   bool plan_bentries = false;   // the last build_seg_bounds plan wrote bentries
   int table_cap = 0;
   int seg_cap = 0, block_cap = 0, tok_cap = 0, entry_cap = 0;
-  int ptok = 0;                 // plan positions `part` holds (fused_ptok: those a call spreads its d-ranges by)
   uint64_t part_words = 0, consumed_words = 0;
   int n_cu = 256;  // compute units of the device
   int32_t entry_offset = 0;  // table-mode calls on device-built plans read dtable + entry_offset
@@ -521,7 +523,16 @@ bool has_fine(const wp_engine* e) { return e->plan_bt <= kFineTokens || e->plan_
 // as close as the plan allows (decode-sized plans keep theirs within 64 KB of
 // each other at rank 32).
 int fused_ptok(const wp_engine* e) {
-  return static_cast<int>(std::min<int64_t>(e->ptok, std::max<int64_t>(ceil_div(e->plan_T, kSmallPlanTokens), 1) * kSmallPlanTokens));
+  const int64_t up = std::max<int64_t>(ceil_div(e->plan_T, kSmallPlanTokens), 1) * kSmallPlanTokens;
+  return static_cast<int>(std::min<int64_t>(up, e->tok_cap));
+}
+
+// A call's partials fit the buffer: the rules below keep them inside (at most
+// kPartTokens tokens at 64 columns, more at fewer).
+int check_part(const wp_engine* e, const char* who, const ApplyArgs& a) {
+  if (static_cast<uint64_t>(a.n_chunks) * a.hs * a.ptok > e->part_words)
+    return fail(WP_ERR_CAPACITY, "%s: the call's partials exceed the engine's buffer", who);
+  return WP_OK;
 }
 
 // Which of a plan's two tables a call runs on, past kSmallPlanTokens tokens
@@ -722,8 +733,7 @@ int wp_create(const wp_config* cfg_in, wp_engine** out) {
   e->block_cap = cfg.max_tokens + kRefMaxSegments;
   e->entry_cap = kRefMaxSegments;
   e->table_cap = cfg.max_adapter_ids;
-  e->ptok = cfg.max_tokens;
-  e->part_words = static_cast<uint64_t>(kMaxChunks) * e->ptok * kMaxRank;
+  e->part_words = static_cast<uint64_t>(kMaxChunks) * std::min(cfg.max_tokens, kPartTokens) * kMaxRank;
   e->consumed_words = static_cast<uint64_t>(e->block_cap) * kCounterStride;
   size_t off = 0;
   auto carve = [&](size_t bytes) {
@@ -746,10 +756,10 @@ int wp_create(const wp_config* cfg_in, wp_engine** out) {
   const size_t o_fblk = carve(sizeof(Block) * e->block_cap);
   const size_t o_fbperm = carve(sizeof(int32_t) * static_cast<size_t>(e->block_cap) * kBlockTokens);
   const size_t o_fbent = carve(sizeof(Entry) * e->block_cap);
+  const size_t o_part = carve(sizeof(float) * e->part_words);
   const size_t o_spart = carve(sizeof(float) * kMaxChunks * static_cast<size_t>(e->tok_cap) * kMaxRank);
   const size_t hbuf_bytes = sizeof(uint16_t) * static_cast<size_t>(e->tok_cap) * kMaxSlices * kMaxRank;
   const size_t o_hbuf = carve(hbuf_bytes);
-  const size_t o_part = carve(sizeof(float) * e->part_words);
   if (hipMalloc(reinterpret_cast<void**>(&e->ws), off) != hipSuccess)
     return bail(fail(WP_ERR_HIP, "wp_create: workspace allocation (%zu bytes) failed", off));
   e->header = reinterpret_cast<uint32_t*>(e->ws + o_hdr);
@@ -771,8 +781,10 @@ int wp_create(const wp_config* cfg_in, wp_engine** out) {
   e->spart = reinterpret_cast<float*>(e->ws + o_spart);
   e->hbuf = e->ws + o_hbuf;
   e->part = reinterpret_cast<float*>(e->ws + o_part);
-  // Everything starts at zero except the partials (kPartialEmpty) and the
-  // publications' ids (-1: nothing published); filled by kernels, then waited for.
+  // Everything before the partials starts at zero, the partials at
+  // kPartialEmpty, the publications' ids at -1 (nothing published); the d-range
+  // partials of shrink() and the H rows behind them need no state.  Filled by
+  // kernels, then waited for.
   if (launch_fill_u32(reinterpret_cast<uint32_t*>(e->ws), 0u, o_part / 4, nullptr) != hipSuccess ||
       launch_fill_u32(reinterpret_cast<uint32_t*>(e->part), kPartialEmpty, e->part_words, nullptr) != hipSuccess)
     return bail(fail(WP_ERR_HIP, "wp_create: workspace fill failed"));
@@ -1421,6 +1433,7 @@ int wp_shrink(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t ran
     // d-range streaming every rank row.
     shrink_small_split(d_model, rank, &a);
     a.red_first = reducers_first(e, a);
+    if ((rc = check_part(e, "shrink", a)) != WP_OK) return rc;
     WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, a, stream));
   } else {
     shrink_range_split(d_model, &a);
@@ -1535,6 +1548,7 @@ int add_lora_impl(wp_engine* e, const char* who, void* y, const void* x, int32_t
     return WP_OK;
   }
   fused_split(&a, rank, d_model, e->n_cu);
+  if ((rc = check_part(e, who, a)) != WP_OK) return rc;
   WP_HIP(launch_fused(dtype == WP_DTYPE_BF16, a, stream));
   return WP_OK;
 }
@@ -1614,6 +1628,7 @@ int wp_linear_lora(wp_engine* e, void* y, const void* x, const void* w, int64_t 
   l.hflag = e->lin_flag;
   l.hcnt = e->lin_flag + e->block_cap;
   if (a.n_slots > e->block_cap) return fail(WP_ERR_CAPACITY, "%s: more block slots than the engine holds", who);
+  if ((rc = check_part(e, who, a)) != WP_OK) return rc;
   WP_HIP(launch_linear(dtype == WP_DTYPE_BF16, a, l, stream));
   return WP_OK;
 }
@@ -1676,6 +1691,7 @@ int wp_shrink_expand(wp_engine* e, const void* X, void* Y, int32_t d_model, int3
   a.n_ochunks = a.w.oc_start[1];
   a.n_slots = block_bound(e, resolvable_ids(e, stream), true);
   fused_split(&a, rank, d_model, e->n_cu);
+  if ((rc = check_part(e, "shrink_expand", a)) != WP_OK) return rc;
   WP_HIP(launch_fused(dtype == WP_DTYPE_BF16, a, stream));
   return WP_OK;
 }
@@ -1761,6 +1777,7 @@ int wp_shrink_expand_slices(wp_engine* e, const void* X, void* Y, int32_t d_mode
   const int64_t window = ids_per_layer > 0 ? ids_per_layer : static_cast<int64_t>(e->table_cap);
   a.n_slots = block_bound(e, call_ids(e, stream, static_cast<int64_t>(e->adapters.size()), window), true);
   fused_split(&a, rank, d_model, e->n_cu);
+  if ((rc = check_part(e, "shrink_expand_slices", a)) != WP_OK) return rc;
   WP_HIP(launch_fused(dtype == WP_DTYPE_BF16, a, stream));
   return WP_OK;
 }
@@ -1840,6 +1857,7 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
     // under 1 (a step of four layers, three slices each 125 -> 68 us, MI355X).
     shrink_small_split(d_model, rank, &a);
     a.red_first = reducers_first(e, a);
+    if ((rc = check_part(e, who, a)) != WP_OK) return rc;
     WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, a, stream));
   } else {
     shrink_range_split(d_model, &a);
