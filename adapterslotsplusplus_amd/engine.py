@@ -27,6 +27,7 @@ Additions (each a superset of the reference behaviour):
 from __future__ import annotations
 
 import ctypes
+import struct
 from typing import List, Optional, Sequence, Tuple
 
 import torch
@@ -44,15 +45,27 @@ def _dtype_code(t: torch.Tensor, what: str) -> int:
     return code
 
 
-def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _ptr(t: torch.Tensor) -> int:
+    return t.data_ptr()
 
 
 def _current_raw_stream(device_index: int) -> int:
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is not None:
-        return int(raw(device_index))
     return int(torch.cuda.current_stream(device_index).cuda_stream)
+
+
+# The raw handle of torch's current stream on a device, without a
+# torch.cuda.Stream object per call.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or _current_raw_stream
+
+# Argument arrays of 64-bit (pointers, strides) and 32-bit values as bytes
+# objects, which ctypes passes as they are: a third of a ctypes array's cost.
+# 32-bit values wrap, as a ctypes array's do; the library checks them.
+def _i64s(v) -> bytes:
+    return struct.pack(f"{len(v)}q", *v)
+
+
+def _i32s(v) -> bytes:
+    return struct.pack(f"{len(v)}I", *[k & 0xFFFFFFFF for k in v])
 
 
 class _Ext:
@@ -125,10 +138,8 @@ class WarpPipeEngine:
         except Exception:
             pass
 
-    def _stream(self) -> ctypes.c_void_p:
-        # The raw handle of torch's current stream on the engine's device,
-        # without building a torch.cuda.Stream object per call.
-        return ctypes.c_void_p(_current_raw_stream(self._dev_index))
+    def _stream(self) -> int:
+        return _raw_stream(self._dev_index)
 
     def _on_device(self, t: torch.Tensor, what: str) -> None:
         # get_device() is an int (-1 on the CPU): cheaper per call than
@@ -213,13 +224,13 @@ class WarpPipeEngine:
         self._on_device(idx, "token_lora_indices")
         if idx.dtype not in (torch.int64, torch.int32):
             idx = idx.to(torch.int64)
-        idx = idx.reshape(-1)
+        if idx.dim() != 1:
+            idx = idx.reshape(-1)
         if not idx.is_contiguous():
             idx = idx.contiguous()
-        T = int(idx.numel())
-        rc = _lib.check(self._lib.wp_build_seg_bounds(self._handle, _ptr(idx), 1 if idx.dtype == torch.int64 else 0,
-                                                      T, self._stream()), "build_seg_bounds")
-        return rc == _lib.WP_OK
+        rc = self._lib.wp_build_seg_bounds(self._handle, idx.data_ptr(), 1 if idx.dtype == torch.int64 else 0,
+                                           idx.numel(), _raw_stream(self._dev_index))
+        return _lib.check(rc, "build_seg_bounds") == _lib.WP_OK
 
     def read_segments(self) -> List[Tuple[int, int, int]]:
         """The current segment table as (adapter_id, token_start, token_count)
@@ -440,67 +451,83 @@ class WarpPipeEngine:
         [L, 1, r, d] tensor shared by every slice (one shrink: packed q/k/v over
         one A) or a sequence with one per slice (vLLM's packed layers, each slice
         with its own lora_a); x is read once either way."""
+        # An eager call is bound by this function, not by its kernel (a tenth
+        # of a microsecond per tensor query): each tensor's shape is read once
+        # and nothing is reshaped that is 2-D already.
         per_slice_a = isinstance(wa_t_all, (list, tuple))
-        was = list(wa_t_all) if per_slice_a else [wa_t_all]
-        rank = int(wb_t_alls[0].size(-1))
-        ok = self._ranks.get(rank)
-        if ok is None:
-            ok = self._ranks[rank] = bool(self._ext.rank_supported(rank))
-        if not ok:
+        was = wa_t_all if per_slice_a else (wa_t_all,)
+        rank = wb_t_alls[0].size(-1)
+        if not self._rank_ok(rank):
             return False
-        self._on_device(x, "x")
-        self._on_device(y, "y")
-        dt = _dtype_code(x, "x")
-        if (y.dtype != x.dtype or any(w.dtype != x.dtype for w in was)
-                or any(w.dtype != x.dtype for w in wb_t_alls)):
+        dev = self._dev_index
+        if x.get_device() != dev or y.get_device() != dev:
+            self._on_device(x, "x")
+            self._on_device(y, "y")
+        dtype = x.dtype
+        dt = _DTYPES.get(dtype)
+        if dt is None:
+            _dtype_code(x, "x")
+        same = y.dtype == dtype
+        for w in was:
+            same = same and w.dtype == dtype
+        for w in wb_t_alls:
+            same = same and w.dtype == dtype
+        if not same:
             raise RuntimeError("add_lora_packed: x, y and the LoRA weights must share one dtype")
-        x2 = x.reshape(-1, x.size(-1))
-        y2 = y.reshape(-1, y.size(-1))
+        x2 = x if x.dim() == 2 else x.reshape(-1, x.size(-1))
+        y2 = y if y.dim() == 2 else y.reshape(-1, y.size(-1))
         if not (x2.is_contiguous() and y2.is_contiguous()):
             raise RuntimeError("add_lora_packed: x/y must be contiguous")
-        if y2.data_ptr() != y.data_ptr():
+        if y2 is not y and y2.data_ptr() != y.data_ptr():
             raise RuntimeError("add_lora_packed: y must be viewable as 2-D in place")
-        if not all(w.is_contiguous() for w in was) or not all(w.is_contiguous() for w in wb_t_alls):
+        whole = True
+        for w in was:
+            whole = whole and w.is_contiguous()
+        for w in wb_t_alls:
+            whole = whole and w.is_contiguous()
+        if not whole:
             raise RuntimeError("add_lora_packed: wa_t_all/wb_t_all must be contiguous")
-        T = int(x2.size(0))
-        d_model = int(x2.size(1))
-        L = int(was[0].size(0))
+        T, d_model = x2.shape
+        L = was[0].size(0)
         n = len(wb_t_alls)
         if per_slice_a and len(was) != n:
             raise RuntimeError(f"add_lora_packed: {len(was)} lora_a tensors for {n} slices")
         for w in was:
-            self._on_device(w, "wa_t_all")
-            if int(w.size(0)) != L or int(w.size(-1)) != d_model or int(w.size(-2)) != rank:
-                raise RuntimeError(f"add_lora_packed: wa_t_all {tuple(w.shape)} does not match x and rank {rank}")
+            if w.get_device() != dev:
+                self._on_device(w, "wa_t_all")
+            s = w.shape
+            if s[0] != L or s[-1] != d_model or s[-2] != rank:
+                raise RuntimeError(f"add_lora_packed: wa_t_all {tuple(s)} does not match x and rank {rank}")
         outs = []
         for i, w in enumerate(wb_t_alls):
-            self._on_device(w, "wb_t_all")
-            if int(w.size(0)) != L or int(w.size(-1)) != rank:
-                raise RuntimeError(f"add_lora_packed: wb_t_all {tuple(w.shape)} does not match wa_t_all")
-            o = int(w.size(-2))
+            if w.get_device() != dev:
+                self._on_device(w, "wb_t_all")
+            s = w.shape
+            if s[0] != L or s[-1] != rank:
+                raise RuntimeError(f"add_lora_packed: wb_t_all {tuple(s)} does not match wa_t_all")
+            o = s[-2]
             if y_slice_sizes is not None and y_slice_sizes[i] is not None and int(y_slice_sizes[i]) != o:
                 raise RuntimeError(f"add_lora_packed: y_slice_size {y_slice_sizes[i]} != wb_t_all rows {o}")
             outs.append(o)
-        if int(y2.size(0)) != T:
+        Ty, width = y2.shape
+        if Ty != T:
             raise RuntimeError("add_lora_packed: x and y have different token counts")
-        wb_ptrs = (ctypes.c_void_p * n)(*[w.data_ptr() for w in wb_t_alls])
-        wb_strides = (ctypes.c_int64 * n)(*[int(w.stride(0)) for w in wb_t_alls])
-        o_arr = (ctypes.c_int32 * n)(*outs)
-        off_arr = (ctypes.c_int32 * n)(*[int(v) for v in y_offsets])
+        wb_ptrs = _i64s([w.data_ptr() for w in wb_t_alls])
+        wb_strides = _i64s([w.stride(0) for w in wb_t_alls])
+        o_arr = _i32s(outs)
+        off_arr = _i32s([int(v) for v in y_offsets])
+        stream = _raw_stream(dev)
         if per_slice_a:
-            wa_ptrs = (ctypes.c_void_p * n)(*[w.data_ptr() for w in was])
-            wa_strides = (ctypes.c_int64 * n)(*[int(w.stride(0)) for w in was])
-            rc = _lib.check(self._lib.wp_add_lora_nslice(self._handle, _ptr(y2), _ptr(x2), n, wa_ptrs, wa_strides,
-                                                         wb_ptrs, wb_strides, o_arr, off_arr, L, float(scale), rank,
-                                                         d_model, T, int(y2.size(1)), dt, self._stream()),
-                            "add_lora_packed_nslice")
+            rc = self._lib.wp_add_lora_nslice(self._handle, y2.data_ptr(), x2.data_ptr(), n,
+                                              _i64s([w.data_ptr() for w in was]), _i64s([w.stride(0) for w in was]),
+                                              wb_ptrs, wb_strides, o_arr, off_arr, L, float(scale), rank, d_model, T,
+                                              width, dt, stream)
         else:
             wa = was[0]
-            rc = _lib.check(self._lib.wp_add_lora(self._handle, _ptr(y2), _ptr(x2), _ptr(wa), int(wa.stride(0)), L, n,
-                                                  wb_ptrs, wb_strides, o_arr, off_arr, float(scale), rank, d_model, T,
-                                                  int(y2.size(1)), dt, self._stream()),
-                            "add_lora_packed")
-        return rc == _lib.WP_OK
+            rc = self._lib.wp_add_lora(self._handle, y2.data_ptr(), x2.data_ptr(), wa.data_ptr(), wa.stride(0), L, n,
+                                       wb_ptrs, wb_strides, o_arr, off_arr, float(scale), rank, d_model, T, width, dt,
+                                       stream)
+        return _lib.check(rc, "add_lora_packed_nslice" if per_slice_a else "add_lora_packed") == _lib.WP_OK
 
     def add_lora_packed_nslice(self, y, x, lora_a_stacked, lora_b_stacked, scale, output_slices) -> bool:
         """vLLM's PunicaWrapper.add_lora_packed_nslice shape: slice i has its own
@@ -512,7 +539,7 @@ class WarpPipeEngine:
         for o in output_slices:
             offs.append(acc)
             acc += int(o)
-        return self.add_lora_slices(y, x, list(lora_a_stacked), list(lora_b_stacked), scale, offs,
+        return self.add_lora_slices(y, x, list(lora_a_stacked), lora_b_stacked, scale, offs,
                                     [int(o) for o in output_slices])
 
     # ------------------------------------------------- vLLM V1 LoRA ops --
@@ -532,14 +559,14 @@ class WarpPipeEngine:
 
     def _stacked(self, ts: Sequence[torch.Tensor], dtype, what: str):
         for t in ts:
-            self._on_device(t, what)
+            if t.get_device() != self._dev_index:
+                self._on_device(t, what)
             if t.dtype != dtype:
                 raise RuntimeError(f"{what} must have the activations' dtype {dtype}, got {t.dtype}")
-            if t.dim() < 2 or not t[0].is_contiguous():
+            # A contiguous stack's matrices are contiguous; others are looked at one by one.
+            if t.dim() < 2 or not ((t.is_contiguous() and t.size(0) > 0) or t[0].is_contiguous()):
                 raise RuntimeError(f"{what}: each adapter's matrix must be contiguous")
-        n = len(ts)
-        return ((ctypes.c_void_p * n)(*[t.data_ptr() for t in ts]),
-                (ctypes.c_int64 * n)(*[int(t.stride(0)) for t in ts]))
+        return _i64s([t.data_ptr() for t in ts]), _i64s([t.stride(0) for t in ts])
 
     def lora_shrink(self, out: torch.Tensor, x: torch.Tensor, lora_a_stacked: Sequence[torch.Tensor],
                     scale: float) -> bool:
@@ -550,45 +577,60 @@ class WarpPipeEngine:
         Tokens without an adapter keep their rows."""
         was = list(lora_a_stacked)
         n = len(was)
-        rank = int(was[0].size(-2))
-        if n < 1 or n > 4 or not self._rank_ok(rank) or any(int(w.size(-2)) != rank for w in was):
+        rank = was[0].size(-2)
+        if n < 1 or n > 4 or not self._rank_ok(rank):
             return False
+        for w in was:
+            if w.size(-2) != rank:
+                return False
         self._on_device(x, "x")
         dt = _dtype_code(x, "x")
-        x2 = x.reshape(-1, x.size(-1))
+        x2 = x if x.dim() == 2 else x.reshape(-1, x.size(-1))
         if not x2.is_contiguous():
             raise RuntimeError("lora_shrink: x must be contiguous")
-        T, d = int(x2.size(0)), int(x2.size(1))
-        L = int(was[0].size(0))
-        if any(int(w.size(0)) != L or int(w.size(-1)) != d for w in was):
-            raise RuntimeError("lora_shrink: every lora_a must be [L, 1, r, d] with x's d")
+        T, d = x2.shape
+        L = was[0].size(0)
+        for w in was:
+            if w.size(0) != L or w.size(-1) != d:
+                raise RuntimeError("lora_shrink: every lora_a must be [L, 1, r, d] with x's d")
         a_ptrs, a_strides = self._stacked(was, x.dtype, "lora_a_stacked")
-        outs = list(out) if isinstance(out, (list, tuple)) else [out[s] for s in range(int(out.size(0)))]
-        if len(outs) != n:
-            raise RuntimeError(f"lora_shrink: {len(outs)} output slices for {n} lora_a tensors")
-        o0 = outs[0]
-        for o in outs:
-            self._on_device(o, "out")
-            if o.dtype != torch.float32 or o.dim() != 2 or o.stride(1) != 1 or int(o.size(0)) < T:
+        if isinstance(out, torch.Tensor) and out.dim() == 3 and out.size(0) == n:
+            # One buffer: its slices are evenly spaced and alike.
+            self._on_device(out, "out")
+            ss, row, unit = out.stride()
+            if out.dtype != torch.float32 or unit != 1 or out.size(1) < T:
                 raise RuntimeError("lora_shrink: out slices must be fp32 [T, >= rank] with unit column stride")
-            if o.stride(0) != o0.stride(0):
-                raise RuntimeError("lora_shrink: out slices must share one row stride")
-        row = int(o0.stride(0))
-        sstride = (outs[1].data_ptr() - o0.data_ptr()) // 4 if n > 1 else 0
-        if any(outs[s].data_ptr() != o0.data_ptr() + 4 * s * sstride for s in range(n)) or sstride < 0:
-            raise RuntimeError("lora_shrink: out slices must be evenly spaced in one buffer")
-        rc = _lib.check(self._lib.wp_lora_shrink(self._handle, _ptr(o0), sstride, row, _ptr(x2), n, a_ptrs, a_strides, L,
-                                                 float(scale), rank, d, T, dt, self._stream()), "lora_shrink")
-        return rc == _lib.WP_OK
+            base, sstride = out.data_ptr(), ss if n > 1 else 0
+        else:
+            outs = list(out) if isinstance(out, (list, tuple)) else [out[s] for s in range(int(out.size(0)))]
+            if len(outs) != n:
+                raise RuntimeError(f"lora_shrink: {len(outs)} output slices for {n} lora_a tensors")
+            o0 = outs[0]
+            for o in outs:
+                self._on_device(o, "out")
+                if o.dtype != torch.float32 or o.dim() != 2 or o.stride(1) != 1 or int(o.size(0)) < T:
+                    raise RuntimeError("lora_shrink: out slices must be fp32 [T, >= rank] with unit column stride")
+                if o.stride(0) != o0.stride(0):
+                    raise RuntimeError("lora_shrink: out slices must share one row stride")
+            row = o0.stride(0)
+            base = o0.data_ptr()
+            sstride = (outs[1].data_ptr() - base) // 4 if n > 1 else 0
+            if any(outs[s].data_ptr() != base + 4 * s * sstride for s in range(n)) or sstride < 0:
+                raise RuntimeError("lora_shrink: out slices must be evenly spaced in one buffer")
+        rc = self._lib.wp_lora_shrink(self._handle, base, sstride, row, x2.data_ptr(), n, a_ptrs, a_strides, L,
+                                      float(scale), rank, d, T, dt, _raw_stream(self._dev_index))
+        return _lib.check(rc, "lora_shrink") == _lib.WP_OK
 
     def _bias_args(self, biases, y, n: int, what: str):
-        bs = list(biases) if biases is not None else [None] * n
+        if biases is None:
+            return _i64s([0] * n), _i64s([0] * n), False
+        bs = list(biases)
         if len(bs) != n:
             raise RuntimeError(f"{what}: {len(bs)} biases for {n} slices")
         ptrs, strides = [], []
         for b in bs:
             if b is None:
-                ptrs.append(None)
+                ptrs.append(0)
                 strides.append(0)
                 continue
             self._on_device(b, "lora_bias_stacked")
@@ -599,7 +641,7 @@ class WarpPipeEngine:
                 raise RuntimeError(f"{what}: each adapter's bias row must be contiguous")
             ptrs.append(b.data_ptr())
             strides.append(int(b2.stride(0)))
-        return (ctypes.c_void_p * n)(*ptrs), (ctypes.c_int64 * n)(*strides), any(b is not None for b in bs)
+        return _i64s(ptrs), _i64s(strides), any(b is not None for b in bs)
 
     def add_bias(self, y: torch.Tensor, lora_bias_stacked, output_slices: Sequence[int], num_loras: int,
                  offset_start: int = 0) -> None:
@@ -614,8 +656,8 @@ class WarpPipeEngine:
         n = len(output_slices)
         offs = [int(offset_start) + sum(int(o) for o in output_slices[:i]) for i in range(n)]
         b_ptrs, b_strides, _ = self._bias_args(lora_bias_stacked, y, n, "add_bias")
-        o_arr = (ctypes.c_int32 * n)(*[int(o) for o in output_slices])
-        off_arr = (ctypes.c_int32 * n)(*offs)
+        o_arr = _i32s([int(o) for o in output_slices])
+        off_arr = _i32s(offs)
         _lib.check(self._lib.wp_add_bias(self._handle, _ptr(y2), int(y2.size(1)), n, b_ptrs, b_strides, o_arr, off_arr,
                                          int(num_loras), int(y2.size(0)), dt, self._stream()), "add_bias")
 
@@ -631,35 +673,44 @@ class WarpPipeEngine:
         an adapter keep their rows."""
         wbs = list(lora_b_stacked)
         n = len(wbs)
-        rank = int(wbs[0].size(-1))
-        if n < 1 or n > 4 or not self._rank_ok(rank) or any(int(w.size(-1)) != rank for w in wbs):
+        rank = wbs[0].size(-1)
+        if n < 1 or n > 4 or not self._rank_ok(rank):
             return False
+        for w in wbs:
+            if w.size(-1) != rank:
+                return False
         self._on_device(y, "y")
         self._on_device(h, "h")
         dt = _dtype_code(y, "y")
-        y2 = y.reshape(-1, y.size(-1))
-        if not y2.is_contiguous() or y2.data_ptr() != y.data_ptr():
+        y2 = y if y.dim() == 2 else y.reshape(-1, y.size(-1))
+        if not y2.is_contiguous() or (y2 is not y and y2.data_ptr() != y.data_ptr()):
             raise RuntimeError("lora_expand: y must be contiguous")
-        T = int(y2.size(0))
-        if h.dim() != 3 or int(h.size(0)) != n or h.stride(2) != 1 or int(h.size(1)) < T or int(h.size(2)) < rank:
+        T, width = y2.shape
+        hs = h.shape
+        if len(hs) != 3 or hs[0] != n or h.stride(2) != 1 or hs[1] < T or hs[2] < rank:
             raise RuntimeError(f"lora_expand: h must be [{n}, >= {T}, >= {rank}] with unit column stride")
-        if h.dtype not in (torch.float32, y.dtype):
+        f32 = h.dtype == torch.float32
+        if not f32 and h.dtype != y.dtype:
             raise RuntimeError("lora_expand: h must be fp32 or y's dtype")
-        L = int(wbs[0].size(0))
+        L = wbs[0].size(0)
         outs = [int(o) for o in output_slices]
-        if len(outs) != n or any(int(w.size(0)) != L or int(w.size(-2)) != o for w, o in zip(wbs, outs)):
+        fit = len(outs) == n
+        if fit:
+            for w, o in zip(wbs, outs):
+                fit = fit and w.size(0) == L and w.size(-2) == o
+        if not fit:
             raise RuntimeError("lora_expand: lora_b_stacked[s] must be [L, 1, output_slices[s], r]")
         b_ptrs, b_strides = self._stacked(wbs, y.dtype, "lora_b_stacked")
         bias_ptrs, bias_strides, _ = self._bias_args(lora_bias_stacked, y, n, "lora_expand")
-        offs = [int(offset_start) + sum(outs[:i]) for i in range(n)]
-        o_arr = (ctypes.c_int32 * n)(*outs)
-        off_arr = (ctypes.c_int32 * n)(*offs)
-        rc = _lib.check(self._lib.wp_lora_expand(self._handle, _ptr(y2), int(y2.size(1)), _ptr(h),
-                                                 1 if h.dtype == torch.float32 else 0, int(h.stride(0)),
-                                                 int(h.stride(1)), n, b_ptrs, b_strides, o_arr, off_arr, bias_ptrs,
-                                                 bias_strides, L, rank, T, 1 if add_inputs else 0, dt, self._stream()),
-                        "lora_expand")
-        return rc == _lib.WP_OK
+        offs, at = [], int(offset_start)
+        for o in outs:
+            offs.append(at)
+            at += o
+        rc = self._lib.wp_lora_expand(self._handle, y2.data_ptr(), width, h.data_ptr(), 1 if f32 else 0, h.stride(0),
+                                      h.stride(1), n, b_ptrs, b_strides, _i32s(outs), _i32s(offs), bias_ptrs,
+                                      bias_strides, L, rank, T, 1 if add_inputs else 0, dt,
+                                      _raw_stream(self._dev_index))
+        return _lib.check(rc, "lora_expand") == _lib.WP_OK
 
     # ------------------------------------------------------------- staging --
     def prefetch_adapter(self, adapter_id, layer=None) -> int:
