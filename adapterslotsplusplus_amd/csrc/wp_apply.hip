@@ -72,6 +72,9 @@ constexpr int kTilesInFlight = kBlockTokens / 16;
 // shrink(): its LDS (two A slices and one X tile per wave: 52 KB at rank 64)
 // holds three workgroups per compute unit.
 constexpr int kShrinkWavesPerSimd = 3;
+// K-slices a shrink_kernel wave holds in flight (three and four measured the
+// same: one compute unit's reads are the limit, not their latency).
+constexpr int kShrinkDepth = 2;
 
 // kFusedMulti: fused, with several output chunks per expand workgroup.
 // kShrinkOnly: shrink() of decode-sized plans: the fused shrink side, and
@@ -1161,13 +1164,16 @@ hipError_t launch_expand_ext_d(const ApplyArgs& a, const ExpandExt& x, hipStream
 // (rows x kSliceK) is loaded once per workgroup and shared by the four
 // waves through LDS (double buffered), and each wave, which owns one
 // 16-token tile, loads its X through a tile of its own.  The
-// block's d-ranges are summed by its last workgroup to finish (a counter per
-// block and group), in d-range order, so the bits do not depend on timing;
+// d-ranges of a 16-token tile are summed by its last wave to finish (a counter
+// per tile and group), in d-range order, so the bits do not depend on timing;
 // nothing waits on another workgroup.
 //
-// A launch takes 10 us however small (a chain of loads, eight slices two at a
-// time, the last arriver's sum), and at 8192 tokens one compute unit's read
-// rate bounds it (X and A of three workgroups at about 40 GB/s).  So one launch
+// One compute unit's read rate bounds it: 35-40 GB/s whatever is in flight (a
+// 16-token workgroup's 8 slices take 5 us, and three or four slices in flight
+// the same), so at 8192 tokens and rank 64 the units that drew three
+// workgroups' X and A set the time, 25.7 us (X alone takes 13 us at the copy rate).
+// Launch overhead and the partial sums are the rest, and a launch never costs
+// less than 10 us.  So one launch
 // for every A slice, with X read once per 64 rows, replaced one launch each:
 // q/k/v with three A of rank 16, call total on MI355X 53.3 -> 34.3 us at 2048
 // tokens, 116 -> 84 at 8192 (rank 64: 79 -> 64, 157 -> 132).  512-column
@@ -1176,6 +1182,8 @@ constexpr int kSliceK = 128;
 constexpr int kSliceStride = kSliceK + 8;  // LDS row stride of an A slice: 16-byte skew per row
 // Words between the counters of a block's slice groups (64 bytes).
 constexpr int kGroupCounter = kCounterStride / kMaxSlices;
+// ... and between those of a group's 16-token tiles.
+constexpr int kTileCounter = kGroupCounter / (kBlockTokens / 16);
 
 // MT: 16-row MFMA tiles of a group's rows (of the largest rank if kMixed).
 // The leading scalar arguments arrive in SGPRs at wave launch, as apply_kernel's do.
@@ -1191,7 +1199,6 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
   // Each wave's X tile of the current slice: only that wave reads it, after
   // writing it, so one buffer suffices.
   __shared__ T s_x[kWaves][16 * kSliceStride];
-  __shared__ int s_last;
   const int tid = static_cast<int>(threadIdx.x);
   const int b = static_cast<int>(blockIdx.x) / per_block;
   const int part = static_cast<int>(blockIdx.x) - b * per_block;
@@ -1303,6 +1310,9 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
     }
 #pragma unroll
     for (int i = 0; i < XL; ++i) *reinterpret_cast<u32x4*>(&sx[(xrow + 4 * i) * kSliceStride + xcol]) = sl.x[i];
+    // The registers are free: the slice kShrinkDepth ahead goes out before the
+    // barrier and the MFMAs.
+    if (more) load_slice(sl, next_k);
     // The slice is in LDS for every wave; the other buffer was last read
     // before this barrier, so the next slice may be written into it.
     lds_barrier();
@@ -1321,7 +1331,6 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
         }
       }
     }
-    if (more) load_slice(sl, next_k);
   };
   // Fully unrolled over the workgroup's kShrinkSlices slices: every path
   // issues the same loads, so each wait is for exactly one slice.  A short
@@ -1329,18 +1338,17 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
   // Blocks of one adapter read the same A slices; each block starts at a
   // different slice of its range (rotation by block index) so that they do
   // not all hit the same lines at once.
-  Slice q0, q1;
+  Slice q[kShrinkDepth];
   for (; k0 < kc_end; k0 += kShrinkSlices * kSliceK, k1 = min(k0 + kShrinkSlices * kSliceK, kc_end)) {
     const int n_sl = (k1 - k0 + kSliceK - 1) / kSliceK;
     const int rot = b % n_sl;
     auto slice_k = [&](int i) { return k0 + (i + rot < n_sl ? i + rot : i + rot - n_sl) * kSliceK; };
-    load_slice(q0, slice_k(0));
-    load_slice(q1, slice_k(1 % n_sl));
 #pragma unroll
-    for (int i = 0; i < kShrinkSlices; i += 2) {
-      run_slice(q0, 0, slice_k(i % n_sl), i < n_sl, i + 2 < kShrinkSlices, slice_k((i + 2) % n_sl));
-      run_slice(q1, 1, slice_k((i + 1) % n_sl), i + 1 < n_sl, i + 3 < kShrinkSlices, slice_k((i + 3) % n_sl));
-    }
+    for (int i = 0; i < kShrinkDepth; ++i) load_slice(q[i], slice_k(i % n_sl));
+#pragma unroll
+    for (int i = 0; i < kShrinkSlices; ++i)
+      run_slice(q[i % kShrinkDepth], i & 1, slice_k(i % n_sl), i < n_sl, i + kShrinkDepth < kShrinkSlices,
+                slice_k((i + kShrinkDepth) % n_sl));
   }
   trace_stamp(a, 2);
   // acc[m]: rows m*16 + 4*(lane/16) + [0, 4) of token slot tl.
@@ -1365,38 +1373,50 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
     }
     return;
   }
-  // Partial of this d-range, stored coherently; the stores have landed
-  // before the count (s_waitcnt), so the last workgroup sees them all.
-  float* prow = a.part + static_cast<int64_t>(blk.first) * a.hs + s0 * rank;
-  const int64_t cs = static_cast<int64_t>(a.ptok) * a.hs;
+  // Partial of this d-range, stored coherently.  From here on each wave is on
+  // its own: its 16-token tile is counted and, by the tile's last wave to
+  // finish, summed and stored without waiting for the workgroup's other tiles.
+  // The partials move as 16-byte sc1 accesses: as pairs of 8 bytes they cost the
+  // loop itself, through the memory side, as much as the sum.  At 8192 tokens,
+  // rank 64, d = 4096 (trace): loop done by 22.9 -> 21.2 us, counted by 24.9 ->
+  // 22.2, last H 29.3 -> 25.0.
+  if (!wave_live) return;
+  // Byte offsets in the partials (at most kMaxChunks x kMaxRank floats per token).
+  const uint32_t cs = static_cast<uint32_t>(a.ptok) * static_cast<uint32_t>(a.hs) * 4u;
+  const auto pbuf = coherent_buffer(a.part, cs * static_cast<uint32_t>(n_kc));
+  const uint32_t prow = (static_cast<uint32_t>(blk.first + wave * 16) * static_cast<uint32_t>(a.hs) + s0 * rank) * 4u;
   if (tok >= 0) {
 #pragma unroll
     for (int m = 0; m < MT; ++m)
-      if (m * 16 + rq < n_rows) coherent_store_f4(prow + c * cs + static_cast<int64_t>(tl) * a.hs + m * 16 + rq, acc[m]);
+      if (m * 16 + rq < n_rows) coherent_store16(pbuf, prow + c * cs + (row * a.hs + m * 16 + rq) * 4u, acc[m]);
   }
+  // The stores have landed before the count, so the last wave sees them all.
   wait_vm();
-  __syncthreads();
-  uint32_t* counter = &a.consumed[static_cast<int64_t>(b) * kCounterStride + grp * kGroupCounter];
-  if (tid == 0) s_last = atomic_add_u(counter, 1u) == static_cast<unsigned>(n_kc - 1) ? 1 : 0;
-  __syncthreads();
+  uint32_t* counter = &a.consumed[static_cast<int64_t>(b) * kCounterStride + grp * kGroupCounter + wave * kTileCounter];
+  unsigned seen = 0;
+  if (lane == 0) seen = atomic_add_u(counter, 1u);
+  seen = __builtin_amdgcn_readfirstlane(seen);
   trace_stamp(a, 3);
-  if (s_last == 0) return;
-  // Last workgroup of the block and group: H = rn(alpha * sum_c part[c]) in
-  // d-range order, then the counter is reset for the next call.  The partials
-  // are left as they are: every launch writes each word it later reads (the
-  // buffer is shrink()'s own, not the fused calls' with its empty pattern).
+  if (seen != static_cast<unsigned>(n_kc - 1)) return;
+  // Last wave of the tile: H = rn(alpha * sum_c part[c]) in d-range order,
+  // then the counter is reset for the next call.  The partials are left as they
+  // are: every launch writes each word it later reads (the buffer is shrink()'s
+  // own, not the fused calls' with its empty pattern).
+  const int tile_tokens = min(16, blk.count - wave * 16);
   const int r4 = n_rows >> 2;
-  const int units = blk.count * r4;
-  // A thread's units are tid + 256 i (at most kBlockTokens * kMaxRank / 4 /
-  // 256 = 4); their loads go out together, four d-ranges at a time.
-  constexpr int kUnits = kBlockTokens * kMaxRank / 4 / kThreads;
-  const float* p0[kUnits];
+  const int units = tile_tokens * r4;
+  // A lane's units are lane + 64 i; their loads go out together, four d-ranges
+  // at a time.
+  constexpr int kUnits = MT;  // 16 tokens x MT * 16 rows / 4 / 64
+  uint32_t p0[kUnits];
   f32x4 sum[kUnits];
+  int32_t utok[kUnits];
 #pragma unroll
   for (int i = 0; i < kUnits; ++i) {
-    const int u = min(tid + i * kThreads, units - 1);
+    const int u = min(lane + i * 64, units - 1);
     const int j = u / r4;
-    p0[i] = prow + static_cast<int64_t>(j) * a.hs + (u - j * r4) * 4;
+    p0[i] = prow + (j * a.hs + (u - j * r4) * 4) * 4u;
+    utok[i] = __shfl(tok, j, 64);
     sum[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   for (int c0 = 0; c0 < n_kc; c0 += 4) {
@@ -1404,7 +1424,7 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int i = 0; i < kUnits; ++i) v[q][i] = coherent_load_f4(p0[i] + min(c0 + q, n_kc - 1) * cs);
+      for (int i = 0; i < kUnits; ++i) v[q][i] = coherent_load16(pbuf, p0[i] + min(c0 + q, n_kc - 1) * cs);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -1413,13 +1433,10 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
   }
 #pragma unroll
   for (int i = 0; i < kUnits; ++i) {
-    const int u = tid + i * kThreads;
-    if (u < units) {
-      const int j = u / r4;
-      put_h(bp[j], (u - j * r4) * 4, sum[i] * res.alpha);
-    }
+    const int u = lane + i * 64;
+    if (u < units) put_h(utok[i], (u - (u / r4) * r4) * 4, sum[i] * res.alpha);
   }
-  if (tid == 0) atomic_store_u(counter, 0u);
+  if (lane == 0) atomic_store_u(counter, 0u);
   trace_stamp(a, 4);
 }
 

@@ -103,6 +103,19 @@ __device__ __forceinline__ void coherent_store_f4(float* p, f32x4 v) {
   coherent_store8(p, __builtin_bit_cast(unsigned long long, u32x2{u[0], u[1]}));
   coherent_store8(p + 2, __builtin_bit_cast(unsigned long long, u32x2{u[2], u[3]}));
 }
+// Device-scope (sc1) 16-byte accesses to a scratch buffer by byte offset, for
+// words that are read only once a count has said they are there (unlike the
+// 8-byte ones above, a 16-byte access is not one atomic access).
+constexpr int kSc1 = 16;  // the buffer instructions' sc1 bit
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t coherent_buffer(void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>(bytes), 0x00020000);
+}
+__device__ __forceinline__ f32x4 coherent_load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kSc1));
+}
+__device__ __forceinline__ void coherent_store16(__amdgpu_buffer_rsrc_t r, uint32_t off, f32x4 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off, 0, kSc1);
+}
 __device__ __forceinline__ unsigned atomic_load_u(const uint32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
