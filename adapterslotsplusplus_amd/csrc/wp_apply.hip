@@ -733,8 +733,14 @@ __device__ __forceinline__ void expand_body(const ApplyArgs& a, int b, int p, co
     }
     wrote = wmask != 0u ? W : 0;
   }
-  // Partial words per token the block's shrink side writes.
-  const int wrote_all = PA ? W * __builtin_popcount(wmask) : wrote;
+  // The slices whose H this workgroup collects: with one chunk, its slice's.
+  // (Every written slice has expand workgroups, each waits for its slice's
+  // words, and the block's partials are emptied once all have counted.)
+  const bool one_slice = PA && ROLE == kFused;
+  const int own = one_slice ? cur.h_col / a.hs1 : 0;
+  const uint32_t need = one_slice ? wmask & (1u << own) : wmask;
+  // Partial words per token it waits for.
+  const int wrote_all = PA ? W * __builtin_popcount(need) : wrote;
   V8 bf[kOT][KS];
   YRows yq;
   load_chunk<T, RANK, kDyn>(a, cur, tok0, bf, yq);
@@ -746,7 +752,7 @@ __device__ __forceinline__ void expand_body(const ApplyArgs& a, int b, int p, co
     // One A per slice over several chunks: a later chunk's slice may have
     // resolved where the first one's did not (table mode), so the workgroup
     // collects H if any slice wrote, and each chunk is tested on its own.
-    go = (PA && ROLE == kFusedMulti ? true : go) && wrote > 0;
+    go = (PA && ROLE == kFusedMulti ? true : go) && wrote > 0 && need != 0u;
     if (go) {
       // Workgroups of small blocks (at most 2048 partial words) poll the
       // data straight away; the probe gate in front pays off for larger
@@ -754,7 +760,7 @@ __device__ __forceinline__ void expand_body(const ApplyArgs& a, int b, int p, co
       // block: cfg5 (88 calls) 736 -> 696 us, cfg1 8.23 -> 7.78 us, cfg2
       // o_proj unchanged.
       go = (blk.count * wrote_all * a.n_chunks > 2048)
-               ? wait_partials<PA>(a, blk, wrote, s_flag, wmask)
+               ? wait_partials<PA>(a, blk, wrote, s_flag, need)
                : true;
       trace_stamp(a, 3);
       if (go) {
@@ -771,7 +777,8 @@ __device__ __forceinline__ void expand_body(const ApplyArgs& a, int b, int p, co
           if constexpr (ROLE == kFusedMulti) {
             collect_partials_pa<8>(a, blk, W, wmask, alphas, to_lds);
           } else {
-            collect_partials_pa<4>(a, blk, W, wmask, alphas, to_lds);
+            collect_partials<4>(a, blk, W / 2, slice_alpha(alphas, own),
+                                [&](int j, int r0, f32x2 v) { to_lds(j, cur.h_col + r0, v); }, cur.h_col);
           }
         } else if constexpr (MIX) {
           // The adapter's rank columns from the partials, zeros past it.

@@ -550,16 +550,17 @@ int check_part(const wp_engine* e, const char* who, const ApplyArgs& a) {
 //   33 / 39 vs 33 / 40; rank 64, 1536 25 / 30 vs 27 / 33, 2048 30 / 36 vs 30 / 34.
 //   3 x 4096 columns: rank 16, 2048 34 / 37 vs 38 / 44, 4096 57 / 63 vs 58 / 68;
 //   rank 64, 640 28 / 42 vs 32 / 48, 1024 37 / 50 vs 36 / 51.
-// With one A per slice the fused launch reads X per slice: ranks up to 32 and
-// 768 tokens (4096 + 2 x 1024 columns, rank 16, 640 tokens 18 / 22 vs 21 / 24,
-// 1024 22 / 29 vs 23 / 26; rank 32, 640 20 / 30 vs 24 / 35, 1024 30 / 37 vs 26 / 37;
-// rank 64, 640 33 / 47 vs 27 / 49).
+// With one A per slice the fused launch reads X per slice: rank times tokens up
+// to 32768, at most 1536 (4096 + 2 x 1024 columns, rank 8, 1024 tokens 17 / 20 vs
+// 19 / 22, 1536 22 / 25 vs 22 / 25; rank 16, 1024 19 / 23 vs 22 / 25; rank 32,
+// 1024 23 / 29 vs 24 / 35, 1536 30 / 37 vs 28 / 38; rank 64, 512 26 / 41 vs 26 /
+// 44, 640 27 / 45 vs 26 / 47, 1024 36 / 53 vs 32 / 51).
 // Mixed ranks count as 48 or 60: 2048 tokens 29 / 31 vs 31 / 34 (3072 39 / 42 vs
 // 34 / 38), to 13824 columns 1024 33 / 42 vs 39 / 48 (1536 45 / 50 vs 43 / 53).
 bool fused_fits(const wp_engine* e, int rank, int n_a, int64_t n_ochunks) {
   if (e->plan_bt <= kFineTokens) return true;
   if (!has_fine(e)) return false;
-  if (n_a > 1) return rank != 0 && rank <= 32 && e->plan_T <= 768;
+  if (n_a > 1) return rank != 0 && e->plan_T <= 1536 && e->plan_T * rank <= 32768;
   const bool wide = n_ochunks > 2 * kExpandWorkgroups;
   const int64_t r = rank != 0 ? rank : wide ? 60 : 48;
   return e->plan_T * r <= (wide ? 61440 : 98304);
@@ -1369,16 +1370,20 @@ void fused_split(ApplyArgs* a, int rank, int d_model, int n_cu) {
     // Several slices, but a grid small enough that the single-chunk kernel
     // (16-row shrink groups, one output chunk per expand workgroup, every
     // workgroup's B and Y loaded before the wait) needs at most twice the
-    // workgroups the device holds at once: that kernel, not the multi-chunk
-    // one that loads its later chunks only after the partials are in.
-    // Measured on MI355X: cfg5's q/k/v (one A per slice) 44-launch step
-    // 535 -> 462 us, cfg2 flatness at 1..16 resident adapters 183 -> 168 us
-    // (N=1); allowing three times the residency slowed cfg2's qkv call
-    // (18.0 -> 19.8 us).
+    // workgroups the device holds at once -- eight times with one A per slice,
+    // where a single-chunk workgroup collects its own slice's H only: that
+    // kernel, not the multi-chunk one that loads its later chunks only after
+    // the partials are in.  Measured on MI355X: cfg5's q/k/v (one A per slice)
+    // 44-launch step 535 -> 462 us, cfg2 flatness at 1..16 resident adapters 183
+    // -> 168 us (N=1); three times the residency slowed cfg2's shared-A qkv call
+    // (18.0 -> 19.8 us).  One A per slice, 4096 + 2 x 1024 columns, 64 adapters,
+    // multi- vs single-chunk: rank 32, 256 tokens 23.4 vs 18.9 us, 512 28.0 vs
+    // 23.0; rank 64, 128 tokens 31.1 vs 24.9, 512 44.7 vs 40.9; gate + up of 13824
+    // columns, mixed ranks, 64 tokens 30.3 vs 22.9.
     ApplyArgs one = *a;
     shrink_split(d_model, rank, kShrinkRows, a->w.n_a, a->hs, a->n_slots, a->n_ochunks, resident, &one);
     const int64_t per_block = static_cast<int64_t>(one.n_chunks) * one.n_rgroups * a->w.n_a + a->n_ochunks;
-    if (a->n_slots * per_block <= 2 * resident) {
+    if (a->n_slots * per_block <= (a->w.n_a > 1 ? 8 : 2) * resident) {
       one.n_sub = 1;
       *a = one;
       return;

@@ -778,8 +778,9 @@ TABLE_LINES = [
     (16, 6144, [132], False, "high"), (16, 6145, [132], False, "high"),
     (8, 8192, [516], False, "one"),
     (64, 960, [8452], False, "low"), (64, 961, [8452], False, "one"),     # ... over 32 output chunks
-    (32, 768, [260, 64], True, "low"), (32, 769, [260, 64], True, "high"),  # one A per slice
-    (64, 513, [260, 64], True, "one"),
+    (32, 1024, [260, 64], True, "low"), (32, 1025, [260, 64], True, "high"),  # one A per slice
+    (8, 1536, [260, 64, 20], True, "high"), (8, 1537, [260, 64, 20], True, "low"),
+    (64, 512, [260, 64], True, "one"), (64, 513, [260, 64], True, "one"),
 ]
 
 
