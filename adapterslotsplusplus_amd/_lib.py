@@ -43,7 +43,7 @@ EXPORTED = (
     "wp_add_lora_nslice", "wp_prefetch_adapters", "wp_release_prefetches", "wp_wait_prefetches", "wp_set_trace",
     "wp_shrink_expand_slices", "wp_linear_lora", "wp_read_probe",
     "wp_set_max_adapters", "wp_read_static_errors", "wp_poll_device_errors", "wp_lora_shrink", "wp_lora_expand",
-    "wp_add_bias", "wp_handoff_probe", "wp_barrier_probe",
+    "wp_add_bias", "wp_handoff_probe", "wp_barrier_probe", "wp_shrink_new",
 )
 
 
@@ -94,6 +94,7 @@ def load():
         "wp_read_plan": ([p, p, i64, p, i64, P(i64), P(i64), p], ctypes.c_int),
         "wp_read_device_errors": ([p, P(ctypes.c_uint32), p], ctypes.c_int),
         "wp_shrink": ([p, p, p, i32, i32, i64, i64, i32, p], ctypes.c_int),
+        "wp_shrink_new": ([p, p, p, i32, i32, i64, i64, i32, p], ctypes.c_int),
         "wp_expand": ([p, p, p, i32, i32, i64, i64, i64, i32, i32, p], ctypes.c_int),
         "wp_add_lora": ([p, p, p, p, i64, i32, i32, p, p, p, p, f32, i32, i32, i64, i64, i32, p], ctypes.c_int),
         "wp_prefetch_adapter": ([p, i32, P(i32)], ctypes.c_int),

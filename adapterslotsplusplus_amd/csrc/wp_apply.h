@@ -73,6 +73,11 @@ struct ApplyArgs {
   // I/O type.  At the end of the arguments: fields placed before the hot
   // kernels' argument reads measured up to 0.3 us more per launch.
   int32_t h_f32;
+  // shrink() of decode-sized plans into a new H: columns of a row that no rank
+  // fills, rows of skipped blocks and of tokens without an adapter are zeroed
+  // (h_fill: columns of a row, 0: H is the caller's; h_rows: its rows).
+  int32_t h_fill;
+  int32_t h_rows;
   int32_t pad_end;
 };
 
@@ -168,7 +173,8 @@ hipError_t launch_fused(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
 hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
 // shrink() of decode-sized plans: the fused kernel's shrink workgroups
 // (kShrinkRowsFused rows x d-range) of every A slice and one reducer per block
-// and slice writing its H at element s * a.ldy of a row;
+// and slice writing its H at element s * a.ldy of a row; with a.h_fill (one
+// slice, device-built plan) further workgroups clear what none writes;
 // a.part is the fused calls' partial buffer (kPartialEmpty between calls).
 hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
 // expand(): expand from a caller-provided token-indexed H.

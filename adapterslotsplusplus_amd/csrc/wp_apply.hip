@@ -879,6 +879,37 @@ __device__ __forceinline__ void expand_body(const ApplyArgs& a, int b, int p, co
   }
 }
 
+// Zeroes columns [from, a.h_fill) of the H rows of block b's tokens (a new H:
+// a.h_fill > 0), 8 columns per step.
+template <typename T>
+__device__ __forceinline__ void zero_h_rows(const ApplyArgs& a, const int32_t* toks, int count, int from) {
+  const int per = (a.h_fill - from) / 8;
+  for (int u = threadIdx.x; u < count * per; u += kThreads) {
+    const int j = u / per;
+    T* p = static_cast<T*>(a.h) + static_cast<int64_t>(toks[j]) * a.ldh + from + (u - j * per) * 8;
+    *reinterpret_cast<u32x4*>(p) = u32x4{0u, 0u, 0u, 0u};
+  }
+}
+
+// A new H's rows of tokens without an adapter, and past the plan's tokens:
+// 64 tokens per wave of workgroup z.
+template <typename T>
+__device__ __forceinline__ void zero_h_unrouted(const ApplyArgs& a, int z) {
+  const int lane = threadIdx.x & 63;
+  const int word = z * kWaves + (threadIdx.x >> 6);
+  const int plan_T = static_cast<int>(a.plan.header[kHdrT]);
+  const uint64_t mask =
+      word * 64 < plan_T ? reinterpret_cast<const uint64_t*>(a.plan.header + kHdrMask)[word] : 0ull;
+  const int per = a.h_fill / 8;
+  for (int u = lane; u < 64 * per; u += 64) {
+    const int j = u / per;
+    const int t = word * 64 + j;
+    if (t >= a.h_rows || ((mask >> j) & 1ull)) continue;
+    T* p = static_cast<T*>(a.h) + static_cast<int64_t>(t) * a.ldh + (u - j * per) * 8;
+    *reinterpret_cast<u32x4*>(p) = u32x4{0u, 0u, 0u, 0u};
+  }
+}
+
 // shrink() of decode-sized plans (role kShrinkOnly): block b's one reader of
 // A slice sa sums its partials into H[token] = rn(alpha * sum_c part[c]) and,
 // once every thread has read its words, restores kPartialEmpty over them.
@@ -888,11 +919,12 @@ __device__ __forceinline__ void reduce_to_h(const ApplyArgs& a, int b, int sa, c
   const Resolved<T> res = resolve_a<T>(a, blk, sa, pre);
   // Rank rows the shrink side wrote (none if it could not resolve the adapter).
   const int wrote = res.ptr != nullptr ? res.rank : 0;
+  const int32_t* toks = a.plan.bperm + static_cast<int64_t>(b) * kBlockTokens;
+  if (a.h_fill > wrote) zero_h_rows<T>(a, toks, blk.count, wrote);
   if (wrote <= 0) return;
   const int col = sa * a.hs1;
   if (blk.count * wrote * a.n_chunks > 2048) wait_partials<false>(a, blk, wrote, s_flag, 1u, col);
   T* H = static_cast<T*>(a.h);
-  const int32_t* toks = a.plan.bperm + static_cast<int64_t>(b) * kBlockTokens;
   const bool f32 = a.h_f32 != 0;
   const int64_t h0 = sa * a.ldy;
   collect_partials<8>(a, blk, wrote / 2, res.alpha, [&](int j, int r0, f32x2 v) {
@@ -998,6 +1030,14 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   // follow.
   const bool red_first = ROLE == kShrinkOnly && a.red_first != 0;
   const int n_red = PA ? a.n_slots * per_block : a.n_slots;
+  if constexpr (ROLE == kShrinkOnly && !PA) {
+    // Behind both roles: a new H's rows that no block holds.
+    if (wg >= n_red + n_shrink) {
+      touch_kernel_args_wait(ka_touch);
+      zero_h_unrouted<T>(a, wg - n_red - n_shrink);
+      return;
+    }
+  }
   const bool shrink_role = ROLE != kExpandOnly && (red_first ? wg >= n_red : wg < S);
   int b, part;
   if (shrink_role) {
@@ -1041,6 +1081,17 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   if (b == a.n_slots - 1 && part == 0 && threadIdx.x == 0 && n_blocks > a.n_slots)
     flag_error(a.plan.header, kErrCapacity);
   if constexpr (!PA || RANK == 0) touch_kernel_args_wait(ka_touch);
+  if constexpr (ROLE == kShrinkOnly && !PA) {
+    // A new H: blocks that are skipped (the partials are poisoned, or the plan
+    // has more blocks than the grid) leave zero rows.
+    if (a.h_fill > 0 && !shrink_role) {
+      if (poison != 0u && b < n_blocks && blk.count > 0)
+        zero_h_rows<T>(a, bperm + static_cast<int64_t>(b) * kBlockTokens, blk.count, 0);
+      if (b == a.n_slots - 1)
+        for (int q = a.n_slots; q < n_blocks; ++q)
+          zero_h_rows<T>(a, bperm + static_cast<int64_t>(q) * kBlockTokens, blocks[q].count, 0);
+    }
+  }
   if ((b >= n_blocks) | (blk.count <= 0) | (tok0 < -1) | (poison != 0u)) return;
   const int32_t t0 = row < blk.count ? tok0 : -1;
   trace_stamp(a, 1);
@@ -1510,7 +1561,8 @@ hipError_t launch_rank(const ApplyArgs& a, hipStream_t stream) {
   const int64_t S = ROLE == kExpandOnly ? 0 : static_cast<int64_t>(a.n_slots) * a.n_chunks * a.n_rgroups * a.w.n_a;
   const int64_t E = static_cast<int64_t>(a.n_slots) *
                     ((a.n_ochunks + a.n_sub - 1) / a.n_sub);
-  const int64_t n = S + E;
+  const int64_t Z = ROLE == kShrinkOnly && a.h_fill > 0 ? (a.h_rows + kThreads - 1) / kThreads : 0;
+  const int64_t n = S + E + Z;
   if (n <= 0) return hipSuccess;
   const dim3 grid(static_cast<unsigned>(n));
   const int32_t per_shrink = a.n_chunks * a.n_rgroups * a.w.n_a;
@@ -2017,7 +2069,8 @@ hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, hipStream_t stream)
 hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
   if (a.srows != kShrinkRowsFused || a.n_ochunks != a.w.n_a || a.n_sub != 1 || a.n_chunks < 1 ||
       a.n_chunks > kMaxChunks || a.w.n_a < 1 || a.w.n_a > kMaxSlices || a.hs != a.w.n_a * a.hs1 ||
-      a.n_chunks * a.hs > kMaxChunks * kMaxRank || (a.w.n_a > 1 && (a.w.mode != kStacked || a.rank == 0)))
+      a.n_chunks * a.hs > kMaxChunks * kMaxRank || (a.w.n_a > 1 && (a.w.mode != kStacked || a.rank == 0)) ||
+      (a.h_fill > 0 && (a.w.n_a > 1 || a.h_f32 != 0 || a.h_fill % 8 != 0 || a.ldh % 8 != 0 || a.h_rows < 1)))
     return hipErrorInvalidValue;
   return launch_role<kShrinkOnly>(dtype_bf16, a, stream);
 }

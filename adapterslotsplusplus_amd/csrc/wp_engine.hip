@@ -742,7 +742,7 @@ int wp_create(const wp_config* cfg_in, wp_engine** out) {
     off += (bytes + 255) & ~size_t(255);
     return at;
   };
-  const size_t o_hdr = carve(sizeof(uint32_t) * kHdrWords);
+  const size_t o_hdr = carve(sizeof(uint32_t) * kHdrWords + sizeof(uint64_t) * mask_words(e->tok_cap));
   const size_t o_seg = carve(sizeof(Segment) * e->seg_cap);
   const size_t o_blk = carve(sizeof(Block) * e->block_cap);
   const size_t o_perm = carve(sizeof(int32_t) * e->tok_cap);
@@ -1396,8 +1396,13 @@ void fused_split(ApplyArgs* a, int rank, int d_model, int n_cu) {
 
 }  // namespace
 
-int wp_shrink(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t rank, int64_t T, int64_t h_row_stride,
-              int32_t dtype, void* stream_) {
+}  // extern "C"
+
+namespace {
+
+// wp_shrink, and (fresh) wp_shrink_new: H's rows are the caller's, or all new.
+int shrink_impl(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t rank, int64_t T, int64_t h_row_stride,
+                int32_t dtype, bool fresh, void* stream_) {
   if (!e) return fail(WP_ERR_INVALID, "shrink: engine is NULL");
   if (rank != 0 && !rank_ok(rank)) return fail(WP_ERR_INVALID, "dispatch_bgmv_shrink: unsupported rank (only 8/16/32/64)");
   int rc = check_io("shrink", dtype, X, "X");
@@ -1439,14 +1444,37 @@ int wp_shrink(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t ran
     shrink_small_split(d_model, rank, &a);
     a.red_first = reducers_first(e, a);
     if ((rc = check_part(e, "shrink", a)) != WP_OK) return rc;
+    if (fresh && e->plan_kind == 2 && T > 0 && T < (int64_t{1} << 31)) {
+      // Zeroes go out with the H rows: a fill of its own took 5 us of a call's
+      // 20 (a 512-token step of three shrink() calls 141.4 -> 136.7 us, MI355X).
+      a.h_fill = static_cast<int32_t>(h_row_stride);
+      a.h_rows = static_cast<int32_t>(T);
+    } else if (fresh) {
+      WP_HIP(launch_fill_u32(static_cast<uint32_t*>(H), 0u, static_cast<size_t>(T * h_row_stride / 2), stream));
+    }
     WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, a, stream));
   } else {
+    if (fresh) WP_HIP(launch_fill_u32(static_cast<uint32_t*>(H), 0u, static_cast<size_t>(T * h_row_stride / 2), stream));
     shrink_range_split(d_model, &a);
     a.part = e->spart;
     a.ptok = e->tok_cap;
     WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, a, stream));
   }
   return WP_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int wp_shrink(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t rank, int64_t T, int64_t h_row_stride,
+              int32_t dtype, void* stream) {
+  return shrink_impl(e, X, H, d_model, rank, T, h_row_stride, dtype, false, stream);
+}
+
+int wp_shrink_new(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t rank, int64_t T, int64_t h_row_stride,
+                  int32_t dtype, void* stream) {
+  return shrink_impl(e, X, H, d_model, rank, T, h_row_stride, dtype, true, stream);
 }
 
 int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_t rank, int64_t T, int64_t h_row_stride,
@@ -2058,6 +2086,8 @@ constexpr size_t kSOffBperm = align256(kSOffPerm + sizeof(int32_t) * kStaticToke
 constexpr size_t kSOffCons = align256(kSOffBperm + sizeof(int32_t) * kStaticBlockCap * kBlockTokens);
 constexpr size_t kSOffPart = align256(kSOffCons + sizeof(uint32_t) * kStaticBlockCap * kCounterStride);
 constexpr size_t kStaticBytes = align256(kSOffPart + sizeof(float) * kMaxChunks * kStaticTokens * kMaxRank);
+static_assert(kSOffSeg - kSOffHdr >= sizeof(uint32_t) * kHdrWords + sizeof(uint64_t) * mask_words(kStaticTokens),
+              "the plan's token mask behind the header");
 static_assert(kStaticBytes == WP_STATIC_SCRATCH_BYTES, "WP_STATIC_SCRATCH_BYTES in the C header");
 
 }  // namespace

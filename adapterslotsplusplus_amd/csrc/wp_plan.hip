@@ -494,7 +494,10 @@ __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, 
     live[e] = __ballot(ok);
     key[e] = static_cast<uint32_t>(static_cast<int>(ids[e]));
     if (ok && key[e] > kmax) kmax = key[e];
-    if (lane == 0) s_start[first + e] = start[e];
+    if (lane == 0) {
+      s_start[first + e] = start[e];
+      if (i < T) reinterpret_cast<uint64_t*>(header + kHdrMask)[first + e] = live[e];
+    }
   }
   kmax = wave_all_reduce(kmax, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
   const uint64_t any_todo = __ballot(todo != 0);

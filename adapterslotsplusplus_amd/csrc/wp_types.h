@@ -96,8 +96,12 @@ enum HeaderWord : int {
   // build without copies stores the complement of the current version, so
   // copies an earlier build left behind never count as current.
   kHdrPlanVer = 10,
-  kHdrWords = 16
+  kHdrWords = 16,
+  // Behind the header: one 64-bit word per 64 tokens of a device-built plan,
+  // bit t set if token t has an adapter (id >= 0).
+  kHdrMask = kHdrWords
 };
+inline constexpr int mask_words(int64_t T) { return static_cast<int>((T + 63) / 64); }
 
 // Bits of header[kHdrErrors], set by kernels that had to skip work.
 enum DeviceError : uint32_t {

@@ -304,16 +304,17 @@ class WarpPipeEngine:
         if X.numel() < T * int(d_model):
             raise RuntimeError(f"X has {X.numel()} elements, fewer than total_tokens x d_model")
         width = rank if rank else 64
+        shrink = self._lib.wp_shrink
         if out is None:
-            H = torch.zeros(T, width, dtype=X.dtype, device=X.device)
+            H = torch.empty(T, width, dtype=X.dtype, device=X.device)
+            shrink = self._lib.wp_shrink_new
         else:
             H = out
             self._on_device(H, "out")
             if H.dtype != X.dtype or not H.is_contiguous() or tuple(H.shape) != (T, width):
                 raise RuntimeError(f"out must be a contiguous [{T}, {width}] tensor of X's dtype")
         self._select_layer(layer)
-        _lib.check(self._lib.wp_shrink(self._handle, _ptr(X), _ptr(H), int(d_model), rank, T, width, dt,
-                                       self._stream()), "shrink")
+        _lib.check(shrink(self._handle, _ptr(X), _ptr(H), int(d_model), rank, T, width, dt, self._stream()), "shrink")
         return H
 
     def expand(self, H, Y, out_features, rank, y_offset: int = 0, layer=None):

@@ -190,6 +190,13 @@ int wp_poll_device_errors(wp_engine* e, uint32_t* flags, void* stream);
  * selects mixed-rank mode (each adapter's own rank, h_row_stride >= 64). */
 int wp_shrink(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t rank, int64_t T,
               int64_t h_row_stride, int32_t dtype, void* stream);
+/* wp_shrink into an uninitialised H: everything that wp_shrink leaves as it is
+ * (rows of tokens without an adapter, of skipped blocks and past the table;
+ * columns past an adapter's rank) is zeroed, in the same launch where the
+ * table is decode-sized.  H must be [T, h_row_stride] and is written whole. */
+int wp_shrink_new(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t rank, int64_t T,
+                  int64_t h_row_stride, int32_t dtype, void* stream);
+
 
 /* Replaces WarpPipeExtension::expand (bindings:141-148):
  *   Y[t, off + o] = rn(Y[t, off + o] + H[t, :] . B_a[o, :]) for every segment token. */

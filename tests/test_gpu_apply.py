@@ -868,3 +868,59 @@ def test_store_on_both_tables(T, rank):
         assert_close(Y, Y_ref, f"Y step {step}", slack=slack)
         assert_close(Y1, Y_ref, f"shrink_expand step {step}", slack=slack)
         assert engine.device_errors() == 0
+
+
+@pytest.mark.parametrize("T", [1, 63, 65, 500, 1025, 2049])
+@pytest.mark.parametrize("rank", [0, 16])
+def test_new_h_is_zero_where_nothing_is_written(T, rank):
+    """shrink() returns a new H: rows of tokens without an adapter, of ids that
+    are not registered (far more blocks of them than the grid has slots for),
+    past the table's tokens, and columns past an adapter's rank are zero over
+    memory that held NaN, also while the partials are poisoned."""
+    dtype, d, K, extra = torch.bfloat16, 136, 3, 70
+    announce(f"new H T={T} rank={rank}")
+    engine = WarpPipeEngine()
+    adapters = {}
+    for i in range(K):
+        r = rank or (8, 64, 32)[i]
+        A, B = randn((r, d), 1300 + i, dtype, 0.05), randn((8, r), 1310 + i, dtype, 0.02)
+        engine.register_adapter(i, A.cuda(), B.cuda(), 1.0, rank=r)
+        adapters[i] = (A, B, 1.0)
+    width = rank or 64
+    X = randn((T + extra, d), 1320, dtype)
+    xd = X.cuda()
+
+    def new_h():
+        # The allocator hands the freed NaN block to shrink()'s H.
+        dirty = torch.full((T + extra, width), float("nan"), dtype=dtype, device="cuda")
+        torch.cuda.synchronize()
+        del dirty
+        return engine.shrink(xd, d, rank, T + extra)
+
+    rng = np.random.default_rng(T)
+    for ids in (rng.integers(-1, K, size=T), np.where(np.arange(T) % 3 == 0, 1, 1000 + np.arange(T))):
+        assert engine.build_seg_bounds(torch.from_numpy(ids.astype(np.int64)).cuda())
+        H = new_h()
+        torch.cuda.synchronize()
+        known = np.where(ids < K, ids, -1)
+        ref = bgmv.shrink(X, so.seg_bounds(known).tolist(), adapters, width, T + extra)
+        got = H.float().cpu()
+        assert torch.isfinite(got).all()
+        if (ids < K).all():
+            assert_close(H, ref, "new H")
+        else:
+            # Ids that are not registered may crowd registered ones out of the grid.
+            wrote = got.abs().sum(1) > 0
+            assert_close(got[wrote], ref[wrote], "new H rows")
+            assert not got[torch.from_numpy(np.concatenate([known < 0, np.ones(extra, bool)]))].any()
+        engine.device_errors()
+    if T <= 512:
+        engine.set_spin_limit(0)
+        assert engine.build_seg_bounds(torch.zeros(T, dtype=torch.int64).cuda())
+        engine.shrink(xd, d, rank, T + extra)  # gives up where a word is not there at once
+        engine.set_spin_limit(None)
+        poisoned = new_h()
+        torch.cuda.synchronize()
+        assert torch.isfinite(poisoned.float()).all()
+        assert not poisoned[T:].any()
+        engine.device_errors()
