@@ -1245,11 +1245,10 @@ hipError_t launch_expand_ext_d(const ApplyArgs& a, const ExpandExt& x, hipStream
 // the same), so at 8192 tokens and rank 64 the units that drew three
 // workgroups' X and A set the time, 25.7 us (X alone takes 13 us at the copy rate).
 // Launch overhead and the partial sums are the rest, and a launch never costs
-// less than 10 us.  So one launch
+// less than 9 us.  So one launch
 // for every A slice, with X read once per 64 rows, replaced one launch each:
 // q/k/v with three A of rank 16, call total on MI355X 53.3 -> 34.3 us at 2048
-// tokens, 116 -> 84 at 8192 (rank 64: 79 -> 64, 157 -> 132).  512-column
-// d-ranges are slower from 2048 tokens up (8192, rank 64: 64.9 -> 73.5 us).
+// tokens, 116 -> 84 at 8192 (rank 64: 79 -> 64, 157 -> 132).
 constexpr int kSliceK = 128;
 constexpr int kSliceStride = kSliceK + 8;  // LDS row stride of an A slice: 16-byte skew per row
 // Words between the counters of a block's slice groups (64 bytes).
@@ -1258,8 +1257,10 @@ constexpr int kGroupCounter = kCounterStride / kMaxSlices;
 constexpr int kTileCounter = kGroupCounter / (kBlockTokens / 16);
 
 // MT: 16-row MFMA tiles of a group's rows (of the largest rank if kMixed).
+// NS: slices per pass over a d-range (kShrinkSlices, or half of it where the
+// d-ranges are that short).
 // The leading scalar arguments arrive in SGPRs at wave launch, as apply_kernel's do.
-template <typename T, int MT, bool kMixed>
+template <typename T, int MT, bool kMixed, int NS>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kShrinkWavesPerSimd)))
 void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, const int32_t* __restrict__ bperm,
                    int32_t n_kc, int32_t per_block, int32_t per_group, ApplyArgs a) {
@@ -1316,11 +1317,11 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
   const int n_rows = kMixed ? rank : min(per_group, a.w.n_a - s0) * rank;
   const int n_mt = kMixed ? (rank + 15) >> 4 : MT;
   const int d = a.d_model;
-  // The d-range [c * dc, ...) in passes of kShrinkSlices slices; k0/k1 are the current
+  // The d-range [c * dc, ...) in passes of NS slices; k0/k1 are the current
   // pass's bounds.
   const int kc_end = min((c + 1) * a.dc, d);
   int k0 = c * a.dc;
-  int k1 = min(k0 + kShrinkSlices * kSliceK, kc_end);
+  int k1 = min(k0 + NS * kSliceK, kc_end);
   const int32_t tok = tl < blk.count ? tok_in : -1;
   const bool wave_live = wave * 16 < blk.count;
   // Every load below is unconditional, at an address clamped into the
@@ -1404,22 +1405,22 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
       }
     }
   };
-  // Fully unrolled over the workgroup's kShrinkSlices slices: every path
+  // Fully unrolled over the workgroup's NS slices: every path
   // issues the same loads, so each wait is for exactly one slice.  A short
   // last d-range skips the MFMAs of its missing slices, not their loads.
   // Blocks of one adapter read the same A slices; each block starts at a
   // different slice of its range (rotation by block index) so that they do
   // not all hit the same lines at once.
   Slice q[kShrinkDepth];
-  for (; k0 < kc_end; k0 += kShrinkSlices * kSliceK, k1 = min(k0 + kShrinkSlices * kSliceK, kc_end)) {
+  for (; k0 < kc_end; k0 += NS * kSliceK, k1 = min(k0 + NS * kSliceK, kc_end)) {
     const int n_sl = (k1 - k0 + kSliceK - 1) / kSliceK;
     const int rot = b % n_sl;
     auto slice_k = [&](int i) { return k0 + (i + rot < n_sl ? i + rot : i + rot - n_sl) * kSliceK; };
 #pragma unroll
     for (int i = 0; i < kShrinkDepth; ++i) load_slice(q[i], slice_k(i % n_sl));
 #pragma unroll
-    for (int i = 0; i < kShrinkSlices; ++i)
-      run_slice(q[i % kShrinkDepth], i & 1, slice_k(i % n_sl), i < n_sl, i + kShrinkDepth < kShrinkSlices,
+    for (int i = 0; i < NS; ++i)
+      run_slice(q[i % kShrinkDepth], i & 1, slice_k(i % n_sl), i < n_sl, i + kShrinkDepth < NS,
                 slice_k((i + kShrinkDepth) % n_sl));
   }
   trace_stamp(a, 2);
@@ -1512,7 +1513,7 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
   trace_stamp(a, 4);
 }
 
-template <typename T>
+template <typename T, int NS>
 hipError_t launch_shrink_t(const ApplyArgs& a0, hipStream_t stream) {
   const int per_group = a0.rank == 0 ? 1 : std::min(a0.w.n_a, kMaxRank / a0.rank);
   const int per_block = a0.n_chunks * ((a0.w.n_a + per_group - 1) / per_group);
@@ -1522,7 +1523,7 @@ hipError_t launch_shrink_t(const ApplyArgs& a0, hipStream_t stream) {
   ApplyArgs a = a0;
   if (a.trace != nullptr && n * kTraceWords > a.trace_words) a.trace = nullptr;
   const auto run = [&](auto mt, auto mixed) {
-    shrink_kernel<T, decltype(mt)::value, decltype(mixed)::value><<<grid, kThreads, 0, stream>>>(
+    shrink_kernel<T, decltype(mt)::value, decltype(mixed)::value, NS><<<grid, kThreads, 0, stream>>>(
         a.plan.header, a.plan.blocks, a.plan.bperm, a.n_chunks, per_block, per_group, a);
   };
   if (a.rank == 0) {  // mixed ranks: each block's adapter decides, up to kMaxRank
@@ -2064,7 +2065,11 @@ hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, hipStream_t stream)
   if (a.n_chunks < 1 || a.w.n_a < 1 || a.w.n_a > kMaxSlices || a.n_chunks * a.hs > kMaxChunks * kMaxRank ||
       (a.w.n_a > 1 && (a.w.mode != kStacked || a.rank == 0)))
     return hipErrorInvalidValue;
-  return dtype_bf16 ? launch_shrink_t<__bf16>(a, stream) : launch_shrink_t<_Float16>(a, stream);
+  if (a.dc <= kShrinkSlices / 2 * kSliceK)
+    return dtype_bf16 ? launch_shrink_t<__bf16, kShrinkSlices / 2>(a, stream)
+                      : launch_shrink_t<_Float16, kShrinkSlices / 2>(a, stream);
+  return dtype_bf16 ? launch_shrink_t<__bf16, kShrinkSlices>(a, stream)
+                    : launch_shrink_t<_Float16, kShrinkSlices>(a, stream);
 }
 hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
   if (a.srows != kShrinkRowsFused || a.n_ochunks != a.w.n_a || a.n_sub != 1 || a.n_chunks < 1 ||

@@ -164,9 +164,18 @@ inline void shrink_small_split(int d, int rank, ApplyArgs* a) {
 
 // d-ranges of a shrink() launch: kShrinkSlices x 128 columns each (a multiple
 // of that where more ranges than kMaxChunks, or more partials than
-// kMaxChunks x kMaxRank per token, would be needed).
-inline void shrink_range_split(int d, ApplyArgs* a) {
-  const int group = kShrinkSlices * 128;
+// kMaxChunks x kMaxRank per token, would be needed).  Half of that where the
+// launch leaves compute units idle (up to 1.5 workgroups each) and streams at
+// most 16 MB of X: a workgroup's slices are one compute unit's reads, 0.6 us
+// each, against one more partial to sum.  512 vs 1024 columns, MI355X, us, 16
+// prompts / 64 adapters: d = 4096, rank 16, 1024 tokens 8.9 / 11.4 vs 10.5 / 11.8,
+// rank 64 14.4 / 16.8 vs 15.9 / 18.2, 2048 tokens 15.4 / 18.3 vs 17.0 / 19.8, 4096
+// tokens 19.2 / 23.5 vs 18.5 / 22.0.
+inline void shrink_range_split(int d, int64_t tokens, int n_cu, ApplyArgs* a) {
+  const int64_t per_group = a->rank == 0 ? 1 : std::min(a->w.n_a, kMaxRank / a->rank);
+  const int64_t grid = a->n_slots * ceil_div(a->w.n_a, per_group) * ceil_div(d, kShrinkSlices * 128);
+  const bool half = 2 * grid <= 3 * n_cu && tokens * d <= int64_t{8} << 20;
+  const int group = (half ? kShrinkSlices / 2 : kShrinkSlices) * 128;
   const int64_t most = std::max(1, kMaxChunks * kMaxRank / std::max(a->hs, kMaxRank));
   const int64_t n = std::min<int64_t>(ceil_div(d, group), most);
   a->dc = static_cast<int>(ceil_div(ceil_div(d, n), group) * group);
@@ -1455,7 +1464,7 @@ int shrink_impl(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t r
     WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, a, stream));
   } else {
     if (fresh) WP_HIP(launch_fill_u32(static_cast<uint32_t*>(H), 0u, static_cast<size_t>(T * h_row_stride / 2), stream));
-    shrink_range_split(d_model, &a);
+    shrink_range_split(d_model, e->plan_T, e->n_cu, &a);
     a.part = e->spart;
     a.ptok = e->tok_cap;
     WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, a, stream));
@@ -1566,7 +1575,7 @@ int add_lora_impl(wp_engine* e, const char* who, void* y, const void* x, int32_t
     a.h = e->hbuf;
     a.ldh = a.hs;
     a.n_sub = 1;
-    shrink_range_split(d_model, &a);
+    shrink_range_split(d_model, e->plan_T, e->n_cu, &a);
     a.part = e->spart;
     a.ptok = e->tok_cap;
     ApplyArgs as = a;
@@ -1893,7 +1902,7 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
     if ((rc = check_part(e, who, a)) != WP_OK) return rc;
     WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, a, stream));
   } else {
-    shrink_range_split(d_model, &a);
+    shrink_range_split(d_model, e->plan_T, e->n_cu, &a);
     a.part = e->spart;
     a.ptok = e->tok_cap;
     WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, a, stream));
