@@ -32,8 +32,8 @@
 // workgroup but keeps the cross-workgroup chain to one hop: the partial
 // stores themselves are the publication (no acknowledgement wait, no
 // counter), and the readers validate every word they use.  Data crosses
-// workgroups only through device-scope atomic loads and stores (sc1:
-// coherent across the XCDs' L2s) -- never through __threadfence, whose L2
+// workgroups only through device-scope loads and stores, of up to 16 bytes
+// (sc1: coherent across the XCDs' L2s) -- never through __threadfence, whose L2
 // writeback + invalidate costs ~60-100 ns serialised over the device, nor
 // through accumulation atomics.
 //
@@ -79,7 +79,12 @@ constexpr int kShrinkDepth = 2;
 // kFusedMulti: fused, with several output chunks per expand workgroup.
 // kShrinkOnly: shrink() of decode-sized plans: the fused shrink side, and
 // one workgroup per block that sums the partials into H.
-enum Role : int { kFused = 0, kShrinkOnly = 1, kExpandOnly = 2, kFusedMulti = 3 };
+// kShrinkNew: kShrinkOnly into a new H, which it also clears (a.h_fill).  A
+// kernel of its own: with the clearing in kShrinkOnly's, calls into the
+// caller's H took 45.7 instead of 43.5 us (a captured 512-slot grid, d = 13824
+// mixed ranks, the call and its expand(); d = 5120: 52.6 instead of 51.8).
+enum Role : int { kFused = 0, kShrinkOnly = 1, kExpandOnly = 2, kFusedMulti = 3, kShrinkNew = 4 };
+constexpr bool shrink_alone(int role) { return role == kShrinkOnly || role == kShrinkNew; }
 
 
 // ---------------------------------------------------------------- shrink ----
@@ -897,6 +902,12 @@ template <typename T>
 __device__ __forceinline__ void zero_h_unrouted(const ApplyArgs& a, int z) {
   const int lane = threadIdx.x & 63;
   const int word = z * kWaves + (threadIdx.x >> 6);
+  // Blocks past the grid's slots (reported by the last slot) leave zero rows.
+  if (z == 0) {
+    const int n_blocks = static_cast<int>(a.plan.header[kHdrNumFine]);
+    for (int q = a.n_slots; q < n_blocks; ++q)
+      zero_h_rows<T>(a, a.plan.bperm + static_cast<int64_t>(q) * kBlockTokens, a.plan.blocks[q].count, 0);
+  }
   const int plan_T = static_cast<int>(a.plan.header[kHdrT]);
   const uint64_t mask =
       word * 64 < plan_T ? reinterpret_cast<const uint64_t*>(a.plan.header + kHdrMask)[word] : 0ull;
@@ -910,17 +921,17 @@ __device__ __forceinline__ void zero_h_unrouted(const ApplyArgs& a, int z) {
   }
 }
 
-// shrink() of decode-sized plans (role kShrinkOnly): block b's one reader of
+// shrink() of decode-sized plans (kShrinkOnly, NEW: kShrinkNew): block b's one reader of
 // A slice sa sums its partials into H[token] = rn(alpha * sum_c part[c]) and,
 // once every thread has read its words, restores kPartialEmpty over them.
-template <typename T>
+template <typename T, bool NEW>
 __device__ __forceinline__ void reduce_to_h(const ApplyArgs& a, int b, int sa, const Block& blk, int* s_flag,
                                             PreEntry pre = PreEntry{}) {
   const Resolved<T> res = resolve_a<T>(a, blk, sa, pre);
   // Rank rows the shrink side wrote (none if it could not resolve the adapter).
   const int wrote = res.ptr != nullptr ? res.rank : 0;
   const int32_t* toks = a.plan.bperm + static_cast<int64_t>(b) * kBlockTokens;
-  if (a.h_fill > wrote) zero_h_rows<T>(a, toks, blk.count, wrote);
+  if constexpr (NEW) zero_h_rows<T>(a, toks, blk.count, wrote);
   if (wrote <= 0) return;
   const int col = sa * a.hs1;
   if (blk.count * wrote * a.n_chunks > 2048) wait_partials<false>(a, blk, wrote, s_flag, 1u, col);
@@ -969,7 +980,7 @@ constexpr int waves_per_simd() {
   constexpr bool wide = RANK == 0 || RANK == 64;
   if (ROLE == kFused) return wide ? 5 : 7;
   if (ROLE == kFusedMulti) return 4;
-  if (ROLE == kShrinkOnly) return 5;
+  if (shrink_alone(ROLE)) return 5;
   if (TILES == 1) return wide ? 5 : 8;
   return wide ? 3 : 5;
 }
@@ -1028,10 +1039,10 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   // shrink() with a.red_first: the block reducers (one per A slice) are
   // workgroups 0..n_red-1, resident from the start, and the shrink workgroups
   // follow.
-  const bool red_first = ROLE == kShrinkOnly && a.red_first != 0;
+  const bool red_first = shrink_alone(ROLE) && a.red_first != 0;
   const int n_red = PA ? a.n_slots * per_block : a.n_slots;
-  if constexpr (ROLE == kShrinkOnly && !PA) {
-    // Behind both roles: a new H's rows that no block holds.
+  if constexpr (ROLE == kShrinkNew) {
+    // Behind both roles: a new H's rows that no block of the grid holds.
     if (wg >= n_red + n_shrink) {
       touch_kernel_args_wait(ka_touch);
       zero_h_unrouted<T>(a, wg - n_red - n_shrink);
@@ -1070,7 +1081,7 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   // entry's registers a wave per SIMD at ranks 8-32 (cfg2 step 1217 -> 1227
   // us, cfg5's 88 calls 697 -> 736 us, measured on MI355X).
   PreEntry pre;
-  if constexpr (ROLE == kShrinkOnly || ROLE == kExpandOnly || RANK == 0) {
+  if constexpr (shrink_alone(ROLE) || ROLE == kExpandOnly || RANK == 0) {
     if (a.w.mode == kTable && a.w.a_base[0] != nullptr) {
       pre.en = load_entry(static_cast<const Entry*>(a.w.a_base[0]) + b);
       pre.ok = header[kHdrTableVer] == header[kHdrPlanVer];
@@ -1081,18 +1092,14 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   if (b == a.n_slots - 1 && part == 0 && threadIdx.x == 0 && n_blocks > a.n_slots)
     flag_error(a.plan.header, kErrCapacity);
   if constexpr (!PA || RANK == 0) touch_kernel_args_wait(ka_touch);
-  if constexpr (ROLE == kShrinkOnly && !PA) {
-    // A new H: blocks that are skipped (the partials are poisoned, or the plan
-    // has more blocks than the grid) leave zero rows.
-    if (a.h_fill > 0 && !shrink_role) {
-      if (poison != 0u && b < n_blocks && blk.count > 0)
+  if ((b >= n_blocks) | (blk.count <= 0) | (tok0 < -1) | (poison != 0u)) {
+    if constexpr (ROLE == kShrinkNew) {
+      // Blocks skipped because the partials are poisoned leave zero rows.
+      if (!shrink_role && b < n_blocks && blk.count > 0)
         zero_h_rows<T>(a, bperm + static_cast<int64_t>(b) * kBlockTokens, blk.count, 0);
-      if (b == a.n_slots - 1)
-        for (int q = a.n_slots; q < n_blocks; ++q)
-          zero_h_rows<T>(a, bperm + static_cast<int64_t>(q) * kBlockTokens, blocks[q].count, 0);
     }
+    return;
   }
-  if ((b >= n_blocks) | (blk.count <= 0) | (tok0 < -1) | (poison != 0u)) return;
   const int32_t t0 = row < blk.count ? tok0 : -1;
   trace_stamp(a, 1);
   trace_tag(a, (shrink_role ? 1u : 2u) | (static_cast<uint64_t>(b) << 8));
@@ -1107,15 +1114,15 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
     const Resolved<T> res = resolve_a<T, PA>(a, blk, sa, pre);
     // Each slice's first workgroup reports its resolution error.
     if (res.err != 0 && k == 0 && threadIdx.x == 0) flag_error(a.plan.header, res.err);
-    if constexpr (ROLE == kFusedMulti || ROLE == kShrinkOnly) {
+    if constexpr (ROLE == kFusedMulti || shrink_alone(ROLE)) {
       shrink_body<T, kShrinkRowsFused / 16>(a, b, c, sa, rg * kShrinkRowsFused, blk, t0, res, s_red, smem.stg());
     } else {
       shrink_body<T, 1>(a, b, c, sa, rg * kShrinkRows, blk, t0, res, s_red, smem.stg());
     }
     return;
   }
-  if constexpr (ROLE == kShrinkOnly) {
-    reduce_to_h<T>(a, b, PA ? part : 0, blk, &s_flag, pre);
+  if constexpr (shrink_alone(ROLE)) {
+    reduce_to_h<T, ROLE == kShrinkNew>(a, b, PA ? part : 0, blk, &s_flag, pre);
   } else if constexpr (RANK != 0) {
     expand_body<T, RANK, ROLE, TILES, PA>(a, b, part, blk, t0, s_h, smem.stage(), &s_flag, pre);
   } else if constexpr (PA) {
@@ -1546,7 +1553,7 @@ void launch_kernel(const ApplyArgs& a, dim3 grid, int32_t per_shrink, int32_t n_
   // One A per slice not in expand() (its H is the caller's); a separate
   // instantiation, so the shared-A kernels keep their constant indexing and
   // single-probe gate.
-  if constexpr (ROLE != kExpandOnly) {
+  if constexpr (ROLE != kExpandOnly && ROLE != kShrinkNew) {
     if (a.w.n_a > 1) {
       apply_kernel<T, RANK, ROLE, TILES, true><<<grid, kThreads, 0, stream>>>(
           a.plan.header, a.plan.blocks, a.plan.bperm, per_shrink, n_shrink, per_block, a);
@@ -1562,7 +1569,7 @@ hipError_t launch_rank(const ApplyArgs& a, hipStream_t stream) {
   const int64_t S = ROLE == kExpandOnly ? 0 : static_cast<int64_t>(a.n_slots) * a.n_chunks * a.n_rgroups * a.w.n_a;
   const int64_t E = static_cast<int64_t>(a.n_slots) *
                     ((a.n_ochunks + a.n_sub - 1) / a.n_sub);
-  const int64_t Z = ROLE == kShrinkOnly && a.h_fill > 0 ? (a.h_rows + kThreads - 1) / kThreads : 0;
+  const int64_t Z = ROLE == kShrinkNew ? (a.h_rows + kThreads - 1) / kThreads : 0;
   const int64_t n = S + E + Z;
   if (n <= 0) return hipSuccess;
   const dim3 grid(static_cast<unsigned>(n));
@@ -1575,7 +1582,7 @@ hipError_t launch_rank(const ApplyArgs& a, hipStream_t stream) {
     at.trace = nullptr;
   }
   const ApplyArgs& a2 = (a.trace != nullptr && n * kTraceWords > a.trace_words) ? at : a;
-  if constexpr (ROLE == kShrinkOnly) {
+  if constexpr (shrink_alone(ROLE)) {
     // Its shrink side takes the rank from each block's adapter.
     launch_kernel<T, 0, ROLE, TILES>(a2, grid, per_shrink, ns, per_block, stream);
   } else {
@@ -1595,7 +1602,7 @@ hipError_t launch_rank(const ApplyArgs& a, hipStream_t stream) {
 
 template <int ROLE>
 hipError_t launch_role(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
-  if constexpr (ROLE != kFused && ROLE != kFusedMulti) {
+  if constexpr (ROLE != kFused && ROLE != kFusedMulti && ROLE != kShrinkNew) {
     if (a.tiles > 1)
       return dtype_bf16 ? launch_rank<__bf16, ROLE, kTilesInFlight>(a, stream)
                         : launch_rank<_Float16, ROLE, kTilesInFlight>(a, stream);
@@ -2077,7 +2084,7 @@ hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t s
       a.n_chunks * a.hs > kMaxChunks * kMaxRank || (a.w.n_a > 1 && (a.w.mode != kStacked || a.rank == 0)) ||
       (a.h_fill > 0 && (a.w.n_a > 1 || a.h_f32 != 0 || a.h_fill % 8 != 0 || a.ldh % 8 != 0 || a.h_rows < 1)))
     return hipErrorInvalidValue;
-  return launch_role<kShrinkOnly>(dtype_bf16, a, stream);
+  return a.h_fill > 0 ? launch_role<kShrinkNew>(dtype_bf16, a, stream) : launch_role<kShrinkOnly>(dtype_bf16, a, stream);
 }
 hipError_t launch_expand(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
   if (a.w.n_a < 1 || a.w.n_a > kMaxSlices) return hipErrorInvalidValue;

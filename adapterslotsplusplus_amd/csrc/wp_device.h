@@ -141,7 +141,8 @@ __device__ __forceinline__ void flag_error(uint32_t* header, uint32_t bits) { at
 // stored; shrink()'s block reducers (role 2) 4 H stored.  Word 7: role (1
 // shrink, 2 expand or reducer) | block << 8.  shrink_kernel
 // (role 3 | block << 8 | d-range << 32): 0 entry, 1 block resolved, 2 slice
-// loop done, 3 partial stored and counted, 4 the last arriver's H stored;
+// loop done, 3 partial stored and counted, 4 H of a
+// token tile stored by the tile's last wave (wave 0's, if it was);
 // word 6: the wave's hardware ids (HW_ID low word, XCC id << 32).
 // linear_kernel: shrink workgroups (role 1) as the fused ones; block reducers
 // (role 4 | block << 8) 0 entry, 1 block resolved, 2 partials there, 3 H

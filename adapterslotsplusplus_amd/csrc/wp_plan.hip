@@ -404,10 +404,11 @@ __device__ __forceinline__ void put_block(Block* blocks, Entry* bentries, int q,
 
 // Measured on MI355X, build_seg_bounds per launch in a graph of 40 (launch
 // included), against a run table sorted by counting or by a bitonic sort
-// (Zipf(1.1) routing over 64 ids, before -> now, us): T=64 8.8 -> 3.9, 256
-// 12.6 -> 4.4, 512 20.1 -> 5.9, 1024 27.0 -> 6.5, 2048 41.7 -> 8.0, 4096
-// 80.5 -> 11.1, 8192 152.7 -> 18.9; 16 contiguous prompts, T=8192 24.2 ->
-// 16.1; ids up to 1e6, T=256 15.2 -> 7.3, T=8192 198.7 -> 41.2.
+// (Zipf(1.1) routing over 64 ids, before -> now, us; past 512 tokens both
+// tables of blocks): T=64 8.8 -> 4.1, 256 12.6 -> 4.5, 512 20.1 -> 6.2, 1024
+// 27.0 -> 7.6, 2048 41.7 -> 8.1, 4096 80.5 -> 11.8, 8192 152.7 -> 20.5; 16
+// contiguous prompts, T=8192 24.2 -> 16.9; ids up to 1e6, T=256 15.2 -> 7.4,
+// T=8192 198.7 -> 46.4.
 template <int NT, int E>
 __global__ __launch_bounds__(NT) void plan_kernel(const void* __restrict__ idx, int idx_is_int64, int T,
                                                   uint32_t* __restrict__ header, Segment* __restrict__ segments,

@@ -35,7 +35,7 @@ constexpr int kBlockTokens = 64;
 // the caches while the blocks run side by side.  Plans over at most
 // kSmallPlanTokens tokens (decode-sized steps) have only these; larger
 // device-built plans have both, and each call takes the table that suits its
-// ranks and sizes (wp_engine.hip fused_pays).
+// ranks and sizes (wp_engine.hip fused_fits).
 constexpr int kFineTokens = 16;
 constexpr int kSmallPlanTokens = 512;
 inline constexpr int plan_block_tokens(int64_t T) { return T <= kSmallPlanTokens ? kFineTokens : kBlockTokens; }
