@@ -505,7 +505,7 @@ def trace_cfg4_shrink(args):
     row("block resolved (entry -> plan and adapter loaded)", dur(0, 1))
     row("slice loop (-> last MFMA)", dur(1, 2))
     row("partial store acknowledged + counter", dur(2, 3))
-    row("last arriver: d-range sum + H store", dur(3, 4, last))
+    row("last wave of a token tile: d-range sum + H store", dur(3, 4, last))
     row("slice loop done, from the first entry", rel(2))
     row("counted, from the first entry", rel(3))
     row("H stored (last arrivers), from the first entry", rel(4, last))
