@@ -639,6 +639,16 @@ int block_bound(const wp_engine* e, int64_t groups, bool fine = false) {
   return static_cast<int>(std::min<int64_t>(T, T / bt + g));
 }
 
+// The bound of a call that ids it cannot resolve may crowd (they sort among
+// the others): what it covers does not depend on the table it runs on.  The
+// tokens of the plan's first B = block_bound(groups) blocks lie in the first
+// sum ceil(count / 16) <= (T + 15 B) / 16 blocks of the 16-token table.
+int cover_bound(const wp_engine* e, int64_t groups, bool fine) {
+  const int64_t B = block_bound(e, groups);
+  if (!fine || e->plan_bt <= kFineTokens) return static_cast<int>(B);
+  return static_cast<int>(std::min<int64_t>(e->plan_T, (e->plan_T + (kFineTokens - 1) * B) / kFineTokens));
+}
+
 // Distinct ids an adapter-store call on a device-built plan can resolve,
 // given `registered` adapters and a table window of `window` ids (the
 // selected layer's: a multi-layer store is not bounded by every layer's
@@ -1445,7 +1455,7 @@ int shrink_impl(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t r
   a.d_model = d_model;
   if ((rc = table_weights(e, stream, &a.w, small)) != WP_OK) return rc;
   a.w.n_slices = 1;
-  a.n_slots = block_bound(e, resolvable_ids(e, stream), small);
+  a.n_slots = cover_bound(e, resolvable_ids(e, stream), small);
   if (small) {
     // Decode-sized plans: many small shrink workgroups and a reducer per
     // block (the fused calls' shrink side), not one workgroup per block and
@@ -1530,7 +1540,7 @@ int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_
   a.w.oc_start[0] = 0;
   a.w.oc_start[1] = static_cast<int32_t>(ceil_div(out_features, cols));
   a.n_ochunks = a.w.oc_start[1];
-  a.n_slots = block_bound(e, resolvable_ids(e, stream), small);
+  a.n_slots = cover_bound(e, resolvable_ids(e, stream), small);
   WP_HIP(launch_expand(dtype == WP_DTYPE_BF16, a, stream));
   return WP_OK;
 }
@@ -1731,7 +1741,7 @@ int wp_shrink_expand(wp_engine* e, const void* X, void* Y, int32_t d_model, int3
   a.w.oc_start[0] = 0;
   a.w.oc_start[1] = static_cast<int32_t>(ceil_div(out_features, cols));
   a.n_ochunks = a.w.oc_start[1];
-  a.n_slots = block_bound(e, resolvable_ids(e, stream), true);
+  a.n_slots = cover_bound(e, resolvable_ids(e, stream), true);
   fused_split(&a, rank, d_model, e->n_cu);
   if ((rc = check_part(e, "shrink_expand", a)) != WP_OK) return rc;
   WP_HIP(launch_fused(dtype == WP_DTYPE_BF16, a, stream));

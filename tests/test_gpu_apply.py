@@ -870,6 +870,44 @@ def test_store_on_both_tables(T, rank):
         assert engine.device_errors() == 0
 
 
+@pytest.mark.parametrize("rank", [0, 16, 64])
+def test_unregistered_ids_leave_registered_tokens_covered(rank):
+    """Unregistered ids sorting before the registered ones: as long as the plan's
+    64-token blocks fit the store calls' bound (T / 64 + registered adapters: 26
+    of 26 here), every registered token is computed, on the 16-token table too
+    (78 blocks, over T / 16 + registered adapters)."""
+    dtype, T, d, o, first, K = torch.bfloat16, 1024, 264, 132, 16, 10
+    announce(f"unregistered ids before registered ones, rank={rank}")
+    engine = WarpPipeEngine()
+    adapters = {}
+    for i in range(first, first + K):
+        r = rank or (8, 16, 32, 64)[i % 4]
+        A, B = randn((r, d), 1400 + i, dtype, 0.05), randn((o, r), 1430 + i, dtype, 0.02)
+        engine.register_adapter(i, A.cuda(), B.cuda(), 0.5, rank=r)
+        adapters[i] = (A, B, 0.5)
+    idx = np.full(T, -1)
+    idx[:39 * (first + K)] = np.repeat(np.arange(first + K), 39)
+    idx = np.random.default_rng(rank).permutation(idx)
+    assert engine.build_seg_bounds(torch.from_numpy(idx.astype(np.int64)).cuda())
+    X, Y0 = randn((T, d), 1460, dtype), randn((T, o), 1461, dtype)
+    H = engine.shrink(X.cuda(), d, rank, T)
+    Y, Y1 = Y0.cuda(), Y0.cuda()
+    engine.expand(H, Y, o, rank)
+    engine.shrink_expand(X.cuda(), Y1, o, rank)
+    torch.cuda.synchronize()
+    segs = so.seg_bounds(np.where(idx < first, -1, idx)).tolist()
+    H_ref = bgmv.shrink(X, segs, adapters, rank or 64, T)
+    Y_ref = bgmv.expand(H_ref, Y0, segs, adapters)
+    slack = torch.zeros(Y0.shape, dtype=torch.float32)
+    for aid, (A, B, alpha) in adapters.items():
+        rows = torch.from_numpy(np.nonzero(idx == aid)[0])
+        slack[rows] += (h_tie_flips(X[rows], A, alpha, dtype) @ B.double().abs().T).float()
+    assert_close(H, H_ref, "H")
+    assert_close(Y, Y_ref, "Y", slack=slack)
+    assert_close(Y1, Y_ref, "shrink_expand", slack=slack)
+    assert engine.device_errors() == 2  # the unregistered ids, and nothing dropped
+
+
 @pytest.mark.parametrize("T", [1, 63, 65, 500, 1025, 2049])
 @pytest.mark.parametrize("rank", [0, 16])
 def test_new_h_is_zero_where_nothing_is_written(T, rank):
