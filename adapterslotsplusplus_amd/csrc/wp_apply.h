@@ -78,7 +78,11 @@ struct ApplyArgs {
   // (h_fill: columns of a row, 0: H is the caller's; h_rows: its rows).
   int32_t h_fill;
   int32_t h_rows;
-  int32_t pad_end;
+  // expand() of the adapter store on the 16-token table of a larger plan: one
+  // more than the plan's own blocks it is bounded by (0: bounded by its slots
+  // only).  Tokens past them are left alone, whatever the slots hold, since
+  // shrink() may have run on that table and then wrote no H for them.
+  int32_t cover;
 };
 
 // Words per workgroup of a traced build's timestamp buffer: stamps 0..6 and

@@ -1067,6 +1067,7 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   // token only after the count had arrived.
   // Only the four-tile expand runs on the plan's coarse table.
   const int n_blocks = static_cast<int>(header[ROLE == kExpandOnly && TILES > 1 ? kHdrNumBlocks : kHdrNumFine]);
+  const uint32_t n_coarse = ROLE == kExpandOnly && TILES == 1 ? header[kHdrNumBlocks] : 0u;
   // Roles that use the partial buffer do nothing while it is poisoned.
   const uint32_t poison = ROLE == kExpandOnly ? 0u : header[kHdrPoison];
   const Block blk = blocks[b];
@@ -1099,6 +1100,13 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
         zero_h_rows<T>(a, bperm + static_cast<int64_t>(b) * kBlockTokens, blk.count, 0);
     }
     return;
+  }
+  if constexpr (ROLE == kExpandOnly && TILES == 1) {
+    if (n_coarse > static_cast<uint32_t>(a.cover) - 1u) {
+      if (wg == 0 && threadIdx.x == 0) flag_error(a.plan.header, kErrCapacity);
+      // Both tables list the tokens in the plan's order.
+      if (blk.first >= a.plan.coarse[a.cover - 1].first) return;
+    }
   }
   const int32_t t0 = row < blk.count ? tok0 : -1;
   trace_stamp(a, 1);

@@ -518,7 +518,7 @@ PlanView plan_view(const wp_engine* e, bool fine = false) {
   const bool second = fine && e->plan_bt > kFineTokens;
   PlanView v;
   v.header = e->header;
-  v.segments = e->segs;
+  v.coarse = e->blocks;
   v.blocks = second ? e->fblocks : e->blocks;
   v.perm = e->perm;
   v.bperm = second ? e->fbperm : e->bperm;
@@ -1419,9 +1419,14 @@ void fused_split(ApplyArgs* a, int rank, int d_model, int n_cu) {
 
 namespace {
 
-// wp_shrink, and (fresh) wp_shrink_new: H's rows are the caller's, or all new.
+// Whose H rows a shrink fills: the caller's (wp_shrink), all new ones
+// (wp_shrink_new), or the engine's, for an expand that follows at once
+// (wp_shrink_expand).  The last runs on the plan's own table only: the small
+// form would leave rows unwritten while the partials are poisoned.
+enum HRows { kCallerRows, kNewRows, kEngineRows };
 int shrink_impl(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t rank, int64_t T, int64_t h_row_stride,
-                int32_t dtype, bool fresh, void* stream_) {
+                int32_t dtype, HRows rows, void* stream_) {
+  const bool fresh = rows == kNewRows;
   if (!e) return fail(WP_ERR_INVALID, "shrink: engine is NULL");
   if (rank != 0 && !rank_ok(rank)) return fail(WP_ERR_INVALID, "dispatch_bgmv_shrink: unsupported rank (only 8/16/32/64)");
   int rc = check_io("shrink", dtype, X, "X");
@@ -1446,7 +1451,7 @@ int shrink_impl(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t r
   }
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  const bool small = small_shrink_fits(e, rank);
+  const bool small = rows != kEngineRows && small_shrink_fits(e, rank);
   ApplyArgs a = base_args(e, rank, small);
   a.x = X;
   a.ldx = d_model;
@@ -1488,16 +1493,22 @@ extern "C" {
 
 int wp_shrink(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t rank, int64_t T, int64_t h_row_stride,
               int32_t dtype, void* stream) {
-  return shrink_impl(e, X, H, d_model, rank, T, h_row_stride, dtype, false, stream);
+  return shrink_impl(e, X, H, d_model, rank, T, h_row_stride, dtype, kCallerRows, stream);
 }
 
 int wp_shrink_new(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t rank, int64_t T, int64_t h_row_stride,
                   int32_t dtype, void* stream) {
-  return shrink_impl(e, X, H, d_model, rank, T, h_row_stride, dtype, true, stream);
+  return shrink_impl(e, X, H, d_model, rank, T, h_row_stride, dtype, kNewRows, stream);
 }
 
-int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_t rank, int64_t T, int64_t h_row_stride,
-              int64_t y_row_stride, int32_t y_col_offset, int32_t dtype, void* stream_) {
+}  // extern "C"
+
+namespace {
+
+// wp_expand; d_model (wp_shrink_expand, else 0): adapters of another input
+// width, whose shrink was skipped, are skipped too.
+int expand_impl(wp_engine* e, const void* H, void* Y, int32_t d_model, int32_t out_features, int32_t rank, int64_t T,
+                int64_t h_row_stride, int64_t y_row_stride, int32_t y_col_offset, int32_t dtype, void* stream_) {
   if (!e) return fail(WP_ERR_INVALID, "expand: engine is NULL");
   if (rank != 0 && !rank_ok(rank)) return fail(WP_ERR_INVALID, "dispatch_bgmv_expand: unsupported rank (only 8/16/32/64)");
   int rc = check_io("expand", dtype, H, "H");
@@ -1532,6 +1543,7 @@ int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_
   a.ldh = h_row_stride;
   a.y = Y;
   a.ldy = y_row_stride;
+  a.d_model = d_model;
   if ((rc = table_weights(e, stream, &a.w, small)) != WP_OK) return rc;
   const int cols = expand_cols_per_workgroup();
   a.w.n_slices = 1;
@@ -1540,9 +1552,20 @@ int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_
   a.w.oc_start[0] = 0;
   a.w.oc_start[1] = static_cast<int32_t>(ceil_div(out_features, cols));
   a.n_ochunks = a.w.oc_start[1];
-  a.n_slots = cover_bound(e, resolvable_ids(e, stream), small);
+  const int64_t ids = resolvable_ids(e, stream);
+  a.n_slots = cover_bound(e, ids, small);
+  a.cover = small && e->plan_bt > kFineTokens ? block_bound(e, ids) + 1 : 0;
   WP_HIP(launch_expand(dtype == WP_DTYPE_BF16, a, stream));
   return WP_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_t rank, int64_t T, int64_t h_row_stride,
+              int64_t y_row_stride, int32_t y_col_offset, int32_t dtype, void* stream) {
+  return expand_impl(e, H, Y, 0, out_features, rank, T, h_row_stride, y_row_stride, y_col_offset, dtype, stream);
 }
 
 }  // extern "C"
@@ -1698,11 +1721,12 @@ int wp_shrink_expand(wp_engine* e, const void* X, void* Y, int32_t d_model, int3
   if (!e) return fail(WP_ERR_INVALID, "shrink_expand: engine is NULL");
   if (e->plan_kind == 0 || !fused_fits(e, rank, 1, ceil_div(out_features, expand_cols_per_workgroup()))) {
     // Large plans: shrink() into the engine's H, then expand() from it (the
-    // same checks and errors as the two calls).
+    // same checks and errors as the two calls).  The expand runs on blocks
+    // whose H this shrink wrote, no others: hbuf holds other calls' rows.
     const int64_t hs = rank == 0 ? kMaxRank : rank;
-    int rc = wp_shrink(e, X, e->hbuf, d_model, rank, T, hs, dtype, stream_);
+    int rc = shrink_impl(e, X, e->hbuf, d_model, rank, T, hs, dtype, kEngineRows, stream_);
     if (rc != WP_OK) return rc;
-    return wp_expand(e, e->hbuf, Y, out_features, rank, T, hs, y_row_stride, y_col_offset, dtype, stream_);
+    return expand_impl(e, e->hbuf, Y, d_model, out_features, rank, T, hs, y_row_stride, y_col_offset, dtype, stream_);
   }
   if (rank != 0 && !rank_ok(rank)) return fail(WP_ERR_INVALID, "shrink_expand: unsupported rank (only 8/16/32/64)");
   int rc = check_io("shrink_expand", dtype, X, "X");
@@ -2181,8 +2205,8 @@ int wp_add_lora_static(void* y, const void* x, const void* idx, int32_t idx_is_i
   char* base = sd->ptr;
   PlanView v;
   v.header = reinterpret_cast<uint32_t*>(base + kSOffHdr);
-  v.segments = reinterpret_cast<const Segment*>(base + kSOffSeg);
   v.blocks = reinterpret_cast<const Block*>(base + kSOffBlk);
+  v.coarse = v.blocks;
   v.perm = reinterpret_cast<const int32_t*>(base + kSOffPerm);
   v.bperm = reinterpret_cast<const int32_t*>(base + kSOffBperm);
   const int bt = plan_block_tokens(T);

@@ -216,7 +216,7 @@ struct Maint {
 
 struct PlanView {
   uint32_t* header;
-  const Segment* segments;
+  const Block* coarse;  // the plan's own table, whichever `blocks` is
   const Block* blocks;
   const int32_t* perm;
   const int32_t* bperm;

@@ -908,6 +908,102 @@ def test_unregistered_ids_leave_registered_tokens_covered(rank):
     assert engine.device_errors() == 2  # the unregistered ids, and nothing dropped
 
 
+def small_store(rank, d, o, ids, seed, dtype=torch.bfloat16):
+    engine = WarpPipeEngine()
+    adapters = {}
+    for n, i in enumerate(ids):
+        r = rank or (8, 64, 32, 16)[n % 4]
+        A, B = randn((r, d), seed + 2 * n, dtype, 0.05), randn((o, r), seed + 2 * n + 1, dtype, 0.02)
+        engine.register_adapter(i, A.cuda(), B.cuda(), 0.5, rank=r)
+        adapters[i] = (A, B, 0.5)
+    return engine, adapters
+
+
+@pytest.mark.parametrize("rank,T,o", [(16, 7000, 132), (32, 3500, 132), (0, 1100, 8452)])
+def test_two_launch_expand_reads_only_the_h_of_its_shrink(rank, T, o):
+    """Two-launch forms whose halves run on different tables, with far more
+    unregistered ids before the registered ones than either grid has slots for:
+    every row of Y is the result or left alone, after calls that left other
+    values in the engine's H, and with NaN in the caller's."""
+    dtype, d = torch.bfloat16, 264
+    announce(f"two-launch halves rank={rank} T={T} o={o}")
+    engine, adapters = small_store(rank, d, o, [5000, 5001], 1500)
+    X, Y0 = randn((T, d), 1510, dtype), randn((T, o), 1511, dtype)
+    rng = np.random.default_rng(T)
+    assert engine.build_seg_bounds(torch.from_numpy(rng.integers(5000, 5002, size=T)).cuda())
+    engine.shrink_expand(torch.full((T, d), 3.0, dtype=dtype).cuda(), Y0.cuda(), o, rank)
+    assert engine.device_errors() == 0
+    idx = rng.integers(5000, 5002, size=T)
+    idx[rng.permutation(T)[:200]] = np.arange(200)
+    assert engine.build_seg_bounds(torch.from_numpy(idx).cuda())
+    Y, Y1 = Y0.cuda(), Y0.cuda()
+    engine.shrink_expand(X.cuda(), Y, o, rank)
+    H = torch.full((T, rank or 64), float("nan"), dtype=dtype).cuda()
+    engine.shrink(X.cuda(), d, rank, T, out=H)
+    engine.expand(H, Y1, o, rank)
+    torch.cuda.synchronize()
+    segs = so.seg_bounds(np.where(idx < 5000, -1, idx)).tolist()
+    Y_ref = bgmv.expand(bgmv.shrink(X, segs, adapters, rank or 64, T), Y0, segs, adapters)
+    slack = torch.zeros(Y0.shape, dtype=torch.float32)
+    for aid, (A, B, alpha) in adapters.items():
+        rows = torch.from_numpy(np.nonzero(idx == aid)[0])
+        slack[rows] += (h_tie_flips(X[rows], A, alpha, dtype) @ B.double().abs().T).float()
+    for what, got in (("shrink_expand", Y), ("shrink(out=) + expand", Y1)):
+        wrote = (got.cpu() != Y0).any(1)
+        assert not wrote[torch.from_numpy(idx < 5000)].any(), what
+        assert_close(got.cpu()[wrote], Y_ref[wrote], what, slack=slack[wrote])
+    assert engine.device_errors() == 2 | 16
+
+
+def test_two_launch_shrink_expand_does_not_depend_on_the_partials():
+    """Mixed ranks to many columns at 1100 tokens (two launches): a give-up, or
+    partials left poisoned by another call's, changes nothing; no launch of the
+    call uses them."""
+    dtype, d, o, T = torch.bfloat16, 264, 8452, 1100
+    announce("two-launch shrink_expand beside poisoned partials")
+    engine, adapters = small_store(0, d, o, [0, 1, 2], 1520)
+    X, Y0 = randn((T, d), 1530, dtype), randn((T, o), 1531, dtype)
+    idx = np.random.default_rng(T).integers(-1, 3, size=T)
+    idx_d = torch.from_numpy(idx).cuda()
+    assert engine.build_seg_bounds(idx_d)
+    engine.shrink_expand(torch.full((T, d), 3.0, dtype=dtype).cuda(), Y0.cuda(), o, 0)
+    segs = so.seg_bounds(idx).tolist()
+    Y_ref = bgmv.expand(bgmv.shrink(X, segs, adapters, 64, T), Y0, segs, adapters)
+    slack = torch.zeros(Y0.shape, dtype=torch.float32)
+    for aid, (A, B, alpha) in adapters.items():
+        rows = torch.from_numpy(np.nonzero(idx == aid)[0])
+        slack[rows] += (h_tie_flips(X[rows], A, alpha, dtype) @ B.double().abs().T).float()
+    engine.set_spin_limit(0)
+    for _ in range(2):
+        Y = Y0.cuda()
+        engine.shrink_expand(X.cuda(), Y, o, 0)
+        torch.cuda.synchronize()
+        assert_close(Y, Y_ref, "shrink_expand", slack=slack)
+        engine.shrink(X.cuda(), d, 0, T)  # gives up where a word is not there at once
+    engine.set_spin_limit(None)
+    torch.cuda.synchronize()
+    engine.device_errors()
+
+
+@pytest.mark.parametrize("rank,T", [(16, 7000), (64, 1600), (16, 1000)])
+def test_shrink_expand_skips_adapters_of_another_input_width(rank, T):
+    """Adapters registered for another d_model than the call's: skipped by both
+    halves, Y left as it was and the shape bit set."""
+    dtype, d, o = torch.bfloat16, 264, 132
+    announce(f"shrink_expand, other input width, rank={rank} T={T}")
+    engine, _ = small_store(rank, d, o, [0, 1], 1540)
+    idx = torch.from_numpy(np.random.default_rng(T).integers(0, 2, size=T)).cuda()
+    assert engine.build_seg_bounds(idx)
+    Y0 = randn((T, o), 1550, dtype).cuda()
+    engine.shrink_expand(randn((T, d), 1551, dtype).cuda(), Y0.clone(), o, rank)
+    assert engine.device_errors() == 0
+    Y = Y0.clone()
+    engine.shrink_expand(randn((T, d + 8), 1552, dtype).cuda(), Y, o, rank)
+    torch.cuda.synchronize()
+    assert torch.equal(Y, Y0)
+    assert engine.device_errors() == 4
+
+
 @pytest.mark.parametrize("T", [1, 63, 65, 500, 1025, 2049])
 @pytest.mark.parametrize("rank", [0, 16])
 def test_new_h_is_zero_where_nothing_is_written(T, rank):
