@@ -2006,7 +2006,10 @@ int wp_lora_expand(wp_engine* e, void* y, int64_t y_row_stride, const void* h, i
   ExpandExt x{};
   ApplyArgs a{};
   {
-    a = stacked_base(e, rank, num_loras, 1.0f, fine_expand_fits(e, rank));
+    const bool fine = fine_expand_fits(e, rank);
+    a = stacked_base(e, rank, num_loras, 1.0f, fine);
+    // Ids past the weights sort last; overwriting clears their rows too.
+    if (!add_inputs) a.n_slots = cover_bound(e, num_loras, fine);
     a.y = y;
     a.ldy = y_row_stride;
     a.w.n_a = n_slices;  // slice s reads its own H

@@ -383,6 +383,27 @@ def test_lora_expand_h_rows_and_modes(T, rows, rank, add_inputs):
     assert eng.device_errors() == 1
 
 
+def test_lora_expand_overwrite_clears_rows_of_ids_past_the_weights():
+    """Overwriting at 686 tokens: 14 ids of 49 tokens, 9 of them past the weights,
+    fill the 64-token blocks' bound (14 of 15) but 56 of the 16-token table's
+    blocks; every row is the product or cleared, and nothing is dropped."""
+    dtype, L, T, rank, outs = torch.bfloat16, 5, 686, 8, (260, 4)
+    announce("lora_expand overwriting rows of ids past the weights")
+    eng = WarpPipeEngine(WarpPipeConfig(max_tokens=1024))
+    ids = torch.from_numpy(np.random.default_rng(0).permutation(np.repeat(np.arange(14), 49)))
+    _, wbs, _ = weights(L, rank, 64, outs, dtype, 720)
+    h = randn((2, T, rank), 721, torch.float32)
+    y0 = randn((T, sum(outs)), 722, dtype)
+    assert eng.build_seg_bounds(ids.cuda())
+    y = y0.cuda()
+    assert eng.lora_expand(y, h.cuda(), wbs, outs, 0, False)
+    torch.cuda.synchronize()
+    ref = v1_ops.lora_expand(y0, h, cpu(wbs), outs, torch.where(ids < L, ids, -1), 0, False)
+    ref[ids >= L] = 0
+    assert_close(y, ref, "overwriting")
+    assert eng.device_errors() == 1
+
+
 @pytest.mark.parametrize("T", [5, 130, 512])
 @pytest.mark.parametrize("rank,n,d", [(8, 2, 136), (32, 3, 4096), (64, 2, 10240), (64, 4, 6152)])
 def test_lora_shrink_slices_one_launch(T, rank, n, d):
