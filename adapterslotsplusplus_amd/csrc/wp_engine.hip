@@ -1910,6 +1910,19 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
   if (d_model <= 0 || d_model % 8 != 0) return fail(WP_ERR_INVALID, "%s: d_model must be a positive multiple of 8", who);
   if (num_loras <= 0) return fail(WP_ERR_INVALID, "%s: num_loras must be positive", who);
   if ((rc = check_plan_for(e, who, T)) != WP_OK) return rc;
+  // Slices that share words of the output add to them in turn, a launch each:
+  // within one launch they would race.  Apart are slices whose rows lie side
+  // by side in each row, or one slice behind the other.
+  const bool apart = n_slices == 1 ||
+                     (out_slice_stride >= rank && out_row_stride >= (n_slices - 1) * out_slice_stride + rank) ||
+                     out_slice_stride >= (T - 1) * out_row_stride + rank;
+  if (!apart) {
+    for (int s = 0; s < n_slices; ++s)
+      if ((rc = wp_lora_shrink(e, out + s * out_slice_stride, 0, out_row_stride, x, 1, wa + s, wa_stride0 + s, num_loras,
+                               scale, rank, d_model, T, dtype, stream_)) != WP_OK)
+        return rc;
+    return WP_OK;
+  }
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   const bool small = e->plan_bt <= kFineTokens;

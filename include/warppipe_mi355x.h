@@ -314,7 +314,9 @@ int wp_add_lora_nslice(wp_engine* e, void* y, const void* x, int32_t n_slices, c
  * fp32, unrounded (V1's lora_shrink buffer), for every token t of the table
  * and slice s; slice s of out starts out_slice_stride floats after slice 0,
  * rows out_row_stride floats apart (both multiples of 4; out 16-byte
- * aligned).  WP_NOT_HANDLED for a rank without kernels. */
+ * aligned).  One launch; slices that share words (a slice stride under rank, or
+ * rows of one slice reaching into another) take one each, in order.
+ * WP_NOT_HANDLED for a rank without kernels. */
 int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t out_row_stride, const void* x,
                    int32_t n_slices, const void* const* wa, const int64_t* wa_stride0, int32_t num_loras, float scale,
                    int32_t rank, int32_t d_model, int64_t T, int32_t dtype, void* stream);

@@ -429,3 +429,29 @@ def test_lora_shrink_slices_one_launch(T, rank, n, d):
         ref = v1_ops.lora_shrink(ref, x, cpu(was), 0.5, ids)
     assert_close(h, ref, "lora_shrink slices", rtol=1e-4, atol=1e-4)
     assert eng.device_errors() == 0
+
+
+@pytest.mark.parametrize("T", [48, 700])
+@pytest.mark.parametrize("stride", ["one", "partial", "rows", "interleaved"])
+def test_lora_shrink_slices_that_share_words_add_up(T, stride):
+    """Slices of one buffer that overlap (an expanded view, a stride under the
+    rank, rows of one slice inside the next) add to it in turn, like separate
+    calls; slices side by side in a row do not overlap and share a launch."""
+    dtype, L, rank, n, d = torch.bfloat16, 5, 16, 3, 136
+    announce(f"lora_shrink overlapping slices {stride} T={T}")
+    ids = torch.from_numpy(np.random.default_rng(T).integers(-1, L, size=T).astype(np.int64))
+    was, _, _ = weights(L, rank, d, (16,) * n, dtype, 940)
+    x = randn((T, d), 941, dtype)
+    ss, row = {"one": (0, 20), "partial": (4, 20), "rows": (20 * (T // 2), 20), "interleaved": (16, 52)}[stride]
+    buf = randn((2 * T + 8, 52), 942, torch.float32).flatten()
+    ref = buf.clone()
+    for s in range(n):
+        view = ref.as_strided((T, rank), (row, 1), s * ss)
+        view.copy_(v1_ops.lora_shrink(view.clone().unsqueeze(0), x, cpu(was[s:s + 1]), 0.5, ids)[0])
+    eng = WarpPipeEngine(WarpPipeConfig(max_tokens=1024))
+    assert eng.build_seg_bounds(ids.cuda())
+    out = buf.cuda()
+    assert eng.lora_shrink(out.as_strided((n, T, rank), (ss, row, 1)), x.cuda(), was, 0.5)
+    torch.cuda.synchronize()
+    assert_close(out, ref, "overlapping slices", rtol=1e-4, atol=1e-4)
+    assert eng.device_errors() == 0
