@@ -540,7 +540,7 @@ class WarpPipeEngine:
         for o in output_slices:
             offs.append(acc)
             acc += int(o)
-        return self.add_lora_slices(y, x, list(lora_a_stacked), lora_b_stacked, scale, offs,
+        return self.add_lora_slices(y, x, list(lora_a_stacked), list(lora_b_stacked), scale, offs,
                                     [int(o) for o in output_slices])
 
     # ------------------------------------------------- vLLM V1 LoRA ops --
