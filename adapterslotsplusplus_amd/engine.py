@@ -59,7 +59,8 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or _current_r
 
 # Argument arrays of 64-bit (pointers, strides) and 32-bit values as bytes
 # objects, which ctypes passes as they are: a third of a ctypes array's cost.
-# 32-bit values wrap, as a ctypes array's do; the library checks them.
+# 32-bit values wrap, as a ctypes array's do; the library checks them.  It reads
+# one value per slice, so the caller sees to it that there are as many.
 def _i64s(v) -> bytes:
     return struct.pack(f"{len(v)}q", *v)
 
@@ -516,7 +517,13 @@ class WarpPipeEngine:
         wb_ptrs = _i64s([w.data_ptr() for w in wb_t_alls])
         wb_strides = _i64s([w.stride(0) for w in wb_t_alls])
         o_arr = _i32s(outs)
-        off_arr = _i32s([int(v) for v in y_offsets])
+        offs = [int(v) for v in y_offsets]
+        if len(offs) != n:
+            # One per slice; those not given are 0.
+            if len(offs) > n:
+                raise IndexError(f"add_lora_packed: {len(offs)} offsets for {n} slices")
+            offs += [0] * (n - len(offs))
+        off_arr = _i32s(offs)
         stream = _raw_stream(dev)
         if per_slice_a:
             rc = self._lib.wp_add_lora_nslice(self._handle, y2.data_ptr(), x2.data_ptr(), n,

@@ -43,3 +43,18 @@ def test_nslice_takes_any_iterable_of_weights(eng, wrap):
     name, args = eng._lib.calls[-1]
     assert name == "wp_add_lora_nslice" and args[3] == 3
     assert struct.unpack("3q", args[6]) == tuple(w.data_ptr() for w in wbs)
+
+
+def test_offsets_reach_the_library_one_per_slice(eng):
+    """The library reads one offset per slice: those not given are 0, and more
+    than the slices are refused."""
+    y, x, was, wbs = slices(3)
+    for given in ([], [4], [0, 12], [0, 12, 24]):
+        assert eng.add_lora_slices(y, x, was[0], wbs, 0.5, given)
+        name, args = eng._lib.calls[-1]
+        assert name == "wp_add_lora" and args[6] == 3
+        assert struct.unpack("3i", args[10]) == tuple((given + [0, 0, 0])[:3])
+    with pytest.raises(IndexError):
+        eng.add_lora_slices(y, x, was[0], wbs, 0.5, [0, 12, 24, 36])
+    with pytest.raises(IndexError):
+        eng.add_lora_packed_nslice(y, x, was, wbs, 0.5, [12, 12, 12, 12])
