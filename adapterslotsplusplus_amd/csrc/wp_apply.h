@@ -174,7 +174,8 @@ hipError_t launch_fused(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
 // shrink(): one workgroup per (block, group of A slices of at most 64 rows,
 // d-range); the block's last workgroup to finish sums the d-ranges into
 // H[token], slice s at element s * a.ldy of an H row.
-hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
+// empty_slots: slots of the grid that a plan of whole blocks would leave empty.
+hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, int64_t empty_slots, hipStream_t stream);
 // shrink() of decode-sized plans: the fused kernel's shrink workgroups
 // (kShrinkRowsFused rows x d-range) of every A slice and one reducer per block
 // and slice writing its H at element s * a.ldy of a row; with a.h_fill (one

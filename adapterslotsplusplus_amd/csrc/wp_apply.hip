@@ -1275,6 +1275,7 @@ constexpr int kTileCounter = kGroupCounter / (kBlockTokens / 16);
 // NS: slices per pass over a d-range (kShrinkSlices, or half of it where the
 // d-ranges are that short).
 // The leading scalar arguments arrive in SGPRs at wave launch, as apply_kernel's do.
+// per_group: A slices of a group, negative where the grid may hold many slots past the plan's blocks.
 template <typename T, int MT, bool kMixed, int NS>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kShrinkWavesPerSimd)))
 void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, const int32_t* __restrict__ bperm,
@@ -1282,6 +1283,12 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
   using V8 = typename VecOf<T>::v8;
   constexpr int KS = kSliceK / 32;              // K-steps per slice
   constexpr int XL = 16 * kSliceK / (64 * 8);   // a wave's whole-row X loads per slice (4)
+  if (per_group < 0) {
+    // Empty slots leave on the count alone, not once the loads below, which a
+    // real block's first weights wait for, have arrived.
+    if (static_cast<int>(blockIdx.x) / per_block >= static_cast<int>(header[kHdrNumBlocks])) return;
+    per_group = -per_group;
+  }
   const uint32_t ka_touch = touch_kernel_args_issue<static_cast<int>(sizeof(ApplyKernelArgs))>();
   __shared__ T s_a[2][MT * 16 * kSliceStride];
   // Each wave's X tile of the current slice: only that wave reads it, after
@@ -1528,8 +1535,15 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
   trace_stamp(a, 4);
 }
 
+// Empty workgroups from which shrink_kernel tests the block count first (a
+// store call captured with no declared maximum has a slot per token).  MI355X,
+// loads first vs count first, us: d = 4096, rank 16, 4096 tokens and slots 20.0
+// vs 13.2, 6144 28.9 vs 16.9, rank 64, 8192 56.5 vs 28.6; at 8192 empty
+// workgroups and below the same, rank 64 up to 1 us slower.
+constexpr int64_t kLooseWorkgroups = 8192;
+
 template <typename T, int NS>
-hipError_t launch_shrink_t(const ApplyArgs& a0, hipStream_t stream) {
+hipError_t launch_shrink_t(const ApplyArgs& a0, int64_t empty_slots, hipStream_t stream) {
   const int per_group = a0.rank == 0 ? 1 : std::min(a0.w.n_a, kMaxRank / a0.rank);
   const int per_block = a0.n_chunks * ((a0.w.n_a + per_group - 1) / per_group);
   const int64_t n = static_cast<int64_t>(a0.n_slots) * per_block;
@@ -1537,9 +1551,10 @@ hipError_t launch_shrink_t(const ApplyArgs& a0, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(n));
   ApplyArgs a = a0;
   if (a.trace != nullptr && n * kTraceWords > a.trace_words) a.trace = nullptr;
+  const int signed_group = empty_slots * per_block > kLooseWorkgroups ? -per_group : per_group;
   const auto run = [&](auto mt, auto mixed) {
     shrink_kernel<T, decltype(mt)::value, decltype(mixed)::value, NS><<<grid, kThreads, 0, stream>>>(
-        a.plan.header, a.plan.blocks, a.plan.bperm, a.n_chunks, per_block, per_group, a);
+        a.plan.header, a.plan.blocks, a.plan.bperm, a.n_chunks, per_block, signed_group, a);
   };
   if (a.rank == 0) {  // mixed ranks: each block's adapter decides, up to kMaxRank
     run(std::integral_constant<int, kMaxRank / 16>{}, std::true_type{});
@@ -2076,15 +2091,15 @@ hipError_t launch_fused(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) 
     return hipErrorInvalidValue;
   return a.n_sub > 1 ? launch_role<kFusedMulti>(dtype_bf16, a, stream) : launch_role<kFused>(dtype_bf16, a, stream);
 }
-hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
+hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, int64_t empty_slots, hipStream_t stream) {
   if (a.n_chunks < 1 || a.w.n_a < 1 || a.w.n_a > kMaxSlices || a.n_chunks * a.hs > kMaxChunks * kMaxRank ||
       (a.w.n_a > 1 && (a.w.mode != kStacked || a.rank == 0)))
     return hipErrorInvalidValue;
   if (a.dc <= kShrinkSlices / 2 * kSliceK)
-    return dtype_bf16 ? launch_shrink_t<__bf16, kShrinkSlices / 2>(a, stream)
-                      : launch_shrink_t<_Float16, kShrinkSlices / 2>(a, stream);
-  return dtype_bf16 ? launch_shrink_t<__bf16, kShrinkSlices>(a, stream)
-                    : launch_shrink_t<_Float16, kShrinkSlices>(a, stream);
+    return dtype_bf16 ? launch_shrink_t<__bf16, kShrinkSlices / 2>(a, empty_slots, stream)
+                      : launch_shrink_t<_Float16, kShrinkSlices / 2>(a, empty_slots, stream);
+  return dtype_bf16 ? launch_shrink_t<__bf16, kShrinkSlices>(a, empty_slots, stream)
+                    : launch_shrink_t<_Float16, kShrinkSlices>(a, empty_slots, stream);
 }
 hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
   if (a.srows != kShrinkRowsFused || a.n_ochunks != a.w.n_a || a.n_sub != 1 || a.n_chunks < 1 ||

@@ -649,6 +649,11 @@ int cover_bound(const wp_engine* e, int64_t groups, bool fine) {
   return static_cast<int>(std::min<int64_t>(e->plan_T, (e->plan_T + (kFineTokens - 1) * B) / kFineTokens));
 }
 
+// Slots of a call's grid that a plan of whole blocks would leave empty.
+int64_t empty_slots(const wp_engine* e, const ApplyArgs& a) {
+  return e->plan_kind == 1 ? 0 : a.n_slots - e->plan_T / (a.tiles * kFineTokens);
+}
+
 // Distinct ids an adapter-store call on a device-built plan can resolve,
 // given `registered` adapters and a table window of `window` ids (the
 // selected layer's: a multi-layer store is not bounded by every layer's
@@ -1482,7 +1487,7 @@ int shrink_impl(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t r
     shrink_range_split(d_model, e->plan_T, e->n_cu, &a);
     a.part = e->spart;
     a.ptok = e->tok_cap;
-    WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, a, stream));
+    WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, a, empty_slots(e, a), stream));
   }
   return WP_OK;
 }
@@ -1613,7 +1618,7 @@ int add_lora_impl(wp_engine* e, const char* who, void* y, const void* x, int32_t
     a.ptok = e->tok_cap;
     ApplyArgs as = a;
     as.ldy = rank;  // slice s at column s * rank of an H row
-    WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, as, stream));
+    WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, as, empty_slots(e, as), stream));
     // H is by token, so the expand may run on the other table.
     const bool fine = fine_expand_fits(e, rank);
     a.tiles = fine ? 1 : a.tiles;
@@ -1952,7 +1957,7 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
     shrink_range_split(d_model, e->plan_T, e->n_cu, &a);
     a.part = e->spart;
     a.ptok = e->tok_cap;
-    WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, a, stream));
+    WP_HIP(launch_shrink(dtype == WP_DTYPE_BF16, a, empty_slots(e, a), stream));
   }
   return WP_OK;
 }

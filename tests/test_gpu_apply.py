@@ -1004,6 +1004,43 @@ def test_shrink_expand_skips_adapters_of_another_input_width(rank, T):
     assert engine.device_errors() == 4
 
 
+def store_reference(X, Y0, idx, adapters, width):
+    """H, Y of the store calls, and per element of Y the steps that H's rounding
+    ties may take, times |B|."""
+    segs = so.seg_bounds(idx).tolist()
+    H = bgmv.shrink(X, segs, adapters, width, X.shape[0])
+    Y = bgmv.expand(H, Y0, segs, adapters)
+    slack = torch.zeros(Y0.shape, dtype=torch.float32)
+    for aid, (A, B, alpha) in adapters.items():
+        rows = torch.from_numpy(np.nonzero(idx == aid)[0])
+        slack[rows] += (h_tie_flips(X[rows], A, alpha, X.dtype) @ B.double().abs().T).float()
+    return H, Y, slack
+
+
+@pytest.mark.parametrize("rank,T", [(0, 4100), (16, 4100), (64, 2900)])
+def test_large_shrink_with_a_slot_per_token(rank, T):
+    """A declared maximum that bounds nothing: shrink_kernel's grid has a slot per
+    token (over 8192 empty workgroups, which leave on the block count alone);
+    the last real block beside the first empty one, shrink() and both of
+    shrink_expand()'s halves."""
+    dtype, d, o = torch.bfloat16, 2056, 132
+    announce(f"large shrink, a slot per token, rank={rank} T={T}")
+    engine, adapters = small_store(rank, d, o, [0, 1, 2, 3, 4], 1600)
+    engine.set_max_adapters(60000)
+    X, Y0 = randn((T, d), 1610, dtype), randn((T, o), 1611, dtype)
+    idx = np.random.default_rng(T).integers(-1, 5, size=T)
+    assert engine.build_seg_bounds(torch.from_numpy(idx).cuda())
+    H_ref, Y_ref, slack = store_reference(X, Y0, idx, adapters, rank or 64)
+    out = torch.zeros(T, rank or 64, dtype=dtype, device="cuda")
+    Y = Y0.cuda()
+    assert_close(engine.shrink(X.cuda(), d, rank, T), H_ref, "H")
+    assert_close(engine.shrink(X.cuda(), d, rank, T, out=out), H_ref, "H, out=")
+    engine.shrink_expand(X.cuda(), Y, o, rank)
+    torch.cuda.synchronize()
+    assert_close(Y, Y_ref, "Y", slack=slack)
+    assert engine.device_errors() == 0
+
+
 @pytest.mark.parametrize("T", [1, 63, 65, 500, 1025, 2049])
 @pytest.mark.parametrize("rank", [0, 16])
 def test_new_h_is_zero_where_nothing_is_written(T, rank):
