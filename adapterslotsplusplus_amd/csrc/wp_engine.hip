@@ -544,54 +544,6 @@ int check_part(const wp_engine* e, const char* who, const ApplyArgs& a) {
   return WP_OK;
 }
 
-// Which of a plan's two tables a call runs on, past kSmallPlanTokens tokens
-// (below that there is only the 16-token one).  Short blocks spread a call
-// over more workgroups and hide its latency, long ones read an adapter's
-// weights once per 64 tokens: so the line lies at a number of tokens that falls
-// with the rank.  All figures MI355X, us per call, d = 4096 unless given, 16
-// contiguous prompts / Zipf(1.1) tokens over 64 adapters.
-
-// One fused launch on 16-token blocks, or shrink and expand launches.  Rank
-// times tokens up to 98304 (narrow outputs) or 61440 (over 32 output chunks,
-// where the expand's weights are the larger part):
-//   4096 columns, fused vs two launches: rank 8, 8192 tokens 42 / 47 vs 45 / 53;
-//   rank 16, 4096 26 / 29 vs 30 / 35; rank 32, 3072 27 / 31 vs 30 / 34, 4096
-//   33 / 39 vs 33 / 40; rank 64, 1536 25 / 30 vs 27 / 33, 2048 30 / 36 vs 30 / 34.
-//   3 x 4096 columns: rank 16, 2048 34 / 37 vs 38 / 44, 4096 57 / 63 vs 58 / 68;
-//   rank 64, 640 28 / 42 vs 32 / 48, 1024 37 / 50 vs 36 / 51.
-// With one A per slice the fused launch reads X per slice: rank times tokens up
-// to 32768, at most 1536 (4096 + 2 x 1024 columns, rank 8, 1024 tokens 17 / 20 vs
-// 19 / 22, 1536 22 / 25 vs 22 / 25; rank 16, 1024 19 / 23 vs 22 / 25; rank 32,
-// 1024 23 / 29 vs 24 / 35, 1536 30 / 37 vs 28 / 38; rank 64, 512 26 / 41 vs 26 /
-// 44, 640 27 / 45 vs 26 / 47, 1024 36 / 53 vs 32 / 51).
-// Mixed ranks count as 48 or 60: 2048 tokens 29 / 31 vs 31 / 34 (3072 39 / 42 vs
-// 34 / 38), to 13824 columns 1024 33 / 42 vs 39 / 48 (1536 45 / 50 vs 43 / 53).
-bool fused_fits(const wp_engine* e, int rank, int n_a, int64_t n_ochunks) {
-  if (e->plan_bt <= kFineTokens) return true;
-  if (!has_fine(e)) return false;
-  if (n_a > 1) return rank != 0 && e->plan_T <= 1536 && e->plan_T * rank <= 32768;
-  const bool wide = n_ochunks > 2 * kExpandWorkgroups;
-  const int64_t r = rank != 0 ? rank : wide ? 60 : 48;
-  return e->plan_T * r <= (wide ? 61440 : 98304);
-}
-
-// shrink() as many small workgroups and a reducer per 16-token block, or one
-// workgroup per 64-token block and d-range: up to 2048 tokens and rank times
-// tokens 65536 (mixed ranks as 32).  Small vs large, rank 16, 2048 tokens 11 /
-// 14 vs 13 / 15, 3072 14 / 16 vs 14 / 16; rank 64, 1024 14 / 18 vs 17 / 20, 2048
-// 19 / 22 vs 18 / 20; mixed, 2048 18 / 18 vs 19 / 20, 3072 21 / 23 vs 20 / 21.
-bool small_shrink_fits(const wp_engine* e, int rank) {
-  if (e->plan_bt <= kFineTokens) return true;
-  return has_fine(e) && e->plan_T <= 2048 && e->plan_T * (rank != 0 ? rank : 32) <= 65536;
-}
-
-// A small shrink's reducers go first when they take at most half of the
-// resident workgroups: they then poll while the shrink workgroups stream
-// instead of being dispatched after them.
-int reducers_first(const wp_engine* e, const ApplyArgs& a) {
-  return 2 * static_cast<int64_t>(a.n_slots) * a.w.n_a <= static_cast<int64_t>(e->n_cu) * shrink_small_waves_per_simd() ? 1 : 0;
-}
-
 // expand() over 16-token blocks, one tile in flight at eight waves per SIMD, or
 // 64-token blocks, four tiles at three to five.  Ranks up to 32 always: rank 16
 // 1024 tokens 9 / 9 vs 11 / 12, 8192 27 / 32 vs 38 / 38; rank 32, 8192 30 / 37
@@ -673,6 +625,68 @@ int64_t resolvable_ids(const wp_engine* e, hipStream_t stream) {
   const int64_t window =
       e->entry_count > 0 ? e->entry_count : std::max<int64_t>(0, static_cast<int64_t>(e->table_cap) - e->entry_offset);
   return call_ids(e, stream, static_cast<int64_t>(e->adapters.size()), window);
+}
+
+// Which of a plan's two tables a call runs on, past kSmallPlanTokens tokens
+// (below that there is only the 16-token one).  Short blocks spread a call
+// over more workgroups and hide its latency, long ones read an adapter's
+// weights once per 64 tokens: so the line lies at a number of tokens that falls
+// with the rank.  All figures MI355X, us per call, d = 4096 unless given, 16
+// contiguous prompts / Zipf(1.1) tokens over 64 adapters.
+
+// One fused launch on 16-token blocks, or shrink and expand launches.  Rank
+// times tokens up to 98304 (narrow outputs) or 61440 (over 32 output chunks,
+// where the expand's weights are the larger part):
+//   4096 columns, fused vs two launches: rank 8, 8192 tokens 42 / 47 vs 45 / 53;
+//   rank 16, 4096 26 / 29 vs 30 / 35; rank 32, 3072 27 / 31 vs 30 / 34, 4096
+//   33 / 39 vs 33 / 40; rank 64, 1536 25 / 30 vs 27 / 33, 2048 30 / 36 vs 30 / 34.
+//   3 x 4096 columns: rank 16, 2048 34 / 37 vs 38 / 44, 4096 57 / 63 vs 58 / 68;
+//   rank 64, 640 28 / 42 vs 32 / 48, 1024 37 / 50 vs 36 / 51.
+// With one A per slice the fused launch reads X per slice: rank times tokens up
+// to 32768, at most 1536 (4096 + 2 x 1024 columns, rank 8, 1024 tokens 17 / 20 vs
+// 19 / 22, 1536 22 / 25 vs 22 / 25; rank 16, 1024 19 / 23 vs 22 / 25; rank 32,
+// 1024 23 / 29 vs 24 / 35, 1536 30 / 37 vs 28 / 38; rank 64, 512 26 / 41 vs 26 /
+// 44, 640 27 / 45 vs 26 / 47, 1024 36 / 53 vs 32 / 51).
+// Mixed ranks count as 48 or 60: 2048 tokens 29 / 31 vs 31 / 34 (3072 39 / 42 vs
+// 34 / 38), to 13824 columns 1024 33 / 42 vs 39 / 48 (1536 45 / 50 vs 43 / 53).
+// `slots`: the 16-token grid's block slots.  Where its bound is loose (a call
+// captured with nothing declared has a slot per token) most are empty, and the
+// fused launch has more workgroups per slot: mixed ranks at 2048 tokens, 1118
+// slots 42 vs 42, 2048 slots 60 vs 54-57; 1536 tokens and slots 47 vs 46-48.
+// Fixed ranks stay ahead on any grid (rank 16, 2048 slots 31 vs 36; rank 64 45 vs
+// 51 at 1536).
+constexpr int64_t kMixedEmptySlots = 1536;
+bool fused_fits(const wp_engine* e, int rank, int n_a, int64_t n_ochunks, int64_t slots) {
+  if (e->plan_bt <= kFineTokens) return true;
+  if (!has_fine(e) || (rank == 0 && slots - e->plan_T / kFineTokens > kMixedEmptySlots)) return false;
+  if (n_a > 1) return rank != 0 && e->plan_T <= 1536 && e->plan_T * rank <= 32768;
+  const bool wide = n_ochunks > 2 * kExpandWorkgroups;
+  const int64_t r = rank != 0 ? rank : wide ? 60 : 48;
+  return e->plan_T * r <= (wide ? 61440 : 98304);
+}
+
+// A small shrink's reducers (one per block slot and A slice) go first when they
+// take at most half of the resident workgroups: they then poll while the shrink
+// workgroups stream instead of being dispatched after them.
+bool reducers_first(const wp_engine* e, int64_t reducers) {
+  return 2 * reducers <= static_cast<int64_t>(e->n_cu) * shrink_small_waves_per_simd();
+}
+
+// shrink() as many small workgroups and a reducer per 16-token block, or one
+// workgroup per 64-token block and d-range: up to 2048 tokens and rank times
+// tokens 65536 (mixed ranks as 32), the line of a new H (which the large form
+// needs a fill for).  Small vs large, a new H, rank 16, 1024 tokens 7.1 / 8.1 vs
+// 9.7 / 10.8, 2048 8.7 / 10.3 vs 10.2 / 11.6; rank 64, 1024 11.3 / 14.5 vs 13.7 /
+// 18.0, 2048 15.6 / 19.2 vs 15.9 / 19.4; mixed, 1024 11.1 / 11.4 vs 13.3 / 15.7, 2048
+// 14.9 / 15.9 vs 15.2 / 16.5.  Into the caller's H: rank 16, 1024 7.0 / 8.1 vs 7.6 /
+// 8.7, 2048 8.5 / 9.7 vs 7.8 / 9.0; mixed, 1024 11.2 / 11.2 vs 11.2 / 13.0, 2048 14.3
+// / 15.1 vs 12.4 / 13.9.
+// And only on grids of so few slots that the reducers go first: mixed,
+// 1024 tokens, 576 / 832 / 1024 slots 12 / 18 / 21 vs 16 / 16 / 16; rank 64 15 / 22
+// / 25 vs 17; rank 16 8 / 10 / 11 vs 10.
+bool small_shrink_fits(const wp_engine* e, int rank, int64_t slots) {
+  if (e->plan_bt <= kFineTokens) return true;
+  return has_fine(e) && e->plan_T <= 2048 && e->plan_T * (rank != 0 ? rank : 32) <= 65536 && reducers_first(e, slots);
 }
 
 // Registration past the declared maximum (wp_set_max_adapters) is refused:
@@ -1456,7 +1470,8 @@ int shrink_impl(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t r
   }
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  const bool small = rows != kEngineRows && small_shrink_fits(e, rank);
+  const int64_t ids = resolvable_ids(e, stream);
+  const bool small = rows != kEngineRows && small_shrink_fits(e, rank, cover_bound(e, ids, true));
   ApplyArgs a = base_args(e, rank, small);
   a.x = X;
   a.ldx = d_model;
@@ -1465,13 +1480,13 @@ int shrink_impl(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t r
   a.d_model = d_model;
   if ((rc = table_weights(e, stream, &a.w, small)) != WP_OK) return rc;
   a.w.n_slices = 1;
-  a.n_slots = cover_bound(e, resolvable_ids(e, stream), small);
+  a.n_slots = cover_bound(e, ids, small);
   if (small) {
     // Decode-sized plans: many small shrink workgroups and a reducer per
     // block (the fused calls' shrink side), not one workgroup per block and
     // d-range streaming every rank row.
     shrink_small_split(d_model, rank, &a);
-    a.red_first = reducers_first(e, a);
+    a.red_first = reducers_first(e, a.n_slots) ? 1 : 0;
     if ((rc = check_part(e, "shrink", a)) != WP_OK) return rc;
     if (fresh && e->plan_kind == 2 && T > 0 && T < (int64_t{1} << 31)) {
       // Zeroes go out with the H rows: a fill of its own took 5 us of a call's
@@ -1594,7 +1609,7 @@ int add_lora_impl(wp_engine* e, const char* who, void* y, const void* x, int32_t
                 (long long)T);
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  const bool fused = fused_fits(e, rank, n_a, a.n_ochunks);
+  const bool fused = fused_fits(e, rank, n_a, a.n_ochunks, block_bound(e, num_loras, true));
   a.tiles = fused ? 1 : (e->plan_bt + 15) / 16;
   a.ptok = fused_ptok(e);
   a.part = e->part;
@@ -1724,7 +1739,8 @@ int wp_add_lora_nslice(wp_engine* e, void* y, const void* x, int32_t n_slices, c
 int wp_shrink_expand(wp_engine* e, const void* X, void* Y, int32_t d_model, int32_t out_features, int32_t rank,
                      int64_t T, int64_t y_row_stride, int32_t y_col_offset, int32_t dtype, void* stream_) {
   if (!e) return fail(WP_ERR_INVALID, "shrink_expand: engine is NULL");
-  if (e->plan_kind == 0 || !fused_fits(e, rank, 1, ceil_div(out_features, expand_cols_per_workgroup()))) {
+  if (e->plan_kind == 0 || !fused_fits(e, rank, 1, ceil_div(out_features, expand_cols_per_workgroup()),
+                                       cover_bound(e, resolvable_ids(e, static_cast<hipStream_t>(stream_)), true))) {
     // Large plans: shrink() into the engine's H, then expand() from it (the
     // same checks and errors as the two calls).  The expand runs on blocks
     // whose H this shrink wrote, no others: hbuf holds other calls' rows.
@@ -1950,7 +1966,7 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
     // Every slice in one launch: a launch takes 7 us at 48 tokens, its bytes
     // under 1 (a step of four layers, three slices each 125 -> 68 us, MI355X).
     shrink_small_split(d_model, rank, &a);
-    a.red_first = reducers_first(e, a);
+    a.red_first = reducers_first(e, static_cast<int64_t>(a.n_slots) * a.w.n_a) ? 1 : 0;
     if ((rc = check_part(e, who, a)) != WP_OK) return rc;
     WP_HIP(launch_shrink_small(dtype == WP_DTYPE_BF16, a, stream));
   } else {

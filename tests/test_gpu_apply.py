@@ -1041,6 +1041,81 @@ def test_large_shrink_with_a_slot_per_token(rank, T):
     assert engine.device_errors() == 0
 
 
+@pytest.mark.parametrize("rank,T,declared", [(16, 1000, 601), (16, 1000, 602), (0, 1000, 601), (0, 1000, 602),
+                                             (0, 2048, 1607), (0, 2048, 1608)])
+def test_store_forms_by_grid_slots(rank, T, declared):
+    """Both sides of the lines that count a grid's slots: the small shrink up to
+    640 of them (601 declared at 1000 tokens), the mixed-rank fused launch up to
+    1536 empty ones (1607 declared at 2048 tokens)."""
+    dtype, d, o = torch.float16, 264, 132
+    announce(f"store forms by slots rank={rank} T={T} declared={declared}")
+    engine, adapters = small_store(rank, d, o, [0, 1, 2, 3, 4], 1700, dtype)
+    engine.set_max_adapters(declared)
+    X, Y0 = randn((T, d), 1710, dtype), randn((T, o), 1711, dtype)
+    idx = np.random.default_rng(T).integers(-1, 5, size=T)
+    assert engine.build_seg_bounds(torch.from_numpy(idx).cuda())
+    H_ref, Y_ref, slack = store_reference(X, Y0, idx, adapters, rank or 64)
+    out = torch.zeros(T, rank or 64, dtype=dtype, device="cuda")
+    Y, Y1 = Y0.cuda(), Y0.cuda()
+    for _ in range(2):  # the first call leaves the partials empty
+        assert_close(engine.shrink(X.cuda(), d, rank, T), H_ref, "H")
+    assert_close(engine.shrink(X.cuda(), d, rank, T, out=out), H_ref, "H, out=")
+    engine.expand(out, Y, o, rank)
+    engine.shrink_expand(X.cuda(), Y1, o, rank)
+    torch.cuda.synchronize()
+    assert_close(Y, Y_ref, "Y", slack=slack)
+    assert_close(Y1, Y_ref, "shrink_expand", slack=slack)
+    assert engine.device_errors() == 0
+
+
+@pytest.mark.parametrize("rank,T", [(0, 640), (16, 1024), (0, 2048), (16, 2600)])
+def test_captured_store_calls_with_a_slot_per_token(rank, T):
+    """Captured with no declared maximum (a slot per token) and replayed with other
+    routings, one of a block per token: every replay against the oracle, with
+    eager work between them."""
+    dtype, d, o = torch.bfloat16, 1032, 132
+    announce(f"captured store calls, a slot per token, rank={rank} T={T}")
+    ids = list(range(40))
+    engine, adapters = small_store(rank, d, o, ids, 1720)
+    X, Y0 = randn((T, d), 1810, dtype), randn((T, o), 1811, dtype)
+    rng = np.random.default_rng(T)
+    routings = [rng.integers(0, 2, size=T), rng.integers(-1, 40, size=T), np.where(np.arange(T) % 65, -1, rng.integers(0, 40, size=T))]
+    x, y0 = X.cuda(), Y0.cuda()
+    idx_buf, y, y1 = torch.from_numpy(routings[0]).cuda(), y0.clone(), y0.clone()
+    out = torch.zeros(T, rank or 64, dtype=dtype, device="cuda")
+
+    def step():
+        engine.build_seg_bounds(idx_buf)
+        h = engine.shrink(x, d, rank, T)
+        engine.shrink(x, d, rank, T, out=out)
+        engine.expand(out, y, o, rank)
+        engine.shrink_expand(x, y1, o, rank)
+        return h
+
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        step()
+    torch.cuda.current_stream().wait_stream(s)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        h = step()
+    for k in (1, 2, 0, 1):
+        announce(f"replay routing {k}")
+        idx_buf.copy_(torch.from_numpy(routings[k]))
+        y.copy_(y0)
+        y1.copy_(y0)
+        _ = (x.float() * 2).sum()  # eager work between replays
+        g.replay()
+        torch.cuda.synchronize()
+        H_ref, Y_ref, slack = store_reference(X, Y0, routings[k], adapters, rank or 64)
+        assert_close(h, H_ref, f"H routing {k}")
+        assert_close(y, Y_ref, f"Y routing {k}", slack=slack)
+        assert_close(y1, Y_ref, f"shrink_expand routing {k}", slack=slack)
+    assert engine.device_errors() == 0
+
+
 @pytest.mark.parametrize("T", [1, 63, 65, 500, 1025, 2049])
 @pytest.mark.parametrize("rank", [0, 16])
 def test_new_h_is_zero_where_nothing_is_written(T, rank):
