@@ -1625,7 +1625,7 @@ hipError_t launch_rank(const ApplyArgs& a, hipStream_t stream) {
 
 template <int ROLE>
 hipError_t launch_role(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
-  if constexpr (ROLE != kFused && ROLE != kFusedMulti && ROLE != kShrinkNew) {
+  if constexpr (ROLE == kExpandOnly) {
     if (a.tiles > 1)
       return dtype_bf16 ? launch_rank<__bf16, ROLE, kTilesInFlight>(a, stream)
                         : launch_rank<_Float16, ROLE, kTilesInFlight>(a, stream);
@@ -2102,7 +2102,8 @@ hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, int64_t empty_slots
                     : launch_shrink_t<_Float16, kShrinkSlices>(a, empty_slots, stream);
 }
 hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
-  if (a.srows != kShrinkRowsFused || a.n_ochunks != a.w.n_a || a.n_sub != 1 || a.n_chunks < 1 ||
+  // Like the fused roles it runs on the 16-token table.
+  if (a.tiles != 1 || a.srows != kShrinkRowsFused || a.n_ochunks != a.w.n_a || a.n_sub != 1 || a.n_chunks < 1 ||
       a.n_chunks > kMaxChunks || a.w.n_a < 1 || a.w.n_a > kMaxSlices || a.hs != a.w.n_a * a.hs1 ||
       a.n_chunks * a.hs > kMaxChunks * kMaxRank || (a.w.n_a > 1 && (a.w.mode != kStacked || a.rank == 0)) ||
       (a.h_fill > 0 && (a.w.n_a > 1 || a.h_f32 != 0 || a.h_fill % 8 != 0 || a.ldh % 8 != 0 || a.h_rows < 1)))
