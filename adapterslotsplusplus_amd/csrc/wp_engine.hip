@@ -1621,8 +1621,8 @@ int add_lora_impl(wp_engine* e, const char* who, void* y, const void* x, int32_t
   a.n_slots = block_bound(e, num_loras, fused);
   if (!fused) {
     // Large plans (prefill-sized, 64-token blocks): shrink into the engine's
-    // H (one launch per A slice, each into its columns of an H row), then
-    // expand from it.  Each launch keeps several token tiles in flight per
+    // H (one launch, each A slice into its columns of an H row), then expand
+    // from it.  Each launch keeps several token tiles in flight per
     // workgroup; the kernel boundary replaces the in-kernel wait.
     if (e->plan_T > e->tok_cap) return fail(WP_ERR_CAPACITY, "%s: table reaches past the engine's H rows", who);
     a.h = e->hbuf;
@@ -1739,8 +1739,11 @@ int wp_add_lora_nslice(wp_engine* e, void* y, const void* x, int32_t n_slices, c
 int wp_shrink_expand(wp_engine* e, const void* X, void* Y, int32_t d_model, int32_t out_features, int32_t rank,
                      int64_t T, int64_t y_row_stride, int32_t y_col_offset, int32_t dtype, void* stream_) {
   if (!e) return fail(WP_ERR_INVALID, "shrink_expand: engine is NULL");
-  if (e->plan_kind == 0 || !fused_fits(e, rank, 1, ceil_div(out_features, expand_cols_per_workgroup()),
-                                       cover_bound(e, resolvable_ids(e, static_cast<hipStream_t>(stream_)), true))) {
+  const int64_t slots = e->plan_bt > kFineTokens
+                            ? cover_bound(e, resolvable_ids(e, static_cast<hipStream_t>(stream_)), true)
+                            : 0;
+  if (e->plan_kind == 0 ||
+      !fused_fits(e, rank, 1, ceil_div(out_features, expand_cols_per_workgroup()), slots)) {
     // Large plans: shrink() into the engine's H, then expand() from it (the
     // same checks and errors as the two calls).  The expand runs on blocks
     // whose H this shrink wrote, no others: hbuf holds other calls' rows.
@@ -1946,6 +1949,8 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
   }
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
+  // Larger plans keep to their own table here; which form is faster with
+  // several slices added to an fp32 output past 512 tokens is not measured.
   const bool small = e->plan_bt <= kFineTokens;
   ApplyArgs a = stacked_base(e, rank, num_loras, scale, small);
   a.x = x;

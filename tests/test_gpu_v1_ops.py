@@ -455,3 +455,29 @@ def test_lora_shrink_slices_that_share_words_add_up(T, stride):
     torch.cuda.synchronize()
     assert_close(out, ref, "overlapping slices", rtol=1e-4, atol=1e-4)
     assert eng.device_errors() == 0
+
+
+@pytest.mark.parametrize("L,n", [(100, 4), (280, 3)])
+def test_lora_shrink_with_the_reducers_dispatched_last(L, n):
+    """More reducers (block slots x slices: 528, 936) than half of the resident
+    workgroups hold go last: on a device of 256 compute units the second shape's
+    do, the first one's go first.  Every id has a token, so real blocks lie over
+    the whole grid; run twice, so that the first call has to leave the partial
+    buffer empty."""
+    dtype, T, rank, d = torch.bfloat16, 512, 16, 1032
+    announce(f"lora_shrink reducers L={L} n={n}")
+    ids = torch.from_numpy(np.random.default_rng(L).permutation(np.arange(T) % (L + 1)) - 1)
+    was, _, _ = weights(L, rank, d, (16,) * n, dtype, 960)
+    x = randn((T, d), 961, dtype)
+    h0 = randn((n, T, rank), 962, torch.float32)
+    eng = WarpPipeEngine(WarpPipeConfig(max_tokens=512))
+    assert eng.build_seg_bounds(ids.cuda())
+    h = h0.cuda()
+    for _ in range(2):
+        assert eng.lora_shrink(h, x.cuda(), was, 0.5)
+    torch.cuda.synchronize()
+    ref = h0
+    for _ in range(2):
+        ref = v1_ops.lora_shrink(ref, x, cpu(was), 0.5, ids)
+    assert_close(h, ref, "lora_shrink, reducers last", rtol=1e-4, atol=1e-4)
+    assert eng.device_errors() == 0
