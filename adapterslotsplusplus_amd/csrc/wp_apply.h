@@ -62,7 +62,7 @@ struct ApplyArgs {
                       // workgroups, so that those always find room)
   float* part;        // fp32 partial H by plan position: [n_chunks][ptok][hs], kPartialEmpty between calls
   uint32_t* consumed; // per block (stride kCounterStride): fused calls count expand workgroups done reading,
-                      // shrink() counts d-range workgroups done; zero between calls
+                      // shrink() counts the d-ranges' waves done with each 16-token tile; zero between calls
   uint32_t spin_limit; // polls before a wait on partials gives up (kDefaultSpinLimit)
   uint64_t* trace;     // traced builds (WP_TRACE) only: kTraceWords timestamps per workgroup, or null
   int64_t trace_words; // capacity of `trace` (a launch whose grid does not fit is not traced)
@@ -165,15 +165,16 @@ struct StageJobs {
 };
 hipError_t launch_stage_copies(const StageJobs& jobs, hipStream_t stream);
 
-// shrink(): a workgroup streams its d-range (a.dc, a multiple of
-// kShrinkSlices * 128 columns) in groups of kShrinkSlices 128-column slices.
+// shrink(): a workgroup streams its d-range (a.dc columns: half of
+// kShrinkSlices * 128, or a multiple of it) in passes of half or all of
+// kShrinkSlices 128-column slices.
 constexpr int kShrinkSlices = 8;
 
 // One launch: shrink + expand of a whole add_lora call (partials, counters).
 hipError_t launch_fused(int dtype_bf16, const ApplyArgs& a, hipStream_t stream);
 // shrink(): one workgroup per (block, group of A slices of at most 64 rows,
-// d-range); the block's last workgroup to finish sums the d-ranges into
-// H[token], slice s at element s * a.ldy of an H row.
+// d-range); the last wave to finish a 16-token tile of a group sums its
+// d-ranges into H[token], slice s at element s * a.ldy of an H row.
 // empty_slots: slots of the grid that a plan of whole blocks would leave empty.
 hipError_t launch_shrink(int dtype_bf16, const ApplyArgs& a, int64_t empty_slots, hipStream_t stream);
 // shrink() of decode-sized plans: the fused kernel's shrink workgroups

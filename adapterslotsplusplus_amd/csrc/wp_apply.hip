@@ -1247,7 +1247,7 @@ hipError_t launch_expand_ext_d(const ApplyArgs& a, const ExpandExt& x, hipStream
 // per (block, group of A slices, d-range) computes every rank row of the group
 // -- up to 64 rows, whole slices, so slices that share X read it once -- and
 // each X element is read once per group.  The d-range is streamed in K-slices
-// of kSliceK elements, software pipelined one slice ahead: the slice of A
+// of kSliceK elements, kShrinkDepth slices in flight: the slice of A
 // (rows x kSliceK) is loaded once per workgroup and shared by the four
 // waves through LDS (double buffered), and each wave, which owns one
 // 16-token tile, loads its X through a tile of its own.  The
@@ -1257,11 +1257,11 @@ hipError_t launch_expand_ext_d(const ApplyArgs& a, const ExpandExt& x, hipStream
 //
 // One compute unit's read rate bounds it: 35-40 GB/s whatever is in flight (a
 // 16-token workgroup's 8 slices take 5 us, and three or four slices in flight
-// the same), so at 8192 tokens and rank 64 the units that drew three
-// workgroups' X and A set the time, 25.7 us (X alone takes 13 us at the copy rate).
-// Launch overhead and the partial sums are the rest, and a launch never costs
-// less than 9 us.  So one launch
-// for every A slice, with X read once per 64 rows, replaced one launch each:
+// the same; a plain read by one workgroup reaches 38-47), so at 8192 tokens and
+// rank 64 the units that drew three workgroups' X and A set the time, 26-28 us
+// (X alone takes 13 us at the copy rate).  Launch overhead and the partial sums
+// are the rest: 7.5 us at 640 tokens, rank 16, d = 4096.  So one launch for
+// every A slice, with X read once per 64 rows, replaced one launch each:
 // q/k/v with three A of rank 16, call total on MI355X 53.3 -> 34.3 us at 2048
 // tokens, 116 -> 84 at 8192 (rank 64: 79 -> 64, 157 -> 132).
 constexpr int kSliceK = 128;

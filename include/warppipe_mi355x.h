@@ -206,7 +206,7 @@ int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_
 /* shrink() followed by expand() over the adapter store, as one call: no
  * counterpart in the reference (its callers run the two after each other,
  * bindings:132-148).  Plans of up to 512 tokens, and larger build_seg_bounds
- * plans as far as the rank allows (about 98304 / rank tokens), run both halves
+ * plans as far as rank and grid allow (about 98304 / rank tokens), run both halves
  * in one launch with no H round trip (rank = 0: mixed ranks, each adapter's
  * own); others run shrink then expand through the engine's own H.  Results
  * match the two calls within the fp tolerance (the d-range split, and so the
