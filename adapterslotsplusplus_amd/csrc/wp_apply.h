@@ -34,6 +34,14 @@ __device__ __forceinline__ uint32_t touch_kernel_args_issue() {
 }
 __device__ __forceinline__ void touch_kernel_args_wait(uint32_t t) { asm volatile("" ::"s"(t)); }
 
+// What a shrink() or expand() launch does with H.
+enum HMode : int32_t {
+  kHRows = 0,        // shrink(): H = rn(alpha * sum) in the I/O type; expand(): H as it is
+  kHAddFp32 = 1,     // shrink(): H is fp32, alpha * sum is added to it unrounded (vLLM's lora_shrink buffer)
+  kHFromPartials = 2 // expand() on 64-token blocks of the engine's H, which a small shrink wrote just before:
+                     // nothing while the partials are poisoned, as that shrink then left rows unwritten
+};
+
 // Kernel arguments of one shrink or expand launch (passed by value).
 struct ApplyArgs {
   const void* x;   // X [T, ldx]
@@ -68,11 +76,9 @@ struct ApplyArgs {
   int64_t trace_words; // capacity of `trace` (a launch whose grid does not fit is not traced)
   PlanView plan;
   Weights w;
-  // shrink() only: 1 = H is fp32 and the call adds alpha * sum to it,
-  // unrounded (vLLM's lora_shrink buffer); 0 = H = rn(alpha * sum) in the
-  // I/O type.  At the end of the arguments: fields placed before the hot
+  // HMode of H.  At the end of the arguments: fields placed before the hot
   // kernels' argument reads measured up to 0.3 us more per launch.
-  int32_t h_f32;
+  int32_t h_mode;
   // shrink() of decode-sized plans into a new H: columns of a row that no rank
   // fills, rows of skipped blocks and of tokens without an adapter are zeroed
   // (h_fill: columns of a row, 0: H is the caller's; h_rows: its rows).

@@ -936,7 +936,7 @@ __device__ __forceinline__ void reduce_to_h(const ApplyArgs& a, int b, int sa, c
   const int col = sa * a.hs1;
   if (blk.count * wrote * a.n_chunks > 2048) wait_partials<false>(a, blk, wrote, s_flag, 1u, col);
   T* H = static_cast<T*>(a.h);
-  const bool f32 = a.h_f32 != 0;
+  const bool f32 = a.h_mode == kHAddFp32;
   const int64_t h0 = sa * a.ldy;
   collect_partials<8>(a, blk, wrote / 2, res.alpha, [&](int j, int r0, f32x2 v) {
     const int64_t at = h0 + static_cast<int64_t>(toks[j]) * a.ldh + r0;
@@ -1069,7 +1069,7 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   const int n_blocks = static_cast<int>(header[ROLE == kExpandOnly && TILES > 1 ? kHdrNumBlocks : kHdrNumFine]);
   const uint32_t n_coarse = ROLE == kExpandOnly && TILES == 1 ? header[kHdrNumBlocks] : 0u;
   // Roles that use the partial buffer do nothing while it is poisoned.
-  const uint32_t poison = ROLE == kExpandOnly ? 0u : header[kHdrPoison];
+  const uint32_t poison = ROLE == kExpandOnly && TILES == 1 ? 0u : header[kHdrPoison];
   const Block blk = blocks[b];
   const int row = threadIdx.x & 15;
   const int32_t tok0 = bperm[static_cast<int64_t>(b) * kBlockTokens + row];
@@ -1093,13 +1093,17 @@ void apply_kernel(const uint32_t* header, const Block* __restrict__ blocks,
   if (b == a.n_slots - 1 && part == 0 && threadIdx.x == 0 && n_blocks > a.n_slots)
     flag_error(a.plan.header, kErrCapacity);
   if constexpr (!PA || RANK == 0) touch_kernel_args_wait(ka_touch);
-  if ((b >= n_blocks) | (blk.count <= 0) | (tok0 < -1) | (poison != 0u)) {
+  if ((b >= n_blocks) | (blk.count <= 0) | (tok0 < -1) | (ROLE != kExpandOnly && poison != 0u)) {
     if constexpr (ROLE == kShrinkNew) {
       // Blocks skipped because the partials are poisoned leave zero rows.
       if (!shrink_role && b < n_blocks && blk.count > 0)
         zero_h_rows<T>(a, bperm + static_cast<int64_t>(b) * kBlockTokens, blk.count, 0);
     }
     return;
+  }
+  if constexpr (ROLE == kExpandOnly && TILES > 1) {
+    // Behind the exit test: an empty slot's workgroup waits for no argument.
+    if (poison != 0u && a.h_mode == kHFromPartials) return;
   }
   if constexpr (ROLE == kExpandOnly && TILES == 1) {
     if (n_coarse > static_cast<uint32_t>(a.cover) - 1u) {
@@ -1449,7 +1453,7 @@ void shrink_kernel(const uint32_t* header, const Block* __restrict__ blocks, con
   // acc[m]: rows m*16 + 4*(lane/16) + [0, 4) of token slot tl.
   const int rq = (lane >> 4) * 4;
   // fp32 H (vLLM's lora_shrink buffer): alpha * sum added to it, unrounded.
-  const bool f32 = a.h_f32 != 0;
+  const bool f32 = a.h_mode == kHAddFp32;
   auto put_h = [&](int32_t token, int r, f32x4 v) {
     const int s = kMixed || a.w.n_a == 1 ? 0 : r / rank;
     const int64_t at = static_cast<int64_t>(token) * a.ldh + (s0 + s) * a.ldy + (r - s * rank);
@@ -2106,12 +2110,12 @@ hipError_t launch_shrink_small(int dtype_bf16, const ApplyArgs& a, hipStream_t s
   if (a.tiles != 1 || a.srows != kShrinkRowsFused || a.n_ochunks != a.w.n_a || a.n_sub != 1 || a.n_chunks < 1 ||
       a.n_chunks > kMaxChunks || a.w.n_a < 1 || a.w.n_a > kMaxSlices || a.hs != a.w.n_a * a.hs1 ||
       a.n_chunks * a.hs > kMaxChunks * kMaxRank || (a.w.n_a > 1 && (a.w.mode != kStacked || a.rank == 0)) ||
-      (a.h_fill > 0 && (a.w.n_a > 1 || a.h_f32 != 0 || a.h_fill % 8 != 0 || a.ldh % 8 != 0 || a.h_rows < 1)))
+      (a.h_fill > 0 && (a.w.n_a > 1 || a.h_mode != kHRows || a.h_fill % 8 != 0 || a.ldh % 8 != 0 || a.h_rows < 1)))
     return hipErrorInvalidValue;
   return a.h_fill > 0 ? launch_role<kShrinkNew>(dtype_bf16, a, stream) : launch_role<kShrinkOnly>(dtype_bf16, a, stream);
 }
 hipError_t launch_expand(int dtype_bf16, const ApplyArgs& a, hipStream_t stream) {
-  if (a.w.n_a < 1 || a.w.n_a > kMaxSlices) return hipErrorInvalidValue;
+  if (a.w.n_a < 1 || a.w.n_a > kMaxSlices || (a.h_mode == kHFromPartials && a.tiles == 1)) return hipErrorInvalidValue;
   return launch_role<kExpandOnly>(dtype_bf16, a, stream);
 }
 

@@ -1438,10 +1438,15 @@ void fused_split(ApplyArgs* a, int rank, int d_model, int n_cu) {
 
 namespace {
 
-// Whose H rows a shrink fills: the caller's (wp_shrink), all new ones
-// (wp_shrink_new), or the engine's, for an expand that follows at once
-// (wp_shrink_expand).  The last runs on the plan's own table only: the small
-// form would leave rows unwritten while the partials are poisoned.
+// Whether wp_shrink_expand's first launch may be a small shrink: only if its
+// expand runs on 64-token blocks, which test for what that leaves unwritten
+// (the word's load costs the 16-token expand 0.1-0.2 us a call).
+bool small_pair_fits(const wp_engine* e, int rank, int64_t slots) {
+  return small_shrink_fits(e, rank, slots) && !fine_expand_fits(e, rank);
+}
+
+// wp_shrink, (kNewRows) wp_shrink_new, and (kEngineRows) wp_shrink_expand's
+// first launch: whose H rows are filled.
 enum HRows { kCallerRows, kNewRows, kEngineRows };
 int shrink_impl(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t rank, int64_t T, int64_t h_row_stride,
                 int32_t dtype, HRows rows, void* stream_) {
@@ -1471,7 +1476,8 @@ int shrink_impl(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t r
   DeviceGuard g(e->device);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   const int64_t ids = resolvable_ids(e, stream);
-  const bool small = rows != kEngineRows && small_shrink_fits(e, rank, cover_bound(e, ids, true));
+  const int64_t slots = cover_bound(e, ids, true);
+  const bool small = rows == kEngineRows ? small_pair_fits(e, rank, slots) : small_shrink_fits(e, rank, slots);
   ApplyArgs a = base_args(e, rank, small);
   a.x = X;
   a.ldx = d_model;
@@ -1525,10 +1531,12 @@ int wp_shrink_new(wp_engine* e, const void* X, void* H, int32_t d_model, int32_t
 
 namespace {
 
-// wp_expand; d_model (wp_shrink_expand, else 0): adapters of another input
-// width, whose shrink was skipped, are skipped too.
-int expand_impl(wp_engine* e, const void* H, void* Y, int32_t d_model, int32_t out_features, int32_t rank, int64_t T,
-                int64_t h_row_stride, int64_t y_row_stride, int32_t y_col_offset, int32_t dtype, void* stream_) {
+// wp_expand.  As wp_shrink_expand's second launch it skips what the first did:
+// adapters of another input width (d_model, else 0), and everything while the
+// partials are poisoned (h_mode).
+int expand_impl(wp_engine* e, const void* H, void* Y, int32_t d_model, HMode h_mode, int32_t out_features, int32_t rank,
+                int64_t T, int64_t h_row_stride, int64_t y_row_stride, int32_t y_col_offset, int32_t dtype,
+                void* stream_) {
   if (!e) return fail(WP_ERR_INVALID, "expand: engine is NULL");
   if (rank != 0 && !rank_ok(rank)) return fail(WP_ERR_INVALID, "dispatch_bgmv_expand: unsupported rank (only 8/16/32/64)");
   int rc = check_io("expand", dtype, H, "H");
@@ -1564,6 +1572,7 @@ int expand_impl(wp_engine* e, const void* H, void* Y, int32_t d_model, int32_t o
   a.y = Y;
   a.ldy = y_row_stride;
   a.d_model = d_model;
+  a.h_mode = h_mode;
   if ((rc = table_weights(e, stream, &a.w, small)) != WP_OK) return rc;
   const int cols = expand_cols_per_workgroup();
   a.w.n_slices = 1;
@@ -1585,7 +1594,7 @@ extern "C" {
 
 int wp_expand(wp_engine* e, const void* H, void* Y, int32_t out_features, int32_t rank, int64_t T, int64_t h_row_stride,
               int64_t y_row_stride, int32_t y_col_offset, int32_t dtype, void* stream) {
-  return expand_impl(e, H, Y, 0, out_features, rank, T, h_row_stride, y_row_stride, y_col_offset, dtype, stream);
+  return expand_impl(e, H, Y, 0, kHRows, out_features, rank, T, h_row_stride, y_row_stride, y_col_offset, dtype, stream);
 }
 
 }  // extern "C"
@@ -1750,7 +1759,8 @@ int wp_shrink_expand(wp_engine* e, const void* X, void* Y, int32_t d_model, int3
     const int64_t hs = rank == 0 ? kMaxRank : rank;
     int rc = shrink_impl(e, X, e->hbuf, d_model, rank, T, hs, dtype, kEngineRows, stream_);
     if (rc != WP_OK) return rc;
-    return expand_impl(e, e->hbuf, Y, d_model, out_features, rank, T, hs, y_row_stride, y_col_offset, dtype, stream_);
+    return expand_impl(e, e->hbuf, Y, d_model, small_pair_fits(e, rank, slots) ? kHFromPartials : kHRows, out_features,
+                       rank, T, hs, y_row_stride, y_col_offset, dtype, stream_);
   }
   if (rank != 0 && !rank_ok(rank)) return fail(WP_ERR_INVALID, "shrink_expand: unsupported rank (only 8/16/32/64)");
   int rc = check_io("shrink_expand", dtype, X, "X");
@@ -1966,7 +1976,7 @@ int wp_lora_shrink(wp_engine* e, float* out, int64_t out_slice_stride, int64_t o
   a.h = out;
   a.ldh = out_row_stride;
   a.ldy = out_slice_stride;
-  a.h_f32 = 1;
+  a.h_mode = kHAddFp32;
   if (small) {
     // Every slice in one launch: a launch takes 7 us at 48 tokens, its bytes
     // under 1 (a step of four layers, three slices each 125 -> 68 us, MI355X).

@@ -955,10 +955,11 @@ def test_two_launch_expand_reads_only_the_h_of_its_shrink(rank, T, o):
     assert engine.device_errors() == 2 | 16
 
 
-def test_two_launch_shrink_expand_does_not_depend_on_the_partials():
-    """Mixed ranks to many columns at 1100 tokens (two launches): a give-up, or
-    partials left poisoned by another call's, changes nothing; no launch of the
-    call uses them."""
+def test_two_launch_shrink_expand_beside_poisoned_partials():
+    """Mixed ranks to many columns at 1100 tokens (a small shrink and an expand):
+    with a give-up in the call, or partials left poisoned by another, Y is the
+    result or left alone as a whole, never the engine's H of an earlier call;
+    poisoned partials leave it alone, and the next plan build repairs them."""
     dtype, d, o, T = torch.bfloat16, 264, 8452, 1100
     announce("two-launch shrink_expand beside poisoned partials")
     engine, adapters = small_store(0, d, o, [0, 1, 2], 1520)
@@ -973,16 +974,25 @@ def test_two_launch_shrink_expand_does_not_depend_on_the_partials():
     for aid, (A, B, alpha) in adapters.items():
         rows = torch.from_numpy(np.nonzero(idx == aid)[0])
         slack[rows] += (h_tie_flips(X[rows], A, alpha, dtype) @ B.double().abs().T).float()
-    engine.set_spin_limit(0)
-    for _ in range(2):
+    engine.set_spin_limit(0)  # a wait gives up where a word is not there at once
+    gave_up = 0
+    for _ in range(4):
         Y = Y0.cuda()
         engine.shrink_expand(X.cuda(), Y, o, 0)
         torch.cuda.synchronize()
-        assert_close(Y, Y_ref, "shrink_expand", slack=slack)
-        engine.shrink(X.cuda(), d, 0, T)  # gives up where a word is not there at once
+        left = torch.equal(Y.cpu(), Y0)
+        assert left or not gave_up  # still poisoned
+        if left:
+            gave_up += 1
+        else:
+            assert_close(Y, Y_ref, "shrink_expand", slack=slack)
     engine.set_spin_limit(None)
+    assert engine.build_seg_bounds(idx_d)
+    Y = Y0.cuda()
+    engine.shrink_expand(X.cuda(), Y, o, 0)
     torch.cuda.synchronize()
-    engine.device_errors()
+    assert_close(Y, Y_ref, "shrink_expand after the repair", slack=slack)
+    assert (engine.device_errors() != 0) == (gave_up > 0)
 
 
 @pytest.mark.parametrize("rank,T", [(16, 7000), (64, 1600), (16, 1000)])
